@@ -40,7 +40,7 @@ EXPORTS = (
     "gsa_indexer_select_adaptive_workspace_bytes", "gsa_topk_select_adaptive",
     "gsa_proj_packed_bytes", "gsa_proj_pack", "gsa_proj_fused", "gsa_dense_lane_masks",
     "gsa_prologue_vt_lane_masks", "gsa_debug_force_select_fallback",
-    "gsa_indexer_select_noalloc", "gsa_indexer_select_noalloc_max_bytes",
+    "gsa_indexer_select_noalloc", "gsa_indexer_select_noalloc_max_bytes", "gsa_topk_select_i64",
 )
 
 _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
@@ -51,6 +51,7 @@ _PROTOS = {
     "gsa_indexer_scores": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _f32,
                             _i32, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i64, _vp], _i32),
     "gsa_topk_select": ([_vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp, _vp], _i32),
+    "gsa_topk_select_i64": ([_vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp, _vp, _vp], _i32),
     "gsa_topk_select_adaptive": ([_vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
                                   _vp, _vp, _vp, _vp, _vp, _vp], _i32),
     "gsa_indexer_select": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _f32,
@@ -203,6 +204,25 @@ def topk_select(scores: torch.Tensor, k_eff: int, order: int = ORDER_INDEX_ASC,
                              int(order), _ptr(idx), _ptr(cnt), _ptr(mask), _stream(scores))
     _check(st, "gsa_topk_select")
     return idx, cnt, mask
+
+
+def topk_select_i64(scores: torch.Tensor, k_eff: int):
+    """Exact per-row top-k of fp32 scores [B,T,Tkv], by (score desc, index asc)
+    -> (idx int64, mask bool), both [B,T,k_eff]."""
+    lib = load()
+    _need_cuda(scores)
+    if scores.dtype != torch.float32:
+        raise TypeError("scores must be float32")
+    _expect(scores.dim() == 3, "scores: [B,T,Tkv]")
+    B, T, Tkv = scores.shape
+    if scores.stride(2) != 1:
+        raise ValueError("scores must have unit column stride")
+    idx = torch.empty(B, T, k_eff, device=scores.device, dtype=torch.int64)
+    mask = torch.empty(B, T, k_eff, device=scores.device, dtype=torch.bool)
+    st = lib.gsa_topk_select_i64(_ptr(scores), scores.stride(0), scores.stride(1), B, T, Tkv, int(k_eff),
+                                 _ptr(idx), _ptr(mask), _stream(scores))
+    _check(st, "gsa_topk_select_i64")
+    return idx, mask
 
 
 def topk_select_adaptive(scores: torch.Tensor, k_base: int, k_min: int, k_max: int,

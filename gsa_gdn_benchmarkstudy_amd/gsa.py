@@ -249,6 +249,8 @@ class AdaptiveTopKSelector(nn.Module):
         _range_push("gsa_hip/topk_select")
         try:
             if k_eff <= _abi.TOPK_DESC_MAX_K:
+                if not self.adaptive():
+                    return (*_abi.topk_select_i64(s, k_eff), k_eff)
                 idx, _, mask = self._select(s, k_eff, _abi.ORDER_SCORE_DESC)
                 return idx.long(), mask.bool(), k_eff
             # larger k: exact selection in index order, then a stable device sort by score

@@ -107,6 +107,17 @@ int gsa_topk_select(const float* scores, int64_t s_sb, int64_t s_st,
                     void* stream);
 
 /*
+ * gsa_topk_select in GSA_ORDER_SCORE_DESC order with 64-bit indices, the types
+ * that AdaptiveTopKSelector.forward returns (gsa_triton/gsa_opt.py:473-483):
+ * idx_out int64 [B,T,k_eff], mask_out uint8 [B,T,k_eff] (nullable).  Same
+ * selection, order and limits.
+ */
+int gsa_topk_select_i64(const float* scores, int64_t s_sb, int64_t s_st,
+                        int B, int T, int Tkv, int k_eff,
+                        int64_t* idx_out, uint8_t* mask_out,
+                        void* stream);
+
+/*
  * gsa_topk_select with the variance-based per-row k of gsa_explained.ipynb:
  * 577-592 (the rule AdaptiveTopKSelector, gsa_triton/gsa_opt.py:466-483,
  * keeps k_min for but does not apply).  var_out[r] = population variance of

@@ -95,6 +95,46 @@ def test_topk_select_bitexact(dev, T, k, levels):
     assert torch.equal(gc.cpu(), ca)
 
 
+@pytest.mark.parametrize("Tkv,k", [(1, 1), (63, 63), (256, 40), (2048, 2048), (2049, 300), (4096, 4096), (4097, 1),
+                                   (8192, 2048), (8193, 4096), (16384, 2048), (16385, 4000), (70000, 64)])
+def test_topk_select_sorted_orders(dev, Tkv, k):
+    """GSA_ORDER_SCORE_DESC at the edges of the row lengths that the counting sort splits at
+    (registers, block sizes, re-read rows, rows past its limit), int32 and int64 outputs: rows
+    of indexer-like scores, few valid ones, none, ties that fill bins, one value, negative
+    scores, a subnormal range, +-0, infinities and NaN, scores below -1e9."""
+    _log(f"topk sorted Tkv={Tkv} k={k}")
+    g = torch.Generator().manual_seed(Tkv + k)
+    ninf = float("-inf")
+    rows = [torch.rand(4, Tkv, generator=g).sum(0), torch.randn(Tkv, generator=g) - 3.0,
+            torch.randint(0, 50, (Tkv,), generator=g).float(), torch.full((Tkv,), 0.25), torch.full((Tkv,), ninf),
+            torch.rand(Tkv, generator=g) * 1e-39, torch.randn(Tkv, generator=g) * 1e30,
+            torch.rand(Tkv, generator=g) * 2e9 - 1.5e9]
+    few = torch.rand(Tkv, generator=g)
+    few[torch.rand(Tkv, generator=g) < 0.9] = ninf
+    half = torch.rand(Tkv, generator=g)
+    half[Tkv // 2 + 1:] = ninf
+    special = torch.rand(Tkv, generator=g)
+    special[::7] = float("inf")
+    special[3::11] = float("nan")
+    s = torch.stack(rows + [few, half, special])[None]
+    wide = torch.zeros(1, s.shape[1], Tkv + 3)      # an odd row stride
+    wide[..., :Tkv] = s
+    ref_idx, ref_mask = orc.select_topk(s, k)
+    for view in (s.to(dev), wide.to(dev)[..., :Tkv]):
+        i32, cnt, m8 = _abi.topk_select(view, k, _abi.ORDER_SCORE_DESC, want_mask=True)
+        i64, mb = _abi.topk_select_i64(view, k)
+        assert i64.dtype == torch.int64 and mb.dtype == torch.bool
+        assert torch.equal(i64.cpu(), ref_idx) and torch.equal(mb.cpu(), ref_mask)
+        assert torch.equal(i32.cpu().long(), ref_idx) and torch.equal(m8.cpu().bool(), ref_mask)
+        assert torch.equal(cnt.cpu().long(), ref_mask.sum(-1))
+    zeros = torch.tensor([0.0, -0.0, 1.0, -0.0, 0.0, ninf]).repeat(Tkv // 6 + 1)[:Tkv][None, None]
+    key = torch.where(zeros == ninf, torch.tensor(-1e9), zeros)
+    # -0 ranks just below +0, as the selector orders its keys
+    order = torch.sort(key + torch.where(torch.signbit(zeros) & (zeros == 0), -1e-30, 0.0), dim=-1, descending=True,
+                       stable=True).indices[..., :k]
+    assert torch.equal(_abi.topk_select_i64(zeros.to(dev), k)[0].cpu(), order)
+
+
 def test_topk_select_special_values(dev):
     s = torch.tensor([[[0.5, float("nan"), 2.0, float("inf"), -1e9, float("-inf"), -3.0, 0.5]]])
     gi, gc, gm = _abi.topk_select(s.to(dev), 5, _abi.ORDER_INDEX_ASC, want_mask=True)
