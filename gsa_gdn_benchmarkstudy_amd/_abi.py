@@ -41,6 +41,7 @@ EXPORTS = (
     "gsa_proj_packed_bytes", "gsa_proj_pack", "gsa_proj_fused", "gsa_dense_lane_masks",
     "gsa_prologue_vt_lane_masks", "gsa_debug_force_select_fallback",
     "gsa_indexer_select_noalloc", "gsa_indexer_select_noalloc_max_bytes", "gsa_topk_select_i64",
+    "gsa_selected_attn", "gsa_selected_attn_workspace_bytes",
 )
 
 _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
@@ -73,6 +74,10 @@ _PROTOS = {
     "gsa_sparse_attn": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64,
                          _vp, _i64, _i64, _i32, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64,
                          _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _vp], _i32),
+    "gsa_selected_attn_workspace_bytes": ([_i32, _i32, _i32, _i32, _i32, _f32, _i32], ctypes.c_size_t),
+    "gsa_selected_attn": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i32, _i64, _i64, _i32, _vp, _vp,
+                           _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _vp, ctypes.c_size_t, _vp],
+                          _i32),
     "gsa_prologue_vt": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64,
                          _i32, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp], _i32),
     "gsa_selection_mask": ([_vp, _i64, _i64, _i32, _vp, _vp, _i32, _i32, _i32, _vp, _i64, _i64, _vp], _i32),
@@ -459,6 +464,55 @@ def sparse_attn(q, k, v, idx, scale: float, count=None, mask=None, og=None, cos=
                              _ptr(out), *_rows(out, HD), B, T, Tkv, H, d, float(scale),
                              dtype_code(q.dtype), int(flags), _stream(q))
     _check(st, "gsa_sparse_attn")
+    return out
+
+
+# Row strides (elements) up to which gsa_selected_attn's tile loads reach.
+_SELECTED_MAX_STRIDE = 1 << 24
+
+
+def selected_attn(q, k, v, idx, scale: float, mask=None) -> torch.Tensor:
+    """Attention over per-row index lists -> out [B,T,H,d]: on the matrix cores
+    (gsa_selected_attn) where the library serves the sizes that way, else the
+    gather kernel (sparse_attn).  idx: any integer dtype, [B,T,k_sel]; mask: idx's
+    shape, nonzero (as uint8) = valid."""
+    lib = load()
+    _need_cuda(q, k, v, idx, mask)
+
+    def gather():
+        m = None if mask is None else mask.to(torch.uint8).contiguous()
+        return sparse_attn(q, k, v, idx.to(torch.int32).contiguous(), scale, mask=m)
+
+    if q.dim() != 4 or k.dim() != 4 or idx.dim() != 3 or idx.numel() == 0:
+        return gather()                      # (its checks name what is wrong)
+    B, T, H, d = q.shape
+    Tkv, k_sel, HD = k.shape[1], idx.shape[2], H * d
+    if d != 128 or min(B, T, Tkv) < 1 or q.dtype not in (torch.bfloat16, torch.float32):
+        return gather()
+    need = lib.gsa_selected_attn_workspace_bytes(B, T, Tkv, H, k_sel, float(scale), dtype_code(q.dtype))
+    if need == 0 or max(t.stride(1) for t in (q, k, v)) > _SELECTED_MAX_STRIDE:
+        return gather()
+    _expect(k.shape[0] == B and tuple(k.shape[2:]) == (H, d) and tuple(v.shape) == tuple(k.shape),
+            "k, v: [B,Tkv,H,d] matching q")
+    _expect(k.dtype == v.dtype == q.dtype, "q, k, v must share a dtype")
+    _expect(tuple(idx.shape[:2]) == (B, T), "idx: [B,T,k_sel]")
+    if mask is not None:
+        _expect(tuple(mask.shape) == tuple(idx.shape), "mask: idx's shape")
+    try:
+        ws = torch.empty(need, device=q.device, dtype=torch.uint8)
+    except torch.OutOfMemoryError:
+        return gather()                      # needs no workspace
+    if idx.dtype not in (torch.int32, torch.int64):
+        idx = idx.to(torch.int32)
+    idx = idx.contiguous()
+    if mask is not None:
+        mask = (mask if mask.dtype in (torch.bool, torch.uint8) else mask.to(torch.uint8)).contiguous()
+    out = torch.empty(B, T, H, d, device=q.device, dtype=q.dtype)
+    st = lib.gsa_selected_attn(_ptr(q), *_rows(q, HD), _ptr(k), *_rows(k, HD), _ptr(v), *_rows(v, HD),
+                               _ptr(idx), idx.element_size(), idx.stride(0), idx.stride(1), k_sel, None, _ptr(mask),
+                               _ptr(out), *_rows(out, HD), B, T, Tkv, H, d, float(scale), dtype_code(q.dtype),
+                               _ptr(ws), need, _stream(q))
+    _check(st, "gsa_selected_attn")
     return out
 
 

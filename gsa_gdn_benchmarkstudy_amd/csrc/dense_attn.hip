@@ -45,6 +45,8 @@ struct ProVtArgs {
 };
 
 // Block `blk` of the producer (one (b, h, 64-key tile)); sV: kDK * kKS elements of LDS.
+// kGate false: V^T alone (no RoPE, no gate; k, vg, cos, sin and k_out unused).
+template <bool kGate>
 __device__ __forceinline__ void prologue_vt_block(const ProVtArgs& p, int blk, uint16_t* sV) {
   // heads fastest: the blocks that run side by side read one key tile's
   // rows of every head (4 KiB of contiguous k, v and vg per key)
@@ -60,7 +62,7 @@ __device__ __forceinline__ void prologue_vt_block(const ProVtArgs& p, int blk, u
     const int j = j0 + key;
     u32x4 packed = {0u, 0u, 0u, 0u};
     if (j < p.T) {
-      if (p.k) {
+      if (kGate && p.k) {
         float x[8], cs[8], sn[8];
         load8(p.k + b * p.k_sb + (int64_t)j * p.k_st + h * 128 + c * 8, x);
         load8(p.cos + (int64_t)j * p.cs_st + c * 8, cs);
@@ -68,14 +70,19 @@ __device__ __forceinline__ void prologue_vt_block(const ProVtArgs& p, int blk, u
         rope8<uint16_t>(x, cs, sn, li);
         store8(p.k_out + (((int64_t)b * p.T + j) * p.H + h) * 128 + c * 8, x);
       }
-      float vv[8], gg[8];
-      load8(p.v + b * p.v_sb + (int64_t)j * p.v_st + h * 128 + c * 8, vv);
-      load8(p.vg + b * p.g_sb + (int64_t)j * p.g_st + h * 128 + c * 8, gg);
+      const uint16_t* vp = p.v + b * p.v_sb + (int64_t)j * p.v_st + h * 128 + c * 8;
+      if constexpr (kGate) {
+        float vv[8], gg[8];
+        load8(vp, vv);
+        load8(p.vg + b * p.g_sb + (int64_t)j * p.g_st + h * 128 + c * 8, gg);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float a = round_bf16(vv[2 * i] * round_bf16(sigmoidf_fast(gg[2 * i])));
-        const float z = round_bf16(vv[2 * i + 1] * round_bf16(sigmoidf_fast(gg[2 * i + 1])));
-        packed[i] = pack_bf16(a, z);
+        for (int i = 0; i < 4; ++i) {
+          const float a = round_bf16(vv[2 * i] * round_bf16(sigmoidf_fast(gg[2 * i])));
+          const float z = round_bf16(vv[2 * i + 1] * round_bf16(sigmoidf_fast(gg[2 * i + 1])));
+          packed[i] = pack_bf16(a, z);
+        }
+      } else {
+        packed = *reinterpret_cast<const u32x4*>(vp);
       }
     }
     *reinterpret_cast<u32x4*>(sV + key * kKS + c * 8) = packed;
@@ -96,7 +103,7 @@ __device__ __forceinline__ void prologue_vt_block(const ProVtArgs& p, int blk, u
 
 __global__ __launch_bounds__(256) void prologue_vt_kernel(ProVtArgs p) {
   __shared__ __align__(16) uint16_t sV[kDK * kKS];
-  prologue_vt_block(p, blockIdx.x, sV);
+  prologue_vt_block<true>(p, blockIdx.x, sV);
 }
 
 // ---------------------------------------------------------------------------
@@ -150,6 +157,7 @@ struct LaneMaskArgs {
   int T, G, NT, nunits;   // unit = (batch, 32-row group, kLmTiles tiles): 32 threads
   int block_rows;         // causal: query rows per attention block (tiles past a block's last row are skipped); else 0
   u32x4* lm;
+  const int2* range;      // kSel: each row's tile range (Selection::range); a block's tiles outside its rows' are skipped
 };
 
 // Bit i of an 8-bit value moved to bit 4i.
@@ -168,6 +176,7 @@ __device__ __forceinline__ u32x4 mask_nibbles(uint32_t word) {
 }
 
 // Block `blk` of the mask-operand pass: its 256 threads take units 8*blk .. 8*blk+7.
+template <bool kSel>
 __device__ __forceinline__ void lane_mask_block(const LaneMaskArgs& a, int blk) {
   const int gt = blk * 256 + (int)threadIdx.x;
   const int unit = gt >> 5, n = gt & 31;
@@ -181,6 +190,13 @@ __device__ __forceinline__ void lane_mask_block(const LaneMaskArgs& a, int blk) 
   // up to the last row of the group's attention block, as its block does.
   int nt = a.NT;
   if (a.block_rows) nt = min(a.NT, ((32 * g) / a.block_rows + 1) * a.block_rows / kDK);
+  if constexpr (kSel) {
+    constexpr int kRows = 32 * kDenseWaves;
+    const int r0 = (32 * g) / kRows * kRows;
+    const int2 tr = tile_range<32>(a.range, (int64_t)b * a.T, r0, min(r0 + kRows, a.T));
+    if (kt0 + kLmTiles <= tr.x) return;
+    nt = tr.y;
+  }
   if (kt0 >= nt) return;
   const uint64_t* src =
       reinterpret_cast<const uint64_t*>(a.bits + b * a.b_sb + (int64_t)min(row, a.T - 1) * a.b_st) + kt0;
@@ -196,20 +212,21 @@ __device__ __forceinline__ void lane_mask_block(const LaneMaskArgs& a, int blk) 
   }
 }
 
-__global__ __launch_bounds__(256) void lane_mask_kernel(LaneMaskArgs a) { lane_mask_block(a, blockIdx.x); }
+__global__ __launch_bounds__(256) void lane_mask_kernel(LaneMaskArgs a) { lane_mask_block<false>(a, blockIdx.x); }
 
 // The producer and the lane-mask pass in one launch, their blocks interleaved
 // evenly over the grid so that both kinds run side by side: block b is a
 // lane-mask block iff c(b+1) > c(b), c(b) = floor(b * n_lm / (n_pro + n_lm))
 // (the number of lane-mask blocks before b), with lane-mask index c(b) and
-// producer index b - c(b).
+// producer index b - c(b).  kSel: V^T alone and the masks of a Selection.
+template <bool kSel>
 __global__ __launch_bounds__(256) void prologue_vt_lane_mask_kernel(ProVtArgs p, LaneMaskArgs l, int n_pro,
                                                                     int n_lm) {
   __shared__ __align__(16) uint16_t sV[kDK * kKS];
   const int64_t total = (int64_t)n_pro + n_lm, b = blockIdx.x;
   const int c0 = (int)(b * n_lm / total), c1 = (int)((b + 1) * n_lm / total);
-  if (c1 > c0) lane_mask_block(l, c0);
-  else prologue_vt_block(p, (int)(b - c0), sV);
+  if (c1 > c0) lane_mask_block<kSel>(l, c0);
+  else prologue_vt_block<!kSel>(p, (int)(b - c0), sV);
 }
 
 // ---------------------------------------------------------------------------
@@ -255,6 +272,7 @@ struct DenseArgs {
   int B, T, Tkv, H, nqb;
   float scale_l2;
   int flags;
+  const int2* range; uint8_t* redo;       // kSel: Selection::range and ::redo
 };
 
 constexpr int kDenseCausal = 1 << 8;   // internal flag: skip key tiles after the block's last row
@@ -334,6 +352,17 @@ template <int N> struct Int { static constexpr int value = N; };
 // the wave, at the cost of a second S accumulator pair (64 VGPRs).  Every
 // load is issued one iteration before the barrier that publishes it; the
 // loop is unrolled by two so that slot offsets are constants.
+//
+// kSel: the launcher's form (gsa_selected_attn).  The block walks only the
+// tiles that hold a selected key of its rows, and the weights enter the PV
+// product with all their 24 bits: P = the sum of three bf16 operands (each
+// takes 8 bits of what the ones before it leave), three MFMAs per V^T operand
+// read, for the gather kernel, whose place this takes, holds them in fp32.
+// (Two parts, 2^-18 relative, were not enough for outputs near zero.)  A row
+// whose sums are not positive finite numbers (no valid key, infinities or NaN
+// anywhere in its tiles, products beyond the masks' range) is marked for the
+// gather kernel.
+template <bool kSel>
 __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseArgs p, const u32x4* __restrict__ lm) {
   extern __shared__ __align__(16) u32x4 dsm[];   // K slots 0, 1 (kKU units each), V^T slots 0, 1 (kVU), mask slots 0, 1 (512)
   constexpr int kDW = kDenseWaves;                // waves per block
@@ -361,10 +390,15 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   const int q0 = qb * kDQ;
 
   const int last_key = (p.flags & kDenseCausal) ? min(p.Tkv - 1, q0 + kDQ - 1) : p.Tkv - 1;
-  const int nkt = last_key / kDK + 1;
-  const char* kbase = reinterpret_cast<const char*>(p.k + b * p.k_sb + hd * 128);
-  const char* vtb = reinterpret_cast<const char*>(p.vt + b * p.vt_sb + hd * p.vt_sh);
+  int kt0 = 0, nkt = last_key / kDK + 1;                       // first tile, number of tiles
+  if constexpr (kSel) {
+    const int2 tr = tile_range<64>(p.range, (int64_t)b * p.T, q0, min(q0 + kDQ, p.T));
+    kt0 = __builtin_amdgcn_readfirstlane(tr.x);
+    nkt = __builtin_amdgcn_readfirstlane(tr.y) - kt0;
+  }
   const int64_t kstep = (int64_t)kDK * p.k_st * 2;             // bytes from one K tile to the next
+  const char* kbase = reinterpret_cast<const char*>(p.k + b * p.k_sb + hd * 128) + kt0 * kstep;
+  const char* vtb = reinterpret_cast<const char*>(p.vt + b * p.vt_sb + hd * p.vt_sh) + kt0 * (kDK * 2);
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(dsm));
 
   // ---- tile loads: wave w issues K instructions i = kDW*n + w < 17 and V^T
@@ -379,7 +413,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   uint32_t koff[kDmaKW], koff_last[kDmaKW], voff[kDmaVW];
   {
     const uint32_t kst2 = (uint32_t)p.k_st * 2u, ldv2 = (uint32_t)p.ldv * 2u;
-    const int kmax_last = min(kDK - 1, p.Tkv - 1 - (nkt - 1) * kDK);
+    const int kmax_last = min(kDK - 1, p.Tkv - 1 - (kt0 + nkt - 1) * kDK);
     auto k_off = [&](int i, int kmax) {
       const int u = i * 64 + lane, key = u / kKRow, c = u - key * kKRow;
       return (uint32_t)min(key, kmax) * kst2 + (uint32_t)min(c, 15) * 16u;
@@ -400,7 +434,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   const uint32_t vdst = lds0 + (uint32_t)(2 * kKU * 16) + (uint32_t)wu * 1024u;
   const uint32_t mdst = lds0 + (uint32_t)(kMBase * 16) + (uint32_t)wu * 1024u;   // + slot * kDW KiB
   // this wave's mask operands: group kDW*qb + w, 1 KiB per tile
-  const char* mbase = reinterpret_cast<const char*>(lm + ((int64_t)b * p.G + kDW * qb + gw) * p.NT * 64);
+  const char* mbase = reinterpret_cast<const char*>(lm + (((int64_t)b * p.G + kDW * qb + gw) * p.NT + kt0) * 64);
   const uint32_t moff = (uint32_t)lane * 16u;
   auto issue_k = [&](const char* src, int slot, bool last) {   // one K tile into K slot `slot`
 #pragma unroll
@@ -453,7 +487,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   u32x4 qraw[8];
 #pragma unroll
   for (int s = 0; s < 8; ++s) qraw[s] = xt[xs_unit(i32, 2 * s + h)];
-  if (p.flags & GSA_ATTN_ROPE_Q) {
+  if (!kSel && (p.flags & GSA_ATTN_ROPE_Q)) {
     // the cos and sin rows through the same tile, after the q reads returned:
     // one round for a packed table (row: cos[0:64] then sin[0:64]; entries d
     // and d+64 are equal), else cos, then sin
@@ -539,12 +573,12 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   const int mread = kMBase + wu * 64 + lane;
 
   // the mask operands of the tile in mask slot ms (B operand, fp4: first four registers)
-  auto mask_op = [&](int ms) {
+  auto mask_op = [&](int ms) __attribute__((always_inline)) {
     const u32x4 v = dsm[mread + ms * kMSlot];
     return intx8{(int)v[0], (int)v[1], (int)v[2], (int)v[3], 0, 0, 0, 0};
   };
   // S^T of one 32-key half of the tile in K slot ks, starting from its mask product
-  auto s_half = [&](int ks, int c, const intx8& mop) {
+  auto s_half = [&](int ks, int c, const intx8& mop) __attribute__((always_inline)) {
     const u32x4* sK = dsm + ks * kKU + kread;
     bf16x8 f[8];
 #pragma unroll
@@ -569,13 +603,31 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   // runs in a branch the wave takes only when one of its rows moves.
   // exp_half turns a half's scores into P (two B operands of O^T) and adds
   // the bf16 values that the PV product uses to l, one dot2 per pair.
-  auto max_half = [&](const floatx16& acc) -> float {
+  auto max_half = [&](const floatx16& acc) __attribute__((always_inline)) -> float {
     float mx = -__builtin_inff();
 #pragma unroll
     for (int r = 0; r < 16; ++r) mx = fmaxf(mx, acc[r]);
     return mx;                                      // never NaN: the max is seeded with -inf
   };
-  auto exp_half = [&](const floatx16& acc, uint32_t (&pk)[2][4]) {
+  // (kSel: 16 keys at a time, ks = 0, 1; pk[i] = the weights' bf16 parts, i-th
+  // remainder; l sums the weights themselves.)
+  auto exp_split = [&](const floatx16& acc, int ks, uint32_t (&pk)[3][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < 8; r += 2) {
+      float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[8 * ks + r], p.scale_l2, nm));
+      float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[8 * ks + r + 1], p.scale_l2, nm));
+      l += p0;
+      l += p1;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const uint32_t w = pack_bf16(p0, p1);
+        pk[i][r >> 1] = w;
+        p0 -= bf16lo(w);
+        p1 -= bf16hi(w);
+      }
+    }
+  };
+  auto exp_half = [&](const floatx16& acc, uint32_t (&pk)[2][4]) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
       const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(acc[r], p.scale_l2, nm));
@@ -585,13 +637,13 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
       l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), ones2, l, false);
     }
   };
-  auto rescale = [&](float alpha) {
+  auto rescale = [&](float alpha) __attribute__((always_inline)) {
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
   };
-  auto pv_half = [&](int vs, int c, const uint32_t (&pk)[2][4]) {
+  auto pv_half = [&](int vs, int c, const uint32_t (&pk)[2][4]) __attribute__((always_inline)) {
     const u32x4* sV = dsm + vs * kVU + vread;
     bf16x8 f[2][4];
 #pragma unroll
@@ -604,6 +656,19 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
       const bf16x8 pb = __builtin_bit_cast(bf16x8, u32x4{pk[ks][0], pk[ks][1], pk[ks][2], pk[ks][3]});
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[ks][dt], pb, o[dt], 0, 0, 0);
+    }
+  };
+
+  auto pv_split = [&](int vs, int c, int ks, const uint32_t (&pk)[3][4]) __attribute__((always_inline)) {
+    const u32x4* sV = dsm + vs * kVU + vread;
+    bf16x8 f[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) f[dt] = __builtin_bit_cast(bf16x8, sV[32 * dt * kVRow + 4 * c + 2 * ks]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const bf16x8 pb = __builtin_bit_cast(bf16x8, u32x4{pk[i][0], pk[i][1], pk[i][2], pk[i][3]});
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[dt], pb, o[dt], 0, 0, 0);
     }
   };
 
@@ -622,7 +687,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   const char* vsrc = vtb + kDK * 2;                  // V^T tile kt+1
   // Tile kt once both halves' maxima are taken: the softmax decision, P and
   // O^T += V^T(kt) P^T(kt) from V slot vs.
-  auto softmax_pv = [&](int vs, float mx0, float mx1, const floatx16& s0, const floatx16& s1) {
+  auto softmax_pv = [&](int vs, float mx0, float mx1, const floatx16& s0, const floatx16& s1) __attribute__((always_inline)) {
     float mx = max_halves(mx1 > mx0 ? mx1 : mx0);
     mx = mx > kNoKey ? mx * p.scale_l2 : -__builtin_inff();
     // mx > m + kLazy; while m = -inf: any selected key
@@ -635,11 +700,22 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
       mlz = m + kLazy;
       nm = m == -__builtin_inff() ? 0.f : -m;
     }
-    uint32_t pk0[2][4], pk1[2][4];
-    exp_half(s0, pk0);
-    pv_half(vs, 0, pk0);
-    exp_half(s1, pk1);
-    pv_half(vs, 1, pk1);
+    if constexpr (kSel) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          uint32_t pk[3][4];
+          exp_split(c ? s1 : s0, ks, pk);
+          pv_split(vs, c, ks, pk);
+        }
+    } else {
+      uint32_t pk0[2][4], pk1[2][4];
+      exp_half(s0, pk0);
+      pv_half(vs, 0, pk0);
+      exp_half(s1, pk1);
+      pv_half(vs, 1, pk1);
+    }
   };
 
   // S^T of tile kt in sc[kt & 1]: with the loop unrolled by two, each
@@ -657,7 +733,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   // operands and V^T(kt) (issued last iteration) are done and its LDS reads
   // have returned; the barrier publishes every wave's loads and frees K and
   // mask slot P = kt & 1 and V slot 1-P for the next loads.
-  auto sync_issue = [&](int kt, int P) {
+  auto sync_issue = [&](int kt, int P) __attribute__((always_inline)) {
     asm volatile("s_waitcnt vmcnt(0)\n\ts_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (kt + 2 < nkt) {
       issue_k(ksrc, P, kt + 3 == nkt);
@@ -668,11 +744,11 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
     vsrc += kDK * 2;
     // the output-gate rows into the staging tile (free since the q and RoPE
     // reads before the first barrier), awaited at the next barrier
-    if (kt == 0 && (p.flags & GSA_ATTN_OUT_GATE)) stage(p.og + b * p.o_sb + (int64_t)rbase * p.o_st + hd * 128, p.o_st);
+    if (!kSel && kt == 0 && (p.flags & GSA_ATTN_OUT_GATE)) stage(p.og + b * p.o_sb + (int64_t)rbase * p.o_st + hd * 128, p.o_st);
   };
   // One iteration: S^T(kt+1) (stale on the wave's last tile, unused) ||
   // softmax(kt), then PV(kt).
-  auto step = [&](int kt, auto par) {
+  auto step = [&](int kt, auto par) __attribute__((always_inline)) {
     constexpr int P = decltype(par)::value;
     sync_issue(kt, P);
     const intx8 mop = mask_op(1 - P);
@@ -699,6 +775,18 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
 
   // ---- epilogue: normalise, bf16, optional output gate ----
   l = sum_halves(l);
+  if constexpr (kSel) {
+    // l and every sum of the row are finite and l > 0, and its scores stayed
+    // far inside the masks' +-8e36; else the gather kernel computes the row
+    float z = 0.f;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) z = __builtin_fmaf(o[dt][r], 0.f, z);
+    const bool good = l > 0.f && l < __builtin_inff() && z == 0.f && m < 1e28f * p.scale_l2;
+    const int row = q0 + 32 * gw + i32;
+    if (!good && row < p.T) p.redo[(int64_t)b * p.T + row] = 1;
+  }
   // O / l as O * (1/l): one division per row instead of one per element
   // (the product is within 1.5 fp32 ulp of the quotient before the bf16
   // rounding); a row without any selected key (l = 0) gives 0
@@ -717,7 +805,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
       float r[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) r[e] = round_bf16(o[dt][4 * r4 + e] * inv_l);
-      if (p.flags & GSA_ATTN_OUT_GATE) {
+      if (!kSel && (p.flags & GSA_ATTN_OUT_GATE)) {
         const uint2 gw = *xp;
         const float gl[4] = {bf16lo(gw.x), bf16hi(gw.x), bf16lo(gw.y), bf16hi(gw.y)};
 #pragma unroll
@@ -746,7 +834,21 @@ using namespace gsa_host;
 // Per device: the dense kernel's LDS limit has been raised.  (A benign race:
 // concurrent first calls both set the same attribute.)
 static constexpr int kMaxDevices = 64;
-static bool g_dense_lds_set[kMaxDevices] = {};
+
+// Raises the LDS limit of one instantiation on the current device (more than the default 64 KiB per block).
+template <bool kSel>
+static int dense_lds_limit() {
+  static bool done[kMaxDevices] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return GSA_ERR_SHAPE;
+  if (!done[dev]) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gsa::dense_attn_kernel<kSel>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)gsa::kDenseLds);
+    if (e != hipSuccess) return -static_cast<int>(e);
+    done[dev] = true;
+  }
+  return GSA_OK;
+}
 
 namespace {
 int prologue_vt_checks(const void* k, int64_t k_sb, int64_t k_st, const void* v, int64_t v_sb, int64_t v_st,
@@ -841,7 +943,7 @@ gsa::LaneMaskArgs lane_mask_args(const uint32_t* bits, int64_t b_sb, int64_t b_s
   const int G = (int)dense_groups(T, Tkv);
   const int nunits = B * G * ((NT + gsa::kLmTiles - 1) / gsa::kLmTiles);
   const int block_rows = causal ? 32 * gsa::kDenseWaves : 0;
-  return gsa::LaneMaskArgs{bits, b_sb, b_st, T, G, NT, nunits, block_rows, static_cast<gsa::u32x4*>(ws)};
+  return gsa::LaneMaskArgs{bits, b_sb, b_st, T, G, NT, nunits, block_rows, static_cast<gsa::u32x4*>(ws), nullptr};
 }
 
 int launch_lane_masks(const uint32_t* bits, int64_t b_sb, int64_t b_st, int B, int T, int Tkv, int causal,
@@ -878,7 +980,7 @@ extern "C" int gsa_prologue_vt_lane_masks(const void* k, int64_t k_sb, int64_t k
   const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws);
   const int n_pro = B * H * (ldv / 64), n_lm = (l.nunits + 7) / 8;
   if ((int64_t)n_pro + n_lm > 0x7fffffffLL) return GSA_ERR_SHAPE;
-  hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel, dim3(n_pro + n_lm), dim3(256), 0,
+  hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel<false>, dim3(n_pro + n_lm), dim3(256), 0,
                      static_cast<hipStream_t>(stream), a, l, n_pro, n_lm);
   return launch_status();
 }
@@ -938,15 +1040,48 @@ extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
                    static_cast<const uint16_t*>(vt), vt_sb, vt_sh, ldv, (int)G, NT,
                    static_cast<const uint16_t*>(og), o_sb, o_st, static_cast<const uint16_t*>(cos),
                    static_cast<const uint16_t*>(sin), cs_st, static_cast<uint16_t*>(out), out_sb, out_st,
-                   B, T, Tkv, H, nqb, scale * gsa::kLog2e, flags | (causal ? gsa::kDenseCausal : 0)};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return GSA_ERR_SHAPE;
-  if (!g_dense_lds_set[dev]) {   // more than the default 64 KiB of LDS per block
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gsa::dense_attn_kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)gsa::kDenseLds);
-    if (e != hipSuccess) return -static_cast<int>(e);
-    g_dense_lds_set[dev] = true;
-  }
-  hipLaunchKernelGGL(gsa::dense_attn_kernel, dim3(B * H * nqb), dim3(64 * W), gsa::kDenseLds, s, a, lm);
+                   B, T, Tkv, H, nqb, scale * gsa::kLog2e, flags | (causal ? gsa::kDenseCausal : 0), nullptr, nullptr};
+  const int st = dense_lds_limit<false>();
+  if (st) return st;
+  hipLaunchKernelGGL(gsa::dense_attn_kernel<false>, dim3(B * H * nqb), dim3(64 * W), gsa::kDenseLds, s, a, lm);
+  return launch_status();
+}
+
+// Workspace of launch_dense_selected: V^T, then the mask operands.
+static size_t selected_vt_bytes(int B, int Tkv, int H) {
+  return (size_t)B * H * 128 * (size_t)((Tkv + 63) / 64 * 64) * 2;
+}
+size_t gsa_host::dense_selected_bytes(int B, int T, int Tkv, int H) {
+  return selected_vt_bytes(B, Tkv, H) + gsa_dense_attn_workspace_bytes(B, T, Tkv);
+}
+
+// V^T and the mask operands in one launch, then the attention.
+int gsa_host::launch_dense_selected(const AttnShape& s, const gsa::Selection& sel, void* ws, hipStream_t stream) {
+  const int NT = (s.Tkv + 63) / 64, ldv = NT * 64;
+  const int nqb = (s.T + 32 * gsa::kDenseWaves - 1) / (32 * gsa::kDenseWaves);
+  uint16_t* vt = static_cast<uint16_t*>(ws);
+  void* lm = static_cast<char*>(ws) + selected_vt_bytes(s.B, s.Tkv, s.H);
+  int st = dense_lds_limit<true>();
+  if (st) return st;
+  gsa::ProVtArgs p{};
+  p.v = static_cast<const uint16_t*>(s.v); p.v_sb = s.v_sb; p.v_st = s.v_st;
+  p.vt = vt; p.T = s.Tkv; p.H = s.H; p.ldv = ldv; p.ntiles = NT;
+  gsa::LaneMaskArgs l = lane_mask_args(sel.bits, (int64_t)s.T * 2 * NT, 2 * NT, s.B, s.T, s.Tkv, 0, lm);
+  l.range = sel.range;
+  const int n_pro = s.B * s.H * NT, n_lm = (l.nunits + 7) / 8;
+  hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel<true>, dim3(n_pro + n_lm), dim3(256), 0, stream, p, l, n_pro,
+                     n_lm);
+  if ((st = launch_status())) return st;
+  gsa::DenseArgs a{};
+  a.q = static_cast<const uint16_t*>(s.q); a.q_sb = s.q_sb; a.q_st = s.q_st;
+  a.k = static_cast<const uint16_t*>(s.k); a.k_sb = s.k_sb; a.k_st = s.k_st;
+  a.vt = vt; a.vt_sb = (int64_t)s.H * 128 * ldv; a.vt_sh = (int64_t)128 * ldv; a.ldv = ldv;
+  a.G = (int)dense_groups(s.T, s.Tkv); a.NT = NT;
+  a.out = static_cast<uint16_t*>(s.out); a.out_sb = s.out_sb; a.out_st = s.out_st;
+  a.B = s.B; a.T = s.T; a.Tkv = s.Tkv; a.H = s.H; a.nqb = nqb;
+  a.scale_l2 = s.scale * gsa::kLog2e;
+  a.range = sel.range; a.redo = sel.redo;
+  hipLaunchKernelGGL(gsa::dense_attn_kernel<true>, dim3(s.B * s.H * nqb), dim3(64 * gsa::kDenseWaves),
+                     gsa::kDenseLds, stream, a, static_cast<const gsa::u32x4*>(lm));
   return launch_status();
 }

@@ -151,6 +151,34 @@ __device__ __forceinline__ uint32_t score_key(float s) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
+// ---------------------------------------------------------------------------
+// A selection given as index lists, in the form the MFMA attention kernels take
+// (selected_attn.hip writes it, dense_attn.hip and dense_attn_f32.hip read it).
+// ---------------------------------------------------------------------------
+struct Selection {
+  const uint32_t* bits;   // [B*T][W] bitmask, W = 2*ceil(Tkv/64): bit j of a row: key j is selected
+  const int2* range;      // [B*T] first and past-last 64-key tile of the row's keys (none: INT_MAX, 0)
+  uint8_t* redo;          // [B*T] 1: the row's output has to come from the gather kernel
+};
+
+// 64-key tiles [x, y) that hold a selected key of rows r0 .. r1-1 of sequence b
+// (at least one tile), agreed on by the kLanes lanes of an aligned group.
+template <int kLanes>
+__device__ __forceinline__ int2 tile_range(const int2* range, int64_t row_base, int r0, int r1) {
+  int lo = 0x7fffffff, hi = 0;
+  for (int r = r0 + (int)(threadIdx.x & (kLanes - 1)); r < r1; r += kLanes) {
+    const int2 v = range[row_base + r];
+    lo = min(lo, v.x);
+    hi = max(hi, v.y);
+  }
+#pragma unroll
+  for (int o = 1; o < kLanes; o <<= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64));
+    hi = max(hi, __shfl_xor(hi, o, 64));
+  }
+  return hi > lo ? int2{lo, hi} : int2{0, 1};
+}
+
 }  // namespace gsa
 
 // ---------------------------------------------------------------------------
@@ -178,5 +206,27 @@ inline int launch_status() {
 // One launch on `stream`; returns launch_status().
 int launch_adaptive_k(const float* var, int n, int k_base, int k_min, int k_max, int k_cap, int32_t* k_rows,
                       hipStream_t stream);
+
+// Attention over a selection of Tkv keys per row: q, out [B,T,H,128], k, v
+// [B,Tkv,H,128], innermost dimensions contiguous, 16-byte aligned rows.
+struct AttnShape {
+  const void* q; int64_t q_sb, q_st;
+  const void* k; int64_t k_sb, k_st;
+  const void* v; int64_t v_sb, v_st;
+  void* out; int64_t out_sb, out_st;
+  int B, T, Tkv, H;
+  float scale;
+};
+// The index lists a selection came from (idx64: 64-bit indices; count and mask nullable).
+struct IndexLists {
+  const void* idx; int idx64; int64_t i_sb, i_st; int k_sel;
+  const int32_t* count; const uint8_t* mask;
+};
+// bf16 on MFMA (dense_attn.hip); ws: dense_selected_bytes(a) bytes, 256-byte
+// aligned.  Rows it cannot vouch for are marked in sel.redo.
+size_t dense_selected_bytes(int B, int T, int Tkv, int H);
+int launch_dense_selected(const AttnShape& a, const gsa::Selection& sel, void* ws, hipStream_t stream);
+// The gather kernel on the rows marked in `redo` (sparse_attn.hip).
+int launch_gather_rows(const AttnShape& a, const IndexLists& l, const uint8_t* redo, int dtype, hipStream_t stream);
 
 }  // namespace gsa_host

@@ -1,0 +1,161 @@
+// Attention over per-row index lists on the matrix cores (the
+// fused_sparse_attention launcher).
+//
+// The gather kernel (sparse_attn.hip) reads K and V of every selected key once
+// per query row -- 8 KiB per selected key in bf16 at 16 heads, 16 KiB in fp32
+// -- and takes 12.8 ms at T = 8192, k = 2048, where the arithmetic needs 0.1.
+// Here the lists become a bitmask, and the block-dense kernels compute every
+// 64-key tile that holds a selected key of a query block on MFMA, with the
+// bitmask applied to the scores: K and V are read once per 256 query rows
+// (0.50 ms there).
+//
+// Both give the softmax over the selected keys, except where a row's list
+// names a key twice (the lists weigh it twice, a bitmask once) or a value is
+// not finite (a masked tile multiplies it by zero).  Such rows are marked --
+// the first kind here, the second by the attention kernel -- and the gather
+// kernel computes them in a last launch; unmarked rows' blocks end at once.
+#include "gsa_common.h"
+
+#include <algorithm>
+#include <climits>
+
+namespace gsa {
+
+// Index lists -> bitmask, tile range and redo mark of each row: one block per row.
+struct SelRowsArgs {
+  const void* idx; int idx64; int64_t i_sb, i_st; int k_sel;
+  const int32_t* count; const uint8_t* mask;
+  int T, Tkv, W;
+  uint32_t* bits; int2* range; uint8_t* redo;
+};
+
+template <typename IdxT>
+__global__ __launch_bounds__(256) void selected_rows_kernel(SelRowsArgs p) {
+  extern __shared__ uint32_t sw[];           // the row's W words
+  __shared__ int st_lo, st_hi, st_twice;
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+  const int b = row / p.T, t = row % p.T;
+  for (int i = tid; i < p.W; i += 256) sw[i] = 0u;
+  if (tid == 0) { st_lo = INT_MAX; st_hi = 0; st_twice = 0; }
+  __syncthreads();
+  int n = p.k_sel;
+  if (p.count) n = min(n, p.count[row]);
+  const int64_t base = b * p.i_sb + (int64_t)t * p.i_st;
+  const IdxT* irow = static_cast<const IdxT*>(p.idx) + base;
+  const uint8_t* mrow = p.mask ? p.mask + base : nullptr;
+  bool twice = false;
+  for (int m = tid; m < n; m += 256) {
+    if (mrow == nullptr || mrow[m] != 0) {
+      const int j = min(max((int)irow[m], 0), p.Tkv - 1);
+      const uint32_t bit = 1u << (j & 31);
+      twice |= (atomicOr(&sw[j >> 5], bit) & bit) != 0u;
+    }
+  }
+  if (ballot64(twice) && lane == 0) st_twice = 1;
+  __syncthreads();
+  uint32_t* brow = p.bits + (int64_t)row * p.W;
+  int lo = INT_MAX, hi = 0;
+  for (int i = tid; i < p.W; i += 256) {
+    const uint32_t w = sw[i];
+    brow[i] = w;
+    if (w) { lo = min(lo, i >> 1); hi = (i >> 1) + 1; }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    lo = min(lo, __shfl_xor(lo, o, 64));
+    hi = max(hi, __shfl_xor(hi, o, 64));
+  }
+  if (lane == 0 && hi) { atomicMin(&st_lo, lo); atomicMax(&st_hi, hi); }
+  __syncthreads();
+  if (tid == 0) {
+    p.range[row] = int2{st_lo, st_hi};
+    p.redo[row] = (uint8_t)st_twice;
+  }
+}
+
+}  // namespace gsa
+
+using namespace gsa_host;
+
+namespace {
+
+size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+size_t bits_bytes(int B, int T, int Tkv) { return align256((size_t)B * T * ((Tkv + 63) / 64) * 8); }
+
+constexpr size_t kMaxWorkspace = (size_t)4 << 30;
+
+// Whether the matrix-core way is the faster one, from the time each takes (us,
+// measured at 16 heads, bf16).  The gather: 20 + the larger of 0.5 per key of a
+// row (its loads are a chain within the row's block) and 0.0009 per row and
+// key (what it reads); T = 512, k = 128 89; T = 8192, k = 2048 13002.  The
+// matrix cores: 30 for the launches and 2.4 for each 64-key tile of a block's
+// 256 rows, one block per CU at a time: T = 512, k = 128 54; T = 8192, k = 2048
+// 502; T = 256, Tkv = 8192, k = 128 340, where the gather takes 89.  (All Tkv
+// tiles are counted; what a causal selection leaves out is known on the device only.)
+// The masks reach -8e36 times the scale, which has to stay far below every
+// score: a scale outside [1e-10, 1e10] takes the gather.  A row's bits fit the
+// LDS of a block, and the workspace (2 bytes per element of V, 5 bits per row
+// and key) is kept to 4 GiB.
+bool dense_serves(int B, int T, int Tkv, int H, int k_sel, float scale, int dtype) {
+  if (dtype != GSA_DTYPE_BF16) return false;
+  if (!(scale >= 1e-10f && scale <= 1e10f)) return false;
+  if ((size_t)((Tkv + 63) / 64) * 8 > 65536 - 64) return false;
+  const int64_t NT = (Tkv + 63) / 64, groups = ((int64_t)T + 255) / 256 * 8;
+  const double rounds = (double)((B * H * (groups / 8) + 255) / 256);
+  const double gather = 20.0 + std::max(0.5 * k_sel, 0.0009 * B * T * (double)k_sel * H / 16);
+  if (30.0 + 2.4 * NT * rounds > gather) return false;
+  if (B * groups * NT > 0x3fffffffLL / 32 || (int64_t)B * H * NT > 0x3fffffffLL) return false;
+  return bits_bytes(B, T, Tkv) + align256((size_t)B * T * 9) + dense_selected_bytes(B, T, Tkv, H) <= kMaxWorkspace;
+}
+
+}  // namespace
+
+extern "C" size_t gsa_selected_attn_workspace_bytes(int B, int T, int Tkv, int H, int k_sel, float scale, int dtype) {
+  if (B < 1 || T < 1 || Tkv < 1 || H < 1 || H > 64 || !dense_serves(B, T, Tkv, H, k_sel, scale, dtype)) return 0;
+  return bits_bytes(B, T, Tkv) + align256((size_t)B * T * 8) + align256((size_t)B * T) +
+         dense_selected_bytes(B, T, Tkv, H);
+}
+
+extern "C" int gsa_selected_attn(const void* q, int64_t q_sb, int64_t q_st,
+                                 const void* k, int64_t k_sb, int64_t k_st,
+                                 const void* v, int64_t v_sb, int64_t v_st,
+                                 const void* idx, int idx_bytes, int64_t i_sb, int64_t i_st, int k_sel,
+                                 const int32_t* count, const uint8_t* mask,
+                                 void* out, int64_t out_sb, int64_t out_st,
+                                 int B, int T, int Tkv, int H, int d, float scale, int dtype,
+                                 void* ws, size_t ws_bytes, void* stream) {
+  if (!q || !k || !v || !idx || !out || !ws) return GSA_ERR_NULL;
+  if (dtype_size(dtype) == 0) return GSA_ERR_DTYPE;
+  if (B < 1 || T < 1 || Tkv < 1 || d != 128 || H < 1 || H > 64) return GSA_ERR_SHAPE;
+  if ((int64_t)B * T > 0x7fffffffLL) return GSA_ERR_SHAPE;
+  if (k_sel < 0) return GSA_ERR_K;
+  if (idx_bytes != 4 && idx_bytes != 8) return GSA_ERR_DTYPE;
+  const size_t need = gsa_selected_attn_workspace_bytes(B, T, Tkv, H, k_sel, scale, dtype);
+  if (need == 0 || ws_bytes < need) return GSA_ERR_SHAPE;
+  // per-lane load offsets within a tile are 32-bit byte offsets
+  for (const int64_t st : {q_st, k_st, v_st, out_st})
+    if (st < 0 || st > (1 << 24)) return GSA_ERR_SHAPE;
+  if (!vec_ok(q, q_sb, q_st, dtype) || !vec_ok(k, k_sb, k_st, dtype) || !vec_ok(v, v_sb, v_st, dtype) ||
+      !vec_ok(out, out_sb, out_st, dtype) || !aligned(idx, idx_bytes) || (count && !aligned(count, 4)) ||
+      !aligned(ws, 256))
+    return GSA_ERR_ALIGN;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  char* base = static_cast<char*>(ws);
+  uint32_t* bits = reinterpret_cast<uint32_t*>(base);
+  base += bits_bytes(B, T, Tkv);
+  int2* range = reinterpret_cast<int2*>(base);
+  base += align256((size_t)B * T * 8);
+  uint8_t* redo = reinterpret_cast<uint8_t*>(base);
+  base += align256((size_t)B * T);
+  const int W = 2 * ((Tkv + 63) / 64);
+  const gsa::SelRowsArgs r{idx, idx_bytes == 8, i_sb, i_st, k_sel, count, mask, T, Tkv, W, bits, range, redo};
+  if (idx_bytes == 8)
+    hipLaunchKernelGGL(gsa::selected_rows_kernel<int64_t>, dim3(B * T), dim3(256), (size_t)W * 4, s, r);
+  else
+    hipLaunchKernelGGL(gsa::selected_rows_kernel<int32_t>, dim3(B * T), dim3(256), (size_t)W * 4, s, r);
+  int st = launch_status();
+  if (st) return st;
+  const AttnShape a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, out, out_sb, out_st, B, T, Tkv, H, scale};
+  if ((st = launch_dense_selected(a, gsa::Selection{bits, range, redo}, base, s))) return st;
+  return launch_gather_rows(a, IndexLists{idx, idx_bytes == 8, i_sb, i_st, k_sel, count, mask}, redo, dtype, s);
+}

@@ -69,6 +69,8 @@ struct AttnArgs {
   int T, Tkv;
   float scale_l2;   // scale * log2(e): scores live in the log2 domain
   int flags;
+  const uint8_t* redo;   // kRows: the rows to compute ([B*T], nonzero)
+  int idx64;             // kRows: idx holds 64-bit indices
 };
 
 // One key row slice for this lane: 8 elements as raw storage.
@@ -128,11 +130,15 @@ struct QReg {
 template <typename T> struct Chunk { static constexpr int kKeys = 8; };
 template <> struct Chunk<float> { static constexpr int kKeys = 4; };
 
-template <typename T, int kThreads>
+// kRows: only the rows marked in `redo` (the others' blocks end at once), with
+// 32- or 64-bit indices (a 64-bit index counts by its low 32 bits).
+template <typename T, int kThreads, bool kRows>
 __global__ __launch_bounds__(kThreads) void sparse_attn_kernel(AttnArgs p) {
   // keys in flight per buffer; halved for 1024-thread blocks (128-VGPR budget)
   constexpr int C = kThreads > 256 ? Chunk<T>::kKeys / 2 : Chunk<T>::kKeys;
   const int row = blockIdx.x;
+  if constexpr (kRows)
+    if (!p.redo[row]) return;
   const int b = row / p.T, t = row % p.T;
   const int li = threadIdx.x & 15;
   const int e0 = threadIdx.x * 8;   // head*128 + li*8
@@ -149,7 +155,13 @@ __global__ __launch_bounds__(kThreads) void sparse_attn_kernel(AttnArgs p) {
   QReg q;
   q.set(xq);
 
-  const int32_t* irow = p.idx + b * p.i_sb + (int64_t)t * p.i_st;
+  const int64_t ibase = b * p.i_sb + (int64_t)t * p.i_st;
+  const int32_t* irow = p.idx + ibase;
+  auto index = [&](int mm) -> int {
+    if constexpr (kRows)
+      if (p.idx64) return (int)reinterpret_cast<const int64_t*>(p.idx)[ibase + mm];
+    return irow[mm];
+  };
   const uint8_t* mrow = p.mask ? p.mask + b * p.i_sb + (int64_t)t * p.i_st : nullptr;
   int n = p.k_sel;
   if (p.count) n = min(n, p.count[row]);
@@ -170,7 +182,7 @@ __global__ __launch_bounds__(kThreads) void sparse_attn_kernel(AttnArgs p) {
       const int mm = c0 + u;
       ok[u] = mm < n && (mrow == nullptr || mrow[mm] != 0);
       if (ok[u]) {
-        const int j = min(max(irow[mm], 0), p.Tkv - 1);
+        const int j = min(max(index(mm), 0), p.Tkv - 1);
         kr[u].load(kb + (int64_t)j * p.k_st);
         vr[u].load(vb + (int64_t)j * p.v_st);
       }
@@ -260,6 +272,19 @@ extern "C" int gsa_prologue(const void* k, int64_t k_sb, int64_t k_st,
   return launch_status();
 }
 
+template <bool kRows>
+static int launch_gather(const gsa::AttnArgs& a, int B, int H, int dtype, hipStream_t s) {
+  const dim3 grid(B * a.T), block(16 * H);
+  if (dtype == GSA_DTYPE_BF16) {
+    if (H <= 16) hipLaunchKernelGGL((gsa::sparse_attn_kernel<uint16_t, 256, kRows>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((gsa::sparse_attn_kernel<uint16_t, 1024, kRows>), grid, block, 0, s, a);
+  } else {
+    if (H <= 16) hipLaunchKernelGGL((gsa::sparse_attn_kernel<float, 256, kRows>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((gsa::sparse_attn_kernel<float, 1024, kRows>), grid, block, 0, s, a);
+  }
+  return launch_status();
+}
+
 extern "C" int gsa_sparse_attn(const void* q, int64_t q_sb, int64_t q_st,
                                const void* k, int64_t k_sb, int64_t k_st,
                                const void* v, int64_t v_sb, int64_t v_st,
@@ -287,15 +312,15 @@ extern "C" int gsa_sparse_attn(const void* q, int64_t q_sb, int64_t q_st,
     return GSA_ERR_ALIGN;
   gsa::AttnArgs a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, idx, i_sb, i_st, k_sel, count, mask,
                   og, o_sb, o_st, cos, sin, cs_st, out, out_sb, out_st, T, Tkv,
-                  scale * gsa::kLog2e, flags};
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid(B * T), block(16 * H);
-  if (dtype == GSA_DTYPE_BF16) {
-    if (H <= 16) hipLaunchKernelGGL((gsa::sparse_attn_kernel<uint16_t, 256>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((gsa::sparse_attn_kernel<uint16_t, 1024>), grid, block, 0, s, a);
-  } else {
-    if (H <= 16) hipLaunchKernelGGL((gsa::sparse_attn_kernel<float, 256>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((gsa::sparse_attn_kernel<float, 1024>), grid, block, 0, s, a);
-  }
-  return launch_status();
+                  scale * gsa::kLog2e, flags, nullptr, 0};
+  return launch_gather<false>(a, B, H, dtype, static_cast<hipStream_t>(stream));
+}
+
+int gsa_host::launch_gather_rows(const AttnShape& s, const IndexLists& l, const uint8_t* redo, int dtype,
+                                 hipStream_t stream) {
+  gsa::AttnArgs a{s.q, s.q_sb, s.q_st, s.k, s.k_sb, s.k_st, s.v, s.v_sb, s.v_st,
+                  static_cast<const int32_t*>(l.idx), l.i_sb, l.i_st, l.k_sel, l.count, l.mask,
+                  nullptr, 0, 0, nullptr, nullptr, 0, s.out, s.out_sb, s.out_st, s.T, s.Tkv,
+                  s.scale * gsa::kLog2e, 0, redo, l.idx64};
+  return launch_gather<true>(a, s.B, s.H, dtype, stream);
 }

@@ -73,10 +73,8 @@ def fused_sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     """
     _range_push("gsa_hip/sparse_attn")
     try:
-        idx = indices.to(torch.int32).contiguous()
-        m = mask.to(torch.uint8).contiguous()
         q, k, v = (t if t.stride(-1) == 1 else t.contiguous() for t in (q, k, v))
-        return _abi.sparse_attn(q, k, v, idx, scale, mask=m)
+        return _abi.selected_attn(q, k, v, indices, scale, mask=mask)
     finally:
         _range_pop()
 

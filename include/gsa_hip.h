@@ -286,6 +286,32 @@ int gsa_sparse_attn(const void* q, int64_t q_sb, int64_t q_st,
                     void* stream);
 
 /*
+ * gsa_sparse_attn without RoPE and gate, for the sizes where the matrix cores
+ * serve it: fused_sparse_attention (gsa_triton/gsa_opt.py:349-383), same
+ * selection rules (count, mask, clamped indices; a key listed twice counts
+ * twice) and outputs.  The lists become a bitmask, the block-dense attention
+ * computes every 64-key tile that holds a selected key of a query block, and
+ * rows that a bitmask cannot express (a key listed twice) or whose sums are not
+ * finite are computed by gsa_sparse_attn's kernel; four launches in stream order.
+ * idx: 32- or 64-bit indices (idx_bytes 4 or 8; a 64-bit index counts by its
+ * low 32 bits), mask uint8 or bool bytes with idx's strides.
+ * gsa_selected_attn_workspace_bytes is 0 where gsa_sparse_attn is the one to
+ * call: see selected_attn.hip for the rule (sizes, k_sel / Tkv and scale);
+ * gsa_selected_attn then returns GSA_ERR_SHAPE, as it does for row strides of
+ * q, k, v or out beyond 2^24 elements.  ws: 256-byte aligned, overwritten.
+ */
+size_t gsa_selected_attn_workspace_bytes(int B, int T, int Tkv, int H, int k_sel, float scale, int dtype);
+
+int gsa_selected_attn(const void* q, int64_t q_sb, int64_t q_st,
+                      const void* k, int64_t k_sb, int64_t k_st,
+                      const void* v, int64_t v_sb, int64_t v_st,
+                      const void* idx, int idx_bytes, int64_t i_sb, int64_t i_st, int k_sel,
+                      const int32_t* count, const uint8_t* mask,
+                      void* out, int64_t out_sb, int64_t out_st,
+                      int B, int T, int Tkv, int H, int d, float scale, int dtype,
+                      void* ws, size_t ws_bytes, void* stream);
+
+/*
  * Producer for the block-dense attention: RoPE on k (k == NULL skips it) and
  * the G2 gate with V written transposed.  Replaces gsa_triton/gsa_opt.py:
  * 685-697 like gsa_prologue, with the value output laid out for

@@ -1,0 +1,133 @@
+"""fused_sparse_attention on the matrix cores (gsa_selected_attn) against float64 and
+against the gather kernel, whose semantics it keeps.
+
+Bound, bf16: the weights are exact to 2^-17 and the sums are fp32, so an output is
+within one rounding to bf16 (half an ulp, 2^-9 relative, and 2^-8 allowed for a
+value at a rounding boundary) of the float64 result plus fp32 sum error of
+sum_j p_j |v_j| <= max|v|, far below 2^-16 max|v|.
+"""
+
+import pytest
+import torch
+
+from gsa_gdn_benchmarkstudy_amd import _abi
+from gsa_gdn_benchmarkstudy_amd import gsa as G
+
+pytestmark = pytest.mark.gpu
+SCALE = 128 ** -0.5
+
+
+def _log(msg):
+    print(msg, flush=True)
+
+
+def _selection(B, T, Tkv, K, seed, kind):
+    """idx int64 [B,T,K] without repeats per row, mask bool."""
+    g = torch.Generator().manual_seed(seed)
+    r = torch.rand(B, T, Tkv, generator=g)
+    if kind == "causal":
+        r.masked_fill_(torch.ones(T, Tkv, dtype=torch.bool).triu_(1), -1.0)
+    elif kind == "window":          # keys near 2t: the blocks' tiles start past 0 and end before the last
+        d = torch.arange(Tkv)[None, :] - 2 * torch.arange(T)[:, None]
+        r.masked_fill_(d.abs() > K, -1.0)
+    val, idx = r.topk(K, dim=-1)
+    return idx, val >= 0
+
+
+def _attend64(q, k, v, idx, mask, scale):
+    """Every list entry weighs once: counts of repeats multiply exp(s)."""
+    B, T, H, d = q.shape
+    n = torch.zeros(B, T, k.shape[1], dtype=torch.float64, device=q.device)
+    n.scatter_add_(2, idx.clamp(0, k.shape[1] - 1), mask.double())
+    out = torch.zeros(B, T, H, d, dtype=torch.float64, device=q.device)
+    for b in range(B):
+        for h in range(H):
+            s = (q[b, :, h].double() @ k[b, :, h].double().t().contiguous()) * scale
+            s = s + torch.log(n[b])
+            p = torch.softmax(s, dim=-1).nan_to_num(0.0)
+            out[b, :, h] = p @ v[b, :, h].double()
+    return out
+
+
+def _close(out, ref, v, dtype):
+    err = (out.double() - ref).abs()
+    if dtype == torch.bfloat16:
+        bound = ref.abs() * 2.0 ** -8 + v.abs().max().double() * 2.0 ** -16
+    else:
+        # fp32: scores of up to about 8 in log2 units carry 128-term dot products
+        # (128 * 2^-24 relative to sum |q_i k_i|), which enter the weights linearly
+        bound = ref.abs() * 2e-5 + v.abs().max().double() * 1e-5
+    assert torch.all(err <= bound), float((err - bound).max())
+
+
+DTYPES = [torch.bfloat16]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("B,T,Tkv,H,K,kind", [
+    (1, 64, 64, 4, 64, "causal"), (2, 129, 129, 2, 60, "causal"), (1, 255, 255, 1, 100, "causal"),
+    (1, 257, 257, 3, 64, "causal"), (1, 700, 700, 2, 96, "causal"), (2, 300, 1000, 2, 100, "any"),
+    (1, 513, 1100, 2, 120, "window"), (1, 1000, 65, 2, 50, "any"), (1, 100, 2100, 40, 200, "any"),
+])
+def test_selected_attention_vs_float64(dev, dtype, B, T, Tkv, H, K, kind):
+    _log(f"selected attention {dtype} B={B} T={T} Tkv={Tkv} H={H} K={K} {kind}")
+    g = torch.Generator().manual_seed(T + Tkv)
+    q = torch.randn(B, T, H, 128, generator=g).to(dtype).to(dev)
+    kv = torch.randn(B, Tkv, 2 * H + 1, 128, generator=g).to(dtype).to(dev)   # k, v: strided views of one buffer
+    k, v = kv[:, :, :H], kv[:, :, H:2 * H]
+    idx, mask = _selection(B, T, Tkv, K, seed=7, kind=kind)
+    idx, mask = idx.to(dev), mask.to(dev)
+    assert _abi.load().gsa_selected_attn_workspace_bytes(B, T, Tkv, H, K, SCALE, _abi.dtype_code(dtype)) > 0
+    out = G.fused_sparse_attention(q, k, v, idx, mask, SCALE)
+    assert out.dtype == dtype and out.shape == q.shape
+    ref = _attend64(q, k, v, idx, mask, SCALE)
+    _close(out, ref, v, dtype)
+    # another order of the same keys, 32-bit indices: the same bits
+    perm = torch.randperm(K, generator=g).to(dev)
+    again = G.fused_sparse_attention(q, k, v, idx[..., perm].int(), mask[..., perm], SCALE)
+    assert torch.equal(again, out)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_selected_attention_rows_for_the_gather(dev, dtype):
+    """Rows a bitmask cannot express, and values a masked tile cannot skip: keys listed
+    twice, indices outside [0, Tkv), rows without a valid key, infinities and NaN in k
+    and v (selected by some rows and not by others), products past the mask's range.
+    The marked rows equal the gather kernel's bit for bit, the others the same call
+    without them."""
+    B, T, H, K = 1, 320, 2, 60
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(B, T, H, 128, generator=g).to(dtype) for _ in range(3))
+    idx, mask = _selection(B, T, T, K, seed=5, kind="any")
+    idx[0, 10, 3] = idx[0, 10, 4]                 # twice
+    mask[0, 11] = False                           # no key
+    idx[0, 12, 0], idx[0, 12, 1] = -5, T + 9      # clamped to 0 and T - 1
+    idx[0, 13, 0] = 2 ** 32 + 17                  # counts by its low 32 bits
+    qd, kd, vd, idx, mask = (t.to(dev) for t in (q, k, v, idx, mask))
+    plain = G.fused_sparse_attention(qd, kd, vd, idx, mask, SCALE)
+    gather = _abi.sparse_attn(qd, kd, vd, idx.to(torch.int32), SCALE, mask=mask.to(torch.uint8))
+    assert torch.equal(plain[0, 10], gather[0, 10]) and torch.all(plain[0, 11] == 0)
+    _close(plain, _attend64(qd, kd, vd, idx.to(torch.int32).long(), mask, SCALE), vd, dtype)
+
+    for where, what in (("v", float("inf")), ("v", float("nan")), ("k", float("inf")), ("k", float("nan")),
+                        ("k", 3e38), ("q", float("nan")), ("q", 1e30)):
+        kk, vv, qq = kd.clone(), vd.clone(), qd.clone()
+        {"k": kk, "v": vv, "q": qq}[where][0, 200, 1, 5] = what
+        out = G.fused_sparse_attention(qq, kk, vv, idx, mask, SCALE)
+        ref = _abi.sparse_attn(qq, kk, vv, idx.to(torch.int32), SCALE, mask=mask.to(torch.uint8))
+        _log(f"  {where} {what}")
+        assert torch.equal(torch.isfinite(out), torch.isfinite(ref))
+        fin = torch.isfinite(ref)
+        assert torch.allclose(out[fin].double(), ref[fin].double(), rtol=2.0 ** -7, atol=2.0 ** -14)
+        assert torch.equal(out[~fin].isnan(), ref[~fin].isnan())
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.5, 1e-20, 1e20])
+def test_selected_attention_scales_for_the_gather(dev, scale):
+    """Scales for which a masked score would not vanish take the gather kernel: same bits."""
+    B, T, H, K = 1, 130, 2, 60
+    g = torch.Generator().manual_seed(3)
+    q, k, v = (torch.randn(B, T, H, 128, generator=g).bfloat16().to(dev) for _ in range(3))
+    idx, mask = (t.to(dev) for t in _selection(B, T, T, K, seed=5, kind="any"))
+    out = G.fused_sparse_attention(q, k, v, idx, mask, scale)
+    assert torch.equal(out, _abi.sparse_attn(q, k, v, idx.int(), scale, mask=mask.to(torch.uint8)))
