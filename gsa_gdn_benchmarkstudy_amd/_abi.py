@@ -41,7 +41,7 @@ EXPORTS = (
     "gsa_proj_packed_bytes", "gsa_proj_pack", "gsa_proj_fused", "gsa_dense_lane_masks",
     "gsa_prologue_vt_lane_masks", "gsa_debug_force_select_fallback",
     "gsa_indexer_select_noalloc", "gsa_indexer_select_noalloc_max_bytes", "gsa_topk_select_i64",
-    "gsa_selected_attn", "gsa_selected_attn_workspace_bytes",
+    "gsa_selected_attn", "gsa_selected_attn_workspace_bytes", "gsa_masked_attn", "gsa_masked_attn_workspace_bytes",
 )
 
 _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
@@ -78,6 +78,9 @@ _PROTOS = {
     "gsa_selected_attn": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i32, _i64, _i64, _i32, _vp, _vp,
                            _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _vp, ctypes.c_size_t, _vp],
                           _i32),
+    "gsa_masked_attn_workspace_bytes": ([_i32, _i32, _i32, _i32, _i32], ctypes.c_size_t),
+    "gsa_masked_attn": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i32, _vp, _i64, _i64, _vp, _vp, _i64,
+                         _vp, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _vp, ctypes.c_size_t, _vp], _i32),
     "gsa_prologue_vt": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64,
                          _i32, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp], _i32),
     "gsa_selection_mask": ([_vp, _i64, _i64, _i32, _vp, _vp, _i32, _i32, _i32, _vp, _i64, _i64, _vp], _i32),
@@ -513,6 +516,42 @@ def selected_attn(q, k, v, idx, scale: float, mask=None) -> torch.Tensor:
                                _ptr(out), *_rows(out, HD), B, T, Tkv, H, d, float(scale), dtype_code(q.dtype),
                                _ptr(ws), need, _stream(q))
     _check(st, "gsa_selected_attn")
+    return out
+
+
+def masked_attn_serves(B: int, T: int, H: int, k_sel: int, dtype: torch.dtype) -> bool:
+    """Whether masked_attn is the faster way at these sizes (fp32; the library's rule)."""
+    return load().gsa_masked_attn_workspace_bytes(B, T, H, k_sel, dtype_code(dtype)) > 0
+
+
+def masked_attn(q, k, v, bits, k_sel: int, scale: float, og=None, cos=None, sin=None, flags: int = 0) -> torch.Tensor:
+    """fp32 attention over a causal selection bitmask (at most k_sel keys per row)
+    -> out [B,T,H,d]; flags as in sparse_attn."""
+    lib = load()
+    _need_cuda(q, k, v, bits, og, cos, sin)
+    B, T, H, d = q.shape
+    HD = H * d
+    _expect(tuple(k.shape) == tuple(q.shape) and tuple(v.shape) == tuple(q.shape), "k, v: q's shape")
+    _expect(k.dtype == v.dtype == q.dtype, "q, k, v must share a dtype")
+    _expect(tuple(bits.shape) == (B, T, mask_words(T)) and bits.is_contiguous() and bits.dtype == torch.int32,
+            "bits: contiguous int32 [B,T,W]")
+    if og is not None:
+        _expect(tuple(og.shape) == (B, T, H, d) and og.dtype == q.dtype, "og: [B,T,H,d] in q's dtype")
+    if flags & ATTN_ROPE_Q:
+        _expect(cos is not None and sin is not None and cos.dim() == 2 and cos.shape[0] >= T
+                and cos.shape[1] == d and tuple(sin.shape) == tuple(cos.shape)
+                and cos.dtype == sin.dtype == q.dtype and cos.stride(1) == 1 and sin.stride() == cos.stride(),
+                "cos/sin: [>=T, d] in q's dtype")
+    need = lib.gsa_masked_attn_workspace_bytes(B, T, H, int(k_sel), dtype_code(q.dtype))
+    _expect(need > 0, "these sizes take sparse_attn")
+    ws = torch.empty(need, device=q.device, dtype=torch.uint8)
+    out = torch.empty(B, T, H, d, device=q.device, dtype=q.dtype)
+    os_ = _rows(og, HD) if og is not None else (0, 0)
+    cs = cos.stride(0) if cos is not None else 0
+    st = lib.gsa_masked_attn(_ptr(q), *_rows(q, HD), _ptr(k), *_rows(k, HD), _ptr(v), *_rows(v, HD), _ptr(bits),
+                             int(k_sel), _ptr(og), *os_, _ptr(cos), _ptr(sin), cs, _ptr(out), *_rows(out, HD),
+                             B, T, H, d, float(scale), dtype_code(q.dtype), int(flags), _ptr(ws), need, _stream(q))
+    _check(st, "gsa_masked_attn")
     return out
 
 

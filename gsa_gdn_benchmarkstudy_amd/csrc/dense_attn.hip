@@ -295,46 +295,7 @@ constexpr size_t kDenseLds = (size_t)(kXBase + 512 * kDenseWaves) * 16;
 // are both conflict-free.  Unit offset of (row, chunk) within the tile:
 __device__ __forceinline__ int xs_unit(int row, int chunk) { return row * 16 + (chunk ^ (row & 15)); }
 
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef int intx8 __attribute__((ext_vector_type(8)));
-
-// Value of lane l^32 combined with the own value: permlane32_swap of (v, v)
-// leaves {v[l], v[l^32]} in the two results on every lane.  max_halves takes
-// values that are never NaN (maxima seeded with -inf), so a compare-select
-// is enough (fmaxf would first quiet both operands).
-__device__ __forceinline__ float max_halves(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  const float a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
-  return a > b ? a : b;
-}
-__device__ __forceinline__ float sum_halves(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// 32-bit LDS address of a shared-memory pointer.
-__device__ __forceinline__ uint32_t lds_addr(const void* ptr) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)ptr;
-}
-
-// Direct global -> LDS load: every lane's 16 bytes at base + voff land at
-// lds + 16 * lane (base and lds uniform).  Issued as inline asm so that the
-// compiler's own bookkeeping does not make each LDS read wait for every such
-// load in flight; completion is awaited explicitly (vmcnt) before the
-// barrier that publishes a tile.  m0 holds the LDS address; nothing else in
-// this kernel uses m0.  An LDS DMA reads m0 one wait state after the SALU
-// write at the earliest (the s_nop; the compiler pads its own LDS DMA the
-// same way on gfx950).
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void load_lds16(const void* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-// s_waitcnt immediate (gfx9 encoding): vmcnt(0), expcnt and lgkmcnt not waited
-constexpr int kWaitVmcnt0 = (0x7 << 4) | (0xf << 8);
 
 __device__ __forceinline__ int swap_bits23(int i) { return (i & ~12) | ((i & 4) << 1) | ((i & 8) >> 1); }
 
@@ -785,7 +746,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
       for (int r = 0; r < 16; ++r) z = __builtin_fmaf(o[dt][r], 0.f, z);
     const bool good = l > 0.f && l < __builtin_inff() && z == 0.f && m < 1e28f * p.scale_l2;
     const int row = q0 + 32 * gw + i32;
-    if (!good && row < p.T) p.redo[(int64_t)b * p.T + row] = 1;
+    if (row < p.T) mark_row(p.redo + ((int64_t)b * p.T + row) * p.H + hd, good);
   }
   // O / l as O * (1/l): one division per row instead of one per element
   // (the product is within 1.5 fp32 ulp of the quotient before the bf16

@@ -14,6 +14,7 @@
 namespace gsa {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -152,14 +153,63 @@ __device__ __forceinline__ uint32_t score_key(float s) {
 }
 
 // ---------------------------------------------------------------------------
-// A selection given as index lists, in the form the MFMA attention kernels take
-// (selected_attn.hip writes it, dense_attn.hip and dense_attn_f32.hip read it).
+// Helpers of the block-dense attention kernels (lane l and l^32: one query row)
+// ---------------------------------------------------------------------------
+// Value of lane l^32 combined with the own value: permlane32_swap of (v, v)
+// leaves {v[l], v[l^32]} in the two results on every lane.  max_halves takes
+// values that are never NaN (maxima seeded with -inf), so a compare-select
+// is enough (fmaxf would first quiet both operands).
+__device__ __forceinline__ float max_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  const float a = __uint_as_float(r[0]), b = __uint_as_float(r[1]);
+  return a > b ? a : b;
+}
+__device__ __forceinline__ float sum_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// 32-bit LDS address of a shared-memory pointer.
+__device__ __forceinline__ uint32_t lds_addr(const void* ptr) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)ptr;
+}
+
+// Direct global -> LDS load: every lane's 16 bytes at base + voff land at
+// lds + 16 * lane (base and lds uniform).  Issued as inline asm so that the
+// compiler's own bookkeeping does not make each LDS read wait for every such
+// load in flight; completion is awaited explicitly (vmcnt) before the
+// barrier that publishes a tile.  m0 holds the LDS address; nothing else in
+// this kernel uses m0.  An LDS DMA reads m0 one wait state after the SALU
+// write at the earliest (the s_nop; the compiler pads its own LDS DMA the
+// same way on gfx950).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void load_lds16(const void* base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
+// s_waitcnt immediate (gfx9 encoding): vmcnt(0), expcnt and lgkmcnt not waited
+constexpr int kWaitVmcnt0 = (0x7 << 4) | (0xf << 8);
+
+// ---------------------------------------------------------------------------
+// A selection in the form that the MFMA attention kernels take, and the marks
+// of what the gather kernel has to compute after them.
 // ---------------------------------------------------------------------------
 struct Selection {
   const uint32_t* bits;   // [B*T][W] bitmask, W = 2*ceil(Tkv/64): bit j of a row: key j is selected
   const int2* range;      // [B*T] first and past-last 64-key tile of the row's keys (none: INT_MAX, 0)
-  uint8_t* redo;          // [B*T] 1: the row's output has to come from the gather kernel
+  const uint8_t* twice;   // [B*T] nonzero: the row's list names a key twice, so the bitmask cannot stand for it (or null)
+  uint8_t* redo;          // [B*T*H] written by the attention kernel: nonzero: that head of the row has to come from the gather kernel
 };
+
+// The two lanes of a row agree on its redo mark and write it.
+__device__ __forceinline__ void mark_row(uint8_t* mark, bool good) {
+  const uint32_t g = good ? 1u : 0u;
+  const auto r = __builtin_amdgcn_permlane32_swap(g, g, false, false);
+  *mark = (uint8_t)((r[0] & r[1]) ^ 1u);
+}
 
 // 64-key tiles [x, y) that hold a selected key of rows r0 .. r1-1 of sequence b
 // (at least one tile), agreed on by the kLanes lanes of an aligned group.
@@ -216,17 +266,28 @@ struct AttnShape {
   void* out; int64_t out_sb, out_st;
   int B, T, Tkv, H;
   float scale;
+  // RoPE of q and the output gate, by GSA_ATTN_ROPE_Q and GSA_ATTN_OUT_GATE
+  const void* og; int64_t o_sb, o_st;
+  const void* cos; const void* sin; int64_t cs_st;
+  int flags;
 };
 // The index lists a selection came from (idx64: 64-bit indices; count and mask nullable).
 struct IndexLists {
   const void* idx; int idx64; int64_t i_sb, i_st; int k_sel;
   const int32_t* count; const uint8_t* mask;
 };
-// bf16 on MFMA (dense_attn.hip); ws: dense_selected_bytes(a) bytes, 256-byte
-// aligned.  Rows it cannot vouch for are marked in sel.redo.
+// bf16 on MFMA (dense_attn.hip), without RoPE and gate; ws:
+// dense_selected_bytes bytes, 256-byte aligned.
 size_t dense_selected_bytes(int B, int T, int Tkv, int H);
 int launch_dense_selected(const AttnShape& a, const gsa::Selection& sel, void* ws, hipStream_t stream);
-// The gather kernel on the rows marked in `redo` (sparse_attn.hip).
-int launch_gather_rows(const AttnShape& a, const IndexLists& l, const uint8_t* redo, int dtype, hipStream_t stream);
+// fp32 on MFMA (dense_attn_f32.hip); sel.range null: a causal selection.
+int launch_dense_f32(const AttnShape& a, const gsa::Selection& sel, hipStream_t stream);
+// The gather kernel on what sel.twice and sel.redo mark (sparse_attn.hip).
+int launch_gather_rows(const AttnShape& a, const IndexLists& l, const gsa::Selection& sel, int dtype,
+                       hipStream_t stream);
+// Ascending indices [B*T][k_sel] and counts of the rows of a causal bitmask
+// [B*T][2*ceil(T/64)] that `redo` ([B*T*H]) marks (indexer.hip).
+int launch_marked_indices(const uint32_t* bits, int B, int T, int k_sel, const uint8_t* redo, int H, int32_t* idx,
+                          int32_t* count, hipStream_t stream);
 
 }  // namespace gsa_host

@@ -312,9 +312,6 @@ constexpr int kMaxSelectT = 65536;
 
 enum RowMode : int { kNone = 0, kTrivial = 1, kActive = 2, kFailed = 3 };
 
-// s_waitcnt immediate (gfx9 encoding): vmcnt(0), expcnt and lgkmcnt not waited.
-constexpr int kWaitVmcnt0 = (0x7 << 4) | (0xf << 8);
-
 __device__ __forceinline__ int bin_of(float s, float inv_w) {
   return (int)fmaxf(0.f, fminf(s * inv_w, (float)(kNB - 1)));
 }
@@ -1015,15 +1012,18 @@ __global__ __launch_bounds__(kGroupThreads) void indexer_select_kernel(IdxArgs p
 // t+2, ... up to entry k_t - 1 (the lowest-index invalid entries, as the
 // selector orders them; entries below k_t past n exist only when t+1 < k_t,
 // so these stay below k_t <= T), then index 0 in entries k_t .. k_eff - 1
-// (like the adaptive standalone selector's entries past k_t).
+// (like the adaptive standalone selector's entries past k_t).  With `redo`
+// ([B*T*H]) only the rows that have a nonzero mark are written.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void bits_to_indices_kernel(const uint32_t* __restrict__ bits, int64_t b_sb,
                                                               int64_t b_st, int T, int W, int k_eff,
                                                               const int32_t* __restrict__ k_rows,
                                                               int32_t* __restrict__ idx_out,
-                                                              int32_t* __restrict__ count_out) {
+                                                              int32_t* __restrict__ count_out,
+                                                              const uint8_t* __restrict__ redo, int H) {
   __shared__ int wave_tot[4];
   const int row = blockIdx.x;
+  if (redo && !__syncthreads_or((int)threadIdx.x < H ? redo[(int64_t)row * H + threadIdx.x] : 0)) return;
   const int b = row / T, t = row % T;
   const uint32_t* brow = bits + b * b_sb + (int64_t)t * b_st;
   int32_t* orow = idx_out + (int64_t)row * k_eff;
@@ -1218,6 +1218,14 @@ extern "C" int gsa_debug_force_select_fallback(int on) {
   return g_force_fallback.exchange(on ? 1 : 0);
 }
 
+int gsa_host::launch_marked_indices(const uint32_t* bits, int B, int T, int k_sel, const uint8_t* redo, int H,
+                                    int32_t* idx, int32_t* count, hipStream_t stream) {
+  const int W = 2 * ((T + 63) / 64);
+  hipLaunchKernelGGL(gsa::bits_to_indices_kernel, dim3(B * T), dim3(256), 0, stream, bits, (int64_t)T * W, (int64_t)W,
+                     T, W, k_sel, nullptr, idx, count, redo, H);
+  return launch_status();
+}
+
 int gsa_host::launch_adaptive_k(const float* var, int n, int k_base, int k_min, int k_max, int k_cap,
                                 int32_t* k_rows, hipStream_t stream) {
   hipLaunchKernelGGL(gsa::adaptive_k_kernel, dim3(1), dim3(1024), 0, stream, var, n, k_base, k_min, k_max, k_cap,
@@ -1251,7 +1259,7 @@ static int select_fixed(const gsa::IdxArgs& a, int k_eff, int dtype, uint32_t* b
   if (st || !idx_out) return st;
   const int W = 2 * ((a.T + 63) / 64);
   hipLaunchKernelGGL(gsa::bits_to_indices_kernel, dim3(a.B * a.T), dim3(256), 0, s, bits, b_sb, b_st, a.T, W,
-                     k_eff, nullptr, idx_out, count_out);
+                     k_eff, nullptr, idx_out, count_out, nullptr, 0);
   return launch_status();
 }
 
@@ -1369,6 +1377,6 @@ extern "C" int gsa_indexer_select_adaptive(const void* q_idx, int64_t q_sb, int6
   if (st || !idx_out) return st;
   const int W = 2 * ((T + 63) / 64);
   hipLaunchKernelGGL(gsa::bits_to_indices_kernel, dim3(B * T), dim3(256), 0, s, bits, b_sb, b_st, T, W, k_cap,
-                     krow, idx_out, count_out);
+                     krow, idx_out, count_out, nullptr, 0);
   return launch_status();
 }

@@ -95,26 +95,11 @@ __global__ __launch_bounds__(256) void pack_kernel(const uint16_t* __restrict__ 
   if (u < 5 * D) bp[u] = bias ? bf16lo(bias[packed_source_row((int)u, D)]) : 0.f;
 }
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// Direct global -> LDS load: each lane's 16 bytes at base + voff land at
-// lds + 16 * lane.  Completion is awaited with explicit vmcnt waits.  The
-// s_nop is the wait state an LDS DMA needs after the SALU write of m0.
-__device__ __forceinline__ void load_lds16(const void* base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "s"(lds)
-               : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
 // s_waitcnt vmcnt(N) (gfx9 encoding, N < 64); expcnt and lgkmcnt not waited.
 template <int N>
 __device__ __forceinline__ void wait_vm() {
   static_assert(N >= 0 && N < 64, "vmcnt");
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0xf << 8));
-}
-
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
 }
 
 __device__ __forceinline__ void tile_coords(int t, int ntm, int ntn, int& bm, int& bn) {

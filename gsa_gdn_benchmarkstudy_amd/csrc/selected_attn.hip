@@ -18,15 +18,16 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 
 namespace gsa {
 
-// Index lists -> bitmask, tile range and redo mark of each row: one block per row.
+// Index lists -> bitmask, tile range and repeat mark of each row: one block per row.
 struct SelRowsArgs {
   const void* idx; int idx64; int64_t i_sb, i_st; int k_sel;
   const int32_t* count; const uint8_t* mask;
   int T, Tkv, W;
-  uint32_t* bits; int2* range; uint8_t* redo;
+  uint32_t* bits; int2* range; uint8_t* twice;
 };
 
 template <typename IdxT>
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(256) void selected_rows_kernel(SelRowsArgs p) {
   __syncthreads();
   if (tid == 0) {
     p.range[row] = int2{st_lo, st_hi};
-    p.redo[row] = (uint8_t)st_twice;
+    p.twice[row] = (uint8_t)st_twice;
   }
 }
 
@@ -82,38 +83,48 @@ namespace {
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 size_t bits_bytes(int B, int T, int Tkv) { return align256((size_t)B * T * ((Tkv + 63) / 64) * 8); }
 
+// Bitmask, tile ranges, repeat marks, redo marks, then the bf16 kernel's own.
+size_t workspace(int B, int T, int Tkv, int H, int dtype) {
+  return bits_bytes(B, T, Tkv) + align256((size_t)B * T * 8) + align256((size_t)B * T) + align256((size_t)B * T * H) +
+         (dtype == GSA_DTYPE_BF16 ? dense_selected_bytes(B, T, Tkv, H) : 0);
+}
+
 constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 
 // Whether the matrix-core way is the faster one, from the time each takes (us,
-// measured at 16 heads, bf16).  The gather: 20 + the larger of 0.5 per key of a
+// measured at 16 heads).  The gather, bf16: 20 + the larger of 0.5 per key of a
 // row (its loads are a chain within the row's block) and 0.0009 per row and
 // key (what it reads); T = 512, k = 128 89; T = 8192, k = 2048 13002.  The
 // matrix cores: 30 for the launches and 2.4 for each 64-key tile of a block's
 // 256 rows, one block per CU at a time: T = 512, k = 128 54; T = 8192, k = 2048
-// 502; T = 256, Tkv = 8192, k = 128 340, where the gather takes 89.  (All Tkv
-// tiles are counted; what a causal selection leaves out is known on the device only.)
+// 502; T = 256, Tkv = 8192, k = 128 340, where the gather takes 89.  In
+// fp32 the gather reads twice as much, and a 64-key tile of a 128-row block
+// takes 8: T = 512, k = 128 96 against 103, T = 2048, k = 2048 311 against 2904,
+// T = 4096, k = 128 745 by the gather.  (All Tkv tiles are counted; what a causal
+// selection leaves out is known on the device only.)
 // The masks reach -8e36 times the scale, which has to stay far below every
 // score: a scale outside [1e-10, 1e10] takes the gather.  A row's bits fit the
 // LDS of a block, and the workspace (2 bytes per element of V, 5 bits per row
 // and key) is kept to 4 GiB.
 bool dense_serves(int B, int T, int Tkv, int H, int k_sel, float scale, int dtype) {
-  if (dtype != GSA_DTYPE_BF16) return false;
+  const bool bf16 = dtype == GSA_DTYPE_BF16;
+  if (!bf16 && dtype != GSA_DTYPE_F32) return false;
   if (!(scale >= 1e-10f && scale <= 1e10f)) return false;
   if ((size_t)((Tkv + 63) / 64) * 8 > 65536 - 64) return false;
   const int64_t NT = (Tkv + 63) / 64, groups = ((int64_t)T + 255) / 256 * 8;
-  const double rounds = (double)((B * H * (groups / 8) + 255) / 256);
-  const double gather = 20.0 + std::max(0.5 * k_sel, 0.0009 * B * T * (double)k_sel * H / 16);
-  if (30.0 + 2.4 * NT * rounds > gather) return false;
+  const double gather = 20.0 + std::max(0.5 * k_sel, 0.0009 * B * T * (double)k_sel * H / 16) * (bf16 ? 1 : 2);
+  const double blocks = bf16 ? B * H * (groups / 8) : B * H * ((T + 127) / 128);
+  const double tile = bf16 ? 2.4 : 8.0;
+  if (30.0 + tile * NT * std::ceil(blocks / 256) > gather) return false;
   if (B * groups * NT > 0x3fffffffLL / 32 || (int64_t)B * H * NT > 0x3fffffffLL) return false;
-  return bits_bytes(B, T, Tkv) + align256((size_t)B * T * 9) + dense_selected_bytes(B, T, Tkv, H) <= kMaxWorkspace;
+  return workspace(B, T, Tkv, H, dtype) <= kMaxWorkspace;
 }
 
 }  // namespace
 
 extern "C" size_t gsa_selected_attn_workspace_bytes(int B, int T, int Tkv, int H, int k_sel, float scale, int dtype) {
   if (B < 1 || T < 1 || Tkv < 1 || H < 1 || H > 64 || !dense_serves(B, T, Tkv, H, k_sel, scale, dtype)) return 0;
-  return bits_bytes(B, T, Tkv) + align256((size_t)B * T * 8) + align256((size_t)B * T) +
-         dense_selected_bytes(B, T, Tkv, H);
+  return workspace(B, T, Tkv, H, dtype);
 }
 
 extern "C" int gsa_selected_attn(const void* q, int64_t q_sb, int64_t q_st,
@@ -145,17 +156,86 @@ extern "C" int gsa_selected_attn(const void* q, int64_t q_sb, int64_t q_st,
   base += bits_bytes(B, T, Tkv);
   int2* range = reinterpret_cast<int2*>(base);
   base += align256((size_t)B * T * 8);
-  uint8_t* redo = reinterpret_cast<uint8_t*>(base);
+  uint8_t* twice = reinterpret_cast<uint8_t*>(base);
   base += align256((size_t)B * T);
+  uint8_t* redo = reinterpret_cast<uint8_t*>(base);
+  base += align256((size_t)B * T * H);
   const int W = 2 * ((Tkv + 63) / 64);
-  const gsa::SelRowsArgs r{idx, idx_bytes == 8, i_sb, i_st, k_sel, count, mask, T, Tkv, W, bits, range, redo};
+  const gsa::SelRowsArgs r{idx, idx_bytes == 8, i_sb, i_st, k_sel, count, mask, T, Tkv, W, bits, range, twice};
   if (idx_bytes == 8)
     hipLaunchKernelGGL(gsa::selected_rows_kernel<int64_t>, dim3(B * T), dim3(256), (size_t)W * 4, s, r);
   else
     hipLaunchKernelGGL(gsa::selected_rows_kernel<int32_t>, dim3(B * T), dim3(256), (size_t)W * 4, s, r);
   int st = launch_status();
   if (st) return st;
-  const AttnShape a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, out, out_sb, out_st, B, T, Tkv, H, scale};
-  if ((st = launch_dense_selected(a, gsa::Selection{bits, range, redo}, base, s))) return st;
-  return launch_gather_rows(a, IndexLists{idx, idx_bytes == 8, i_sb, i_st, k_sel, count, mask}, redo, dtype, s);
+  AttnShape a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, out, out_sb, out_st, B, T, Tkv, H, scale};
+  const gsa::Selection sel{bits, range, twice, redo};
+  st = dtype == GSA_DTYPE_BF16 ? launch_dense_selected(a, sel, base, s) : launch_dense_f32(a, sel, s);
+  if (st) return st;
+  return launch_gather_rows(a, IndexLists{idx, idx_bytes == 8, i_sb, i_st, k_sel, count, mask}, sel, dtype, s);
+}
+
+// ---------------------------------------------------------------------------
+// The layer's fp32 attention: the selection is there as a causal bitmask.
+// ---------------------------------------------------------------------------
+
+// Workspace of gsa_masked_attn: the redo marks, then the index lists and counts
+// of marked rows.
+static size_t masked_workspace(int B, int T, int H, int k_sel) {
+  return align256((size_t)B * T * H) + align256((size_t)B * T * k_sel * 4) + align256((size_t)B * T * 4);
+}
+
+// From the time each way takes (us, fp32, 16 heads): the gather as in
+// dense_serves, twice its bf16 cost per key; the matrix cores 20 for the launches
+// and 3.9 per 32-key tile of 128 rows, the longest block's or the mean CU's.
+extern "C" size_t gsa_masked_attn_workspace_bytes(int B, int T, int H, int k_sel, int dtype) {
+  if (B < 1 || T < 1 || H < 1 || H > 64 || k_sel < 1 || k_sel > T || dtype != GSA_DTYPE_F32) return 0;
+  if ((int64_t)B * T > 0x7fffffffLL) return 0;
+  const double k = k_sel, pairs = B * (k * (k + 1) / 2 + (T - k) * k);
+  const double gather = 20.0 + std::max(0.5 * k, 0.0018 * pairs * H / 16);
+  const double longest = (T + 31) / 32, tiles = longest * ((T + 127) / 128 + 1) / 2 * B * H;
+  if (20.0 + 3.9 * std::max(longest, tiles / 256) > gather) return 0;
+  return masked_workspace(B, T, H, k_sel);
+}
+
+extern "C" int gsa_masked_attn(const void* q, int64_t q_sb, int64_t q_st,
+                               const void* k, int64_t k_sb, int64_t k_st,
+                               const void* v, int64_t v_sb, int64_t v_st,
+                               const uint32_t* bits, int k_sel,
+                               const void* og, int64_t o_sb, int64_t o_st,
+                               const void* cos, const void* sin, int64_t cs_st,
+                               void* out, int64_t out_sb, int64_t out_st,
+                               int B, int T, int H, int d, float scale, int dtype, int flags,
+                               void* ws, size_t ws_bytes, void* stream) {
+  if (!q || !k || !v || !bits || !out || !ws) return GSA_ERR_NULL;
+  if (flags & ~(GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE)) return GSA_ERR_FLAGS;
+  if ((flags & GSA_ATTN_ROPE_Q) && (!cos || !sin)) return GSA_ERR_NULL;
+  if ((flags & GSA_ATTN_OUT_GATE) && !og) return GSA_ERR_NULL;
+  if (dtype != GSA_DTYPE_F32) return GSA_ERR_DTYPE;
+  if (B < 1 || T < 1 || d != 128 || H < 1 || H > 64) return GSA_ERR_SHAPE;
+  if ((int64_t)B * T > 0x7fffffffLL || (int64_t)B * H * ((T + 127) / 128) > 0x7fffffffLL) return GSA_ERR_SHAPE;
+  if (k_sel < 1 || k_sel > T) return GSA_ERR_K;
+  if (!(scale > 0.f)) return GSA_ERR_SHAPE;             // a row's largest score is found before the scale
+  if (ws_bytes < masked_workspace(B, T, H, k_sel)) return GSA_ERR_SHAPE;
+  for (const int64_t st : {k_st, v_st})                 // 32-bit byte offsets within a tile
+    if (st < 0 || st > (1 << 24)) return GSA_ERR_SHAPE;
+  if (!vec_ok(q, q_sb, q_st, dtype) || !vec_ok(k, k_sb, k_st, dtype) || !vec_ok(v, v_sb, v_st, dtype) ||
+      !vec_ok(out, out_sb, out_st, dtype) || !aligned(bits, 8) || !aligned(ws, 256))
+    return GSA_ERR_ALIGN;
+  if ((flags & GSA_ATTN_OUT_GATE) && !vec_ok(og, o_sb, o_st, dtype)) return GSA_ERR_ALIGN;
+  if ((flags & GSA_ATTN_ROPE_Q) && (!vec_ok(cos, 0, cs_st, dtype) || !vec_ok(sin, 0, cs_st, dtype)))
+    return GSA_ERR_ALIGN;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  char* base = static_cast<char*>(ws);
+  uint8_t* redo = reinterpret_cast<uint8_t*>(base);
+  base += align256((size_t)B * T * H);
+  int32_t* idx = reinterpret_cast<int32_t*>(base);
+  int32_t* count = reinterpret_cast<int32_t*>(base + align256((size_t)B * T * k_sel * 4));
+  const AttnShape a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, out, out_sb, out_st, B, T, T, H, scale,
+                    og, o_sb, o_st, cos, sin, cs_st, flags};
+  const gsa::Selection sel{bits, nullptr, nullptr, redo};
+  int st = launch_dense_f32(a, sel, s);
+  if (st) return st;
+  if ((st = launch_marked_indices(bits, B, T, k_sel, redo, H, idx, count, s))) return st;
+  return launch_gather_rows(a, IndexLists{idx, 0, (int64_t)T * k_sel, k_sel, k_sel, count, nullptr}, sel, dtype, s);
 }

@@ -69,8 +69,10 @@ struct AttnArgs {
   int T, Tkv;
   float scale_l2;   // scale * log2(e): scores live in the log2 domain
   int flags;
-  const uint8_t* redo;   // kRows: the rows to compute ([B*T], nonzero)
-  int idx64;             // kRows: idx holds 64-bit indices
+  // kRows: compute rows marked in twice ([B*T], nullable) and heads of rows
+  // marked in redo ([B*T*H]); idx64: idx holds 64-bit indices
+  const uint8_t* twice; const uint8_t* redo;
+  int H, idx64;
 };
 
 // One key row slice for this lane: 8 elements as raw storage.
@@ -130,15 +132,15 @@ struct QReg {
 template <typename T> struct Chunk { static constexpr int kKeys = 8; };
 template <> struct Chunk<float> { static constexpr int kKeys = 4; };
 
-// kRows: only the rows marked in `redo` (the others' blocks end at once), with
-// 32- or 64-bit indices (a 64-bit index counts by its low 32 bits).
+// kRows: only what twice and redo mark (the other rows' blocks end at once),
+// with 32- or 64-bit indices (a 64-bit index counts by its low 32 bits).
 template <typename T, int kThreads, bool kRows>
 __global__ __launch_bounds__(kThreads) void sparse_attn_kernel(AttnArgs p) {
   // keys in flight per buffer; halved for 1024-thread blocks (128-VGPR budget)
   constexpr int C = kThreads > 256 ? Chunk<T>::kKeys / 2 : Chunk<T>::kKeys;
   const int row = blockIdx.x;
   if constexpr (kRows)
-    if (!p.redo[row]) return;
+    if (!(p.twice && p.twice[row]) && !p.redo[(int64_t)row * p.H + (threadIdx.x >> 4)]) return;   // by whole 16-lane rows
   const int b = row / p.T, t = row % p.T;
   const int li = threadIdx.x & 15;
   const int e0 = threadIdx.x * 8;   // head*128 + li*8
@@ -312,15 +314,15 @@ extern "C" int gsa_sparse_attn(const void* q, int64_t q_sb, int64_t q_st,
     return GSA_ERR_ALIGN;
   gsa::AttnArgs a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, idx, i_sb, i_st, k_sel, count, mask,
                   og, o_sb, o_st, cos, sin, cs_st, out, out_sb, out_st, T, Tkv,
-                  scale * gsa::kLog2e, flags, nullptr, 0};
+                  scale * gsa::kLog2e, flags, nullptr, nullptr, H, 0};
   return launch_gather<false>(a, B, H, dtype, static_cast<hipStream_t>(stream));
 }
 
-int gsa_host::launch_gather_rows(const AttnShape& s, const IndexLists& l, const uint8_t* redo, int dtype,
+int gsa_host::launch_gather_rows(const AttnShape& s, const IndexLists& l, const gsa::Selection& sel, int dtype,
                                  hipStream_t stream) {
   gsa::AttnArgs a{s.q, s.q_sb, s.q_st, s.k, s.k_sb, s.k_st, s.v, s.v_sb, s.v_st,
                   static_cast<const int32_t*>(l.idx), l.i_sb, l.i_st, l.k_sel, l.count, l.mask,
-                  nullptr, 0, 0, nullptr, nullptr, 0, s.out, s.out_sb, s.out_st, s.T, s.Tkv,
-                  s.scale * gsa::kLog2e, 0, redo, l.idx64};
+                  s.og, s.o_sb, s.o_st, s.cos, s.sin, s.cs_st, s.out, s.out_sb, s.out_st, s.T, s.Tkv,
+                  s.scale * gsa::kLog2e, s.flags, sel.twice, sel.redo, s.H, l.idx64};
   return launch_gather<true>(a, s.B, s.H, dtype, stream);
 }

@@ -326,8 +326,8 @@ class GatedSparseAttention(nn.Module):
          transposed, or gsa_prologue);
       4. join, then the attention with RoPE(q) and the output gate fused --
          gsa_dense_attn (bf16: MFMA over every causal key tile, masked to the
-         selection) or gsa_sparse_attn (per-row gather of the selected keys)
-         -- and the o_proj GEMM.
+         selection), gsa_masked_attn (its fp32 form) or gsa_sparse_attn
+         (per-row gather of the selected keys) -- and the o_proj GEMM.
     """
 
     def __init__(self, hidden_size: int, num_heads: int, k_max: int = 4096, d_indexer: int = 64,
@@ -362,7 +362,9 @@ class GatedSparseAttention(nn.Module):
         self._indexer_stream: Optional[torch.cuda.Stream] = None
         # Attention kernel: "dense" (block-dense MFMA over the causal key tiles
         # with the selection as a bitmask, bf16), "gather" (per-row gather of
-        # the selected keys, bf16 and fp32), or "auto" (dense for bf16).
+        # the selected keys, bf16 and fp32), or "auto" (dense for bf16; for fp32
+        # its fp32 form over the same bitmask, gsa_masked_attn, or the gather,
+        # whichever is faster at the sizes).
         self.attn_impl = "auto"
         # Where the fused indexer + top-k runs relative to the main projection
         # GEMM: "gemm" (on a side stream beside the GEMM), "producer" (after
@@ -543,6 +545,8 @@ class GatedSparseAttention(nn.Module):
         cur = torch.cuda.current_stream(dev)
 
         dense = self.uses_dense(x.dtype)
+        k_sel = self.topk_selector.k_effective(T)
+        masked = self.attn_impl == "auto" and not dense and _abi.masked_attn_serves(B, T, self.num_heads, k_sel, x.dtype)
         fused_proj = self.uses_fused_projection(x)
         cos, sin = self.rotary_emb(T, dev, x.dtype)
         cos, sin = cos.contiguous(), sin.contiguous()
@@ -583,7 +587,7 @@ class GatedSparseAttention(nn.Module):
             side.wait_stream(cur)
         with torch.cuda.stream(side):
             _range_push("gsa_hip/indexer_select")
-            bits, idx, cnt = self.select(views, T, indices=not dense)
+            bits, idx, cnt = self.select(views, T, indices=not dense and not masked)
             _range_pop()
         # The dense attention's lane masks, built from the bitmask off the
         # current stream (beside the projection GEMM / producer) on the
@@ -645,6 +649,9 @@ class GatedSparseAttention(nn.Module):
             else:
                 attn = _abi.dense_attn(views["q"], k_rope, v_gated, bits, self.scale, og=views["og"],
                                        cos=cos, sin=sin, flags=flags, causal=True, ws=lm_ws, masks_ready=True)
+        elif masked:
+            attn = _abi.masked_attn(views["q"], k_rope, v_gated, bits, k_sel, self.scale, og=views["og"], cos=cos,
+                                    sin=sin, flags=flags)
         else:
             attn = _abi.sparse_attn(views["q"], k_rope, v_gated, idx, self.scale, count=cnt,
                                     og=views["og"], cos=cos, sin=sin, flags=flags)

@@ -312,6 +312,28 @@ int gsa_selected_attn(const void* q, int64_t q_sb, int64_t q_st,
                       void* ws, size_t ws_bytes, void* stream);
 
 /*
+ * gsa_sparse_attn in fp32 for a causal selection given as a bitmask (bits
+ * [B,T,W] contiguous, as gsa_indexer_select writes it, at most k_sel keys per
+ * row): the layer's attention (gsa_triton/gsa_opt.py:692-721) on the fp32 matrix
+ * instruction, RoPE(q) and the output gate by `flags` as in gsa_sparse_attn.
+ * Rows whose sums are not finite are computed by gsa_sparse_attn's kernel.
+ * gsa_masked_attn_workspace_bytes is 0 where gsa_sparse_attn is the faster one
+ * (selected_attn.hip has the rule).  fp32 only, scale > 0, k and v row strides
+ * at most 2^24 elements; ws 256-byte aligned, overwritten.
+ */
+size_t gsa_masked_attn_workspace_bytes(int B, int T, int H, int k_sel, int dtype);
+
+int gsa_masked_attn(const void* q, int64_t q_sb, int64_t q_st,
+                    const void* k, int64_t k_sb, int64_t k_st,
+                    const void* v, int64_t v_sb, int64_t v_st,
+                    const uint32_t* bits, int k_sel,
+                    const void* og, int64_t o_sb, int64_t o_st,
+                    const void* cos, const void* sin, int64_t cs_st,
+                    void* out, int64_t out_sb, int64_t out_st,
+                    int B, int T, int H, int d, float scale, int dtype, int flags,
+                    void* ws, size_t ws_bytes, void* stream);
+
+/*
  * Producer for the block-dense attention: RoPE on k (k == NULL skips it) and
  * the G2 gate with V written transposed.  Replaces gsa_triton/gsa_opt.py:
  * 685-697 like gsa_prologue, with the value output laid out for
