@@ -29,6 +29,8 @@
 // where the gather of k = 2048 keys took 25.8 ms.
 #include "gsa_common.h"
 
+#include <cmath>
+
 namespace gsa {
 
 constexpr int kFRows = 128;               // query rows per block
@@ -51,19 +53,28 @@ struct DenseF32Args {
   int B, T, Tkv, H, nqb;
   float scale_l2;
   int flags;
+  float* parts; uint32_t* counters;       // plan.n > 0: slots [B*H][plan.slots], arrivals [B*H][nqb]
 };
 
-__global__ __launch_bounds__(256, 2) void dense_attn_f32_kernel(DenseF32Args p) {
+__global__ __launch_bounds__(256, 2) void dense_attn_f32_kernel(DenseF32Args p, UnitPlan plan) {
   extern __shared__ __align__(16) u32x4 dsm[];       // slot s: K units, then V units
   const int tid = threadIdx.x, lane = tid & 63;
   const int wu = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int i32 = lane & 31, h = lane >> 5;
-  // heaviest query blocks first, heads fastest (a head's blocks share an XCD's L2)
-  const int per_b = p.nqb * p.H;
-  const int b = (int)(blockIdx.x / per_b);
-  const int r2 = (int)(blockIdx.x % per_b);
-  const int qb = p.nqb - 1 - r2 / p.H;
-  const int hd = r2 % p.H;
+  // heads fastest (a head's blocks share an XCD's L2), heaviest query blocks first
+  int b, qb, hd;
+  Unit unit{0, 0, 1, 0};
+  if (plan.n) {
+    hd = blockIdx.x % p.H;
+    b = blockIdx.x / p.H % p.B;
+    unit = plan_unit(plan, blockIdx.x / (p.H * p.B));
+    qb = unit.qb;
+  } else {
+    const int per_b = p.nqb * p.H, r2 = blockIdx.x % per_b;
+    b = blockIdx.x / per_b;
+    qb = p.nqb - 1 - r2 / p.H;
+    hd = r2 % p.H;
+  }
   const int q0 = qb * kFRows;
   const int row = q0 + 32 * wu + i32, rowc = min(row, p.T - 1);
 
@@ -73,6 +84,15 @@ __global__ __launch_bounds__(256, 2) void dense_attn_f32_kernel(DenseF32Args p) 
     const int2 tr = tile_range<64>(p.range, (int64_t)b * p.T, q0, min(q0 + kFRows, p.T));
     kt0 = 2 * __builtin_amdgcn_readfirstlane(tr.x);
     nkt = min(2 * __builtin_amdgcn_readfirstlane(tr.y), (p.Tkv + kFKeys - 1) / kFKeys) - kt0;
+  }
+  const int parts = min(unit.parts, nkt);
+  if (parts > 1) {                         // this unit's share of them (a part past the tiles has none)
+    if (unit.part >= parts) return;
+    const int t0 = nkt * unit.part / parts, t1 = nkt * (unit.part + 1) / parts;
+    kt0 += t0;
+    nkt = t1 - t0;
+  } else if (unit.part) {
+    return;
   }
 
   // ---- tile loads: wave w issues instructions w, w + 4, ... of a tile's 17 (K)
@@ -209,6 +229,13 @@ __global__ __launch_bounds__(256, 2) void dense_attn_f32_kernel(DenseF32Args p) 
 
   // ---- epilogue: normalise, optional output gate; dims 4(8(r/4) + 4h + r%4) + dt ----
   l = sum_halves(l);
+  if (parts > 1) {
+    const int64_t bh = (int64_t)b * p.H + hd;
+    __syncthreads();                       // the tile slots are free: dsm[0] carries the arrival count
+    if (!merge_parts(o, m, l, p.parts + (bh * plan.slots + unit.slot) * (4 * kPartWave), unit.part, parts, 4, wu, lane,
+                     p.counters + bh * p.nqb + qb, reinterpret_cast<uint32_t*>(dsm)))
+      return;
+  }
   float z = 0.f;
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
@@ -239,7 +266,46 @@ __global__ __launch_bounds__(256, 2) void dense_attn_f32_kernel(DenseF32Args p) 
 
 using namespace gsa_host;
 
-int gsa_host::launch_dense_f32(const AttnShape& s, const gsa::Selection& sel, hipStream_t stream) {
+namespace {
+
+__global__ __launch_bounds__(256) void clear_kernel(uint32_t* p, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
+
+// How the query blocks are split, by sizes alone (query and key length alike are
+// taken for causal): into parts of 0.6 of a CU's mean share of the tiles while
+// that is small (fewer parts, less to add up), 0.33 beyond (finer parts, a shorter
+// tail), 4 tiles at least.  16 heads, causal, us without / with (parts of 0.33
+// and 0.6 of the share): T = 512 96 / 60 60, T = 1537 230 / 166 147, T = 2048
+// 298 / 226 191, B = 2 T = 1537 382 / 250 275, T = 3000 537 / 378 426, T = 4096
+// 815 / 611 725, B = 2 T = 4096 1225 / 1160 1224.
+gsa::UnitPlan f32_plan(int B, int T, int Tkv, int H) {
+  const int nqb = (T + gsa::kFRows - 1) / gsa::kFRows, nt = (Tkv + gsa::kFKeys - 1) / gsa::kFKeys;
+  std::vector<int> tiles(nqb, nt);
+  int64_t total = 0;
+  for (int i = 0; i < nqb; ++i) {
+    if (T == Tkv) tiles[i] = std::min(nt, 4 * (i + 1));
+    total += tiles[i];
+  }
+  const double share = (double)total * B * H / 256;
+  return split_plan(tiles, std::max(4, (int)std::ceil(share * (share < 40 ? 0.6 : 0.33))));
+}
+
+size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+size_t counter_bytes(int B, int T, int H) {
+  return align256((size_t)B * H * ((T + gsa::kFRows - 1) / gsa::kFRows) * sizeof(uint32_t));
+}
+
+}  // namespace
+
+size_t gsa_host::dense_f32_bytes(int B, int T, int Tkv, int H) {
+  const gsa::UnitPlan plan = f32_plan(B, T, Tkv, H);
+  if (!plan.n) return 0;
+  return counter_bytes(B, T, H) + (size_t)B * H * plan.slots * 4 * gsa::kPartWave * sizeof(float);
+}
+
+int gsa_host::launch_dense_f32(const AttnShape& s, const gsa::Selection& sel, void* ws, hipStream_t stream) {
   constexpr int kMaxDevices = 64;
   constexpr size_t kLds = (size_t)2 * gsa::kFSlot * 16;
   static bool done[kMaxDevices] = {};        // (a benign race: concurrent first calls set the same attribute)
@@ -252,12 +318,22 @@ int gsa_host::launch_dense_f32(const AttnShape& s, const gsa::Selection& sel, hi
     done[dev] = true;
   }
   const int nqb = (s.T + gsa::kFRows - 1) / gsa::kFRows;
+  const gsa::UnitPlan plan = f32_plan(s.B, s.T, s.Tkv, s.H);
+  uint32_t* counters = static_cast<uint32_t*>(ws);
+  float* parts = reinterpret_cast<float*>(static_cast<char*>(ws) + counter_bytes(s.B, s.T, s.H));
+  if (plan.n) {
+    const int n = s.B * s.H * nqb;
+    hipLaunchKernelGGL(clear_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, counters, n);
+    const int st = launch_status();
+    if (st) return st;
+  }
   const gsa::DenseF32Args a{
       static_cast<const float*>(s.q), s.q_sb, s.q_st, static_cast<const float*>(s.k), s.k_sb, s.k_st,
       static_cast<const float*>(s.v), s.v_sb, s.v_st, sel.bits, 2 * ((s.Tkv + 63) / 64), sel.range, sel.redo,
       static_cast<const float*>(s.og), s.o_sb, s.o_st, static_cast<const float*>(s.cos),
       static_cast<const float*>(s.sin), s.cs_st, static_cast<float*>(s.out), s.out_sb, s.out_st,
-      s.B, s.T, s.Tkv, s.H, nqb, s.scale * gsa::kLog2e, s.flags};
-  hipLaunchKernelGGL(gsa::dense_attn_f32_kernel, dim3(s.B * s.H * nqb), dim3(256), kLds, stream, a);
+      s.B, s.T, s.Tkv, s.H, nqb, s.scale * gsa::kLog2e, s.flags, parts, counters};
+  hipLaunchKernelGGL(gsa::dense_attn_f32_kernel, dim3(s.B * s.H * (plan.n ? plan.n : nqb)), dim3(256), kLds, stream, a,
+                     plan);
   return launch_status();
 }

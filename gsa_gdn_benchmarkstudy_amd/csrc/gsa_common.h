@@ -5,6 +5,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <vector>
+
 #include "../../include/gsa_hip.h"
 
 // Every product and sum rounds on its own (torch's rounding points); fused
@@ -142,6 +145,73 @@ __device__ __forceinline__ void rope8(float (&x)[8], const float (&c)[8], const 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Query blocks split along their keys (the block-dense attention kernels).
+// With few query blocks, or causal ones of very different length, one block
+// per CU leaves most of the chip idle while the longest runs; a unit is then one
+// of `parts` equal pieces of a query block's key tiles.  Each unit writes its
+// sums and softmax state to its slot and counts itself; the last one to arrive
+// adds all parts in their order (so the result does not depend on which was
+// last) and goes on to the epilogue.  No unit waits for another.
+// ---------------------------------------------------------------------------
+constexpr int kMaxUnits = 512;            // 2 KiB of kernel arguments
+struct UnitPlan {
+  int n;                                  // units per (batch, head), longest first; 0: one unit per query block, in the kernel's own order
+  int slots;                              // partial slots per (batch, head)
+  uint32_t unit[kMaxUnits];               // query block | part << 10 | parts << 15 | first slot << 20
+};
+struct Unit { int qb, part, parts, slot; };
+__device__ __forceinline__ Unit plan_unit(const UnitPlan& plan, int u) {
+  const uint32_t w = plan.unit[u];
+  return Unit{(int)(w & 1023u), (int)((w >> 10) & 31u), (int)((w >> 15) & 31u), (int)(w >> 20)};
+}
+// Floats of one slot: per wave 64 accumulator registers, m and l of 64 lanes.
+constexpr int kPartWave = 66 * 64;
+
+// Publishes this unit's O^T accumulators, reference m and sum l (whole row, in
+// both lanes) and, in the last unit to arrive, replaces them by the sums over
+// all parts; false in the other units, which have nothing left to do.
+// slots: the query block's first slot; `flag`: one word of LDS that no wave
+// uses any more.  Plain stores and loads with an agent-scope release by the
+// counting thread and an acquire after it: units run on different XCDs.
+__device__ __forceinline__ bool merge_parts(floatx16 (&o)[4], float& m, float& l, float* slots, int part, int parts,
+                                            int waves, int wave, int lane, uint32_t* counter, uint32_t* flag) {
+  float* const mine = slots + ((int64_t)part * waves + wave) * kPartWave + lane;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mine[(16 * dt + r) * 64] = o[dt][r];
+  mine[64 * 64] = m;
+  mine[65 * 64] = l;
+  __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xf << 8));     // vmcnt(0): this wave's stores are in L2
+  __syncthreads();
+  if (threadIdx.x == 0)
+    *flag = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (*flag != (uint32_t)(parts - 1)) return false;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  const float* const all = slots + (int64_t)wave * kPartWave + lane;
+  float top = -__builtin_inff();
+  for (int s = 0; s < parts; ++s) top = fmaxf(top, all[(int64_t)s * waves * kPartWave + 64 * 64]);
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[dt][r] = 0.f;
+  l = 0.f;
+  for (int s = 0; s < parts; ++s) {
+    const float* const at = all + (int64_t)s * waves * kPartWave;
+    const float ms = at[64 * 64];
+    const float w = ms == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ms - top);
+    l = __builtin_fmaf(at[65 * 64], w, l);
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = __builtin_fmaf(at[(16 * dt + r) * 64], w, o[dt][r]);
+  }
+  m = top;
+  return true;
+}
+
 // Monotone map of an fp32 score to uint32: a > b  <=>  key(a) > key(b).
 // -inf is first replaced by -1e9 (the selector's fill value) and every NaN
 // ranks above +inf, as torch.topk orders them.
@@ -236,6 +306,31 @@ __device__ __forceinline__ int2 tile_range(const int2* range, int64_t row_base, 
 // ---------------------------------------------------------------------------
 namespace gsa_host {
 
+// Query blocks of `tiles` key tiles each, split into parts of at most `chunk`
+// tiles, longest parts first.  n = 0 (no plan) where nothing is split or the
+// units do not fit.
+inline gsa::UnitPlan split_plan(const std::vector<int>& tiles, int chunk) {
+  gsa::UnitPlan p;
+  p.n = p.slots = 0;
+  struct U { int size; uint32_t w; };
+  std::vector<U> units;
+  if (tiles.size() > 1024 || *std::max_element(tiles.begin(), tiles.end()) <= chunk) return p;
+  for (int qb = (int)tiles.size() - 1; qb >= 0; --qb) {
+    const int parts = std::min(31, std::max(1, (tiles[qb] + chunk - 1) / chunk));
+    for (int i = 0; i < parts; ++i)
+      units.push_back({tiles[qb] * (i + 1) / parts - tiles[qb] * i / parts,
+                       (uint32_t)qb | (uint32_t)i << 10 | (uint32_t)parts << 15 | (uint32_t)p.slots << 20});
+    if (parts > 1) p.slots += parts;
+  }
+  if (p.slots == 0 || (int)units.size() > gsa::kMaxUnits) {
+    p.slots = 0;
+    return p;
+  }
+  std::stable_sort(units.begin(), units.end(), [](const U& a, const U& b) { return a.size > b.size; });
+  for (const U& u : units) p.unit[p.n++] = u.w;
+  return p;
+}
+
 inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
 inline int dtype_size(int dtype) {
   return dtype == GSA_DTYPE_BF16 ? 2 : (dtype == GSA_DTYPE_F32 ? 4 : 0);
@@ -281,7 +376,9 @@ struct IndexLists {
 size_t dense_selected_bytes(int B, int T, int Tkv, int H);
 int launch_dense_selected(const AttnShape& a, const gsa::Selection& sel, void* ws, hipStream_t stream);
 // fp32 on MFMA (dense_attn_f32.hip); sel.range null: a causal selection.
-int launch_dense_f32(const AttnShape& a, const gsa::Selection& sel, hipStream_t stream);
+// ws: dense_f32_bytes bytes, 256-byte aligned.
+size_t dense_f32_bytes(int B, int T, int Tkv, int H);
+int launch_dense_f32(const AttnShape& a, const gsa::Selection& sel, void* ws, hipStream_t stream);
 // The gather kernel on what sel.twice and sel.redo mark (sparse_attn.hip).
 int launch_gather_rows(const AttnShape& a, const IndexLists& l, const gsa::Selection& sel, int dtype,
                        hipStream_t stream);

@@ -83,10 +83,10 @@ namespace {
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 size_t bits_bytes(int B, int T, int Tkv) { return align256((size_t)B * T * ((Tkv + 63) / 64) * 8); }
 
-// Bitmask, tile ranges, repeat marks, redo marks, then the bf16 kernel's own.
+// Bitmask, tile ranges, repeat marks, redo marks, then the attention kernel's own.
 size_t workspace(int B, int T, int Tkv, int H, int dtype) {
   return bits_bytes(B, T, Tkv) + align256((size_t)B * T * 8) + align256((size_t)B * T) + align256((size_t)B * T * H) +
-         (dtype == GSA_DTYPE_BF16 ? dense_selected_bytes(B, T, Tkv, H) : 0);
+         (dtype == GSA_DTYPE_BF16 ? dense_selected_bytes(B, T, Tkv, H) : dense_f32_bytes(B, T, Tkv, H));
 }
 
 constexpr size_t kMaxWorkspace = (size_t)4 << 30;
@@ -98,10 +98,11 @@ constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 // matrix cores: 30 for the launches and 2.4 for each 64-key tile of a block's
 // 256 rows, one block per CU at a time: T = 512, k = 128 54; T = 8192, k = 2048
 // 502; T = 256, Tkv = 8192, k = 128 340, where the gather takes 89.  In
-// fp32 the gather reads twice as much, and a 64-key tile of a 128-row block
-// takes 8: T = 512, k = 128 96 against 103, T = 2048, k = 2048 311 against 2904,
-// T = 4096, k = 128 745 by the gather.  (All Tkv tiles are counted; what a causal
-// selection leaves out is known on the device only.)
+// fp32 the gather reads twice as much; the matrix cores, whose blocks are split
+// evenly over the chip there, take 40 and 9.6 for each 64-key tile of a 128-row
+// block per CU: T = 512, k = 128 62 against 98, T = 2048, k = 2048 212 against
+// 2792, T = 4096, k = 128 765 by the gather.  (All Tkv tiles are counted; what a
+// causal selection leaves out is known on the device only.)
 // The masks reach -8e36 times the scale, which has to stay far below every
 // score: a scale outside [1e-10, 1e10] takes the gather.  A row's bits fit the
 // LDS of a block, and the workspace (2 bytes per element of V, 5 bits per row
@@ -113,9 +114,9 @@ bool dense_serves(int B, int T, int Tkv, int H, int k_sel, float scale, int dtyp
   if ((size_t)((Tkv + 63) / 64) * 8 > 65536 - 64) return false;
   const int64_t NT = (Tkv + 63) / 64, groups = ((int64_t)T + 255) / 256 * 8;
   const double gather = 20.0 + std::max(0.5 * k_sel, 0.0009 * B * T * (double)k_sel * H / 16) * (bf16 ? 1 : 2);
-  const double blocks = bf16 ? B * H * (groups / 8) : B * H * ((T + 127) / 128);
-  const double tile = bf16 ? 2.4 : 8.0;
-  if (30.0 + tile * NT * std::ceil(blocks / 256) > gather) return false;
+  const double dense = bf16 ? 30.0 + 2.4 * NT * std::ceil(B * H * (groups / 8) / 256.0)
+                            : 40.0 + 9.6 * NT * (B * (double)H * ((T + 127) / 128) / 256.0);
+  if (dense > gather) return false;
   if (B * groups * NT > 0x3fffffffLL / 32 || (int64_t)B * H * NT > 0x3fffffffLL) return false;
   return workspace(B, T, Tkv, H, dtype) <= kMaxWorkspace;
 }
@@ -170,7 +171,7 @@ extern "C" int gsa_selected_attn(const void* q, int64_t q_sb, int64_t q_st,
   if (st) return st;
   AttnShape a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, out, out_sb, out_st, B, T, Tkv, H, scale};
   const gsa::Selection sel{bits, range, twice, redo};
-  st = dtype == GSA_DTYPE_BF16 ? launch_dense_selected(a, sel, base, s) : launch_dense_f32(a, sel, s);
+  st = dtype == GSA_DTYPE_BF16 ? launch_dense_selected(a, sel, base, s) : launch_dense_f32(a, sel, base, s);
   if (st) return st;
   return launch_gather_rows(a, IndexLists{idx, idx_bytes == 8, i_sb, i_st, k_sel, count, mask}, sel, dtype, s);
 }
@@ -179,22 +180,23 @@ extern "C" int gsa_selected_attn(const void* q, int64_t q_sb, int64_t q_st,
 // The layer's fp32 attention: the selection is there as a causal bitmask.
 // ---------------------------------------------------------------------------
 
-// Workspace of gsa_masked_attn: the redo marks, then the index lists and counts
-// of marked rows.
+// Workspace of gsa_masked_attn: the redo marks, the index lists and counts of
+// marked rows, then the attention kernel's own.
 static size_t masked_workspace(int B, int T, int H, int k_sel) {
-  return align256((size_t)B * T * H) + align256((size_t)B * T * k_sel * 4) + align256((size_t)B * T * 4);
+  return align256((size_t)B * T * H) + align256((size_t)B * T * k_sel * 4) + align256((size_t)B * T * 4) +
+         dense_f32_bytes(B, T, T, H);
 }
 
-// From the time each way takes (us, fp32, 16 heads): the gather as in
-// dense_serves, twice its bf16 cost per key; the matrix cores 20 for the launches
-// and 3.9 per 32-key tile of 128 rows, the longest block's or the mean CU's.
+// From the time each way takes (us, 16 heads): the gather as in dense_serves, the
+// matrix cores 30 for the launches and 4.9 for each 32-key tile of a 128-row
+// block per CU (T = 2048, k = 256: 191 against 485 and 52 for the index lists).
 extern "C" size_t gsa_masked_attn_workspace_bytes(int B, int T, int H, int k_sel, int dtype) {
   if (B < 1 || T < 1 || H < 1 || H > 64 || k_sel < 1 || k_sel > T || dtype != GSA_DTYPE_F32) return 0;
   if ((int64_t)B * T > 0x7fffffffLL) return 0;
   const double k = k_sel, pairs = B * (k * (k + 1) / 2 + (T - k) * k);
   const double gather = 20.0 + std::max(0.5 * k, 0.0018 * pairs * H / 16);
-  const double longest = (T + 31) / 32, tiles = longest * ((T + 127) / 128 + 1) / 2 * B * H;
-  if (20.0 + 3.9 * std::max(longest, tiles / 256) > gather) return 0;
+  const double tiles = (T + 31) / 32 * (((T + 127) / 128 + 1) / 2.0) * B * H;
+  if (30.0 + 4.9 * tiles / 256 > gather) return 0;
   return masked_workspace(B, T, H, k_sel);
 }
 
@@ -230,11 +232,13 @@ extern "C" int gsa_masked_attn(const void* q, int64_t q_sb, int64_t q_st,
   uint8_t* redo = reinterpret_cast<uint8_t*>(base);
   base += align256((size_t)B * T * H);
   int32_t* idx = reinterpret_cast<int32_t*>(base);
-  int32_t* count = reinterpret_cast<int32_t*>(base + align256((size_t)B * T * k_sel * 4));
+  base += align256((size_t)B * T * k_sel * 4);
+  int32_t* count = reinterpret_cast<int32_t*>(base);
+  base += align256((size_t)B * T * 4);
   const AttnShape a{q, q_sb, q_st, k, k_sb, k_st, v, v_sb, v_st, out, out_sb, out_st, B, T, T, H, scale,
                     og, o_sb, o_st, cos, sin, cs_st, flags};
   const gsa::Selection sel{bits, nullptr, nullptr, redo};
-  int st = launch_dense_f32(a, sel, s);
+  int st = launch_dense_f32(a, sel, base, s);
   if (st) return st;
   if ((st = launch_marked_indices(bits, B, T, k_sel, redo, H, idx, count, s))) return st;
   return launch_gather_rows(a, IndexLists{idx, 0, (int64_t)T * k_sel, k_sel, k_sel, count, nullptr}, sel, dtype, s);
