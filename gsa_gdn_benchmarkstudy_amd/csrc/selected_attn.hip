@@ -98,10 +98,11 @@ constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 // matrix cores: 30 for the launches and 2.4 for each 64-key tile of a block's
 // 256 rows, one block per CU at a time: T = 512, k = 128 54; T = 8192, k = 2048
 // 502; T = 256, Tkv = 8192, k = 128 340, where the gather takes 89.  In
-// fp32 the gather reads twice as much; the matrix cores, whose blocks are split
-// evenly over the chip there, take 40 and 9.6 for each 64-key tile of a 128-row
-// block per CU: T = 512, k = 128 62 against 98, T = 2048, k = 2048 212 against
-// 2792, T = 4096, k = 128 765 by the gather.  (All Tkv tiles are counted; what a
+// fp32 the gather reads twice as much and takes 0.6 per key of a row; the matrix
+// cores, whose blocks are split evenly over the chip there, take 40, 9.6 for each
+// 64-key tile of a 128-row block per CU, and up to 30 to add the parts: T = 512,
+// k = 128 62 against 98, T = 2048, k = 2048 212 against 2792, T = 64, Tkv = 4096,
+// k = 64 109 against 59, k = 256 109 against 172.  (All Tkv tiles are counted; what a
 // causal selection leaves out is known on the device only.)
 // The masks reach -8e36 times the scale, which has to stay far below every
 // score: a scale outside [1e-10, 1e10] takes the gather.  A row's bits fit the
@@ -113,9 +114,10 @@ bool dense_serves(int B, int T, int Tkv, int H, int k_sel, float scale, int dtyp
   if (!(scale >= 1e-10f && scale <= 1e10f)) return false;
   if ((size_t)((Tkv + 63) / 64) * 8 > 65536 - 64) return false;
   const int64_t NT = (Tkv + 63) / 64, groups = ((int64_t)T + 255) / 256 * 8;
-  const double gather = 20.0 + std::max(0.5 * k_sel, 0.0009 * B * T * (double)k_sel * H / 16) * (bf16 ? 1 : 2);
+  const double reads = 0.0009 * B * T * (double)k_sel * H / 16;
+  const double gather = 20.0 + (bf16 ? std::max(0.5 * k_sel, reads) : std::max(0.6 * k_sel, 2 * reads));
   const double dense = bf16 ? 30.0 + 2.4 * NT * std::ceil(B * H * (groups / 8) / 256.0)
-                            : 40.0 + 9.6 * NT * (B * (double)H * ((T + 127) / 128) / 256.0);
+                            : 40.0 + 9.6 * NT * (B * (double)H * ((T + 127) / 128) / 256.0) + std::min(30.0, 3.0 * NT);
   if (dense > gather) return false;
   if (B * groups * NT > 0x3fffffffLL / 32 || (int64_t)B * H * NT > 0x3fffffffLL) return false;
   return workspace(B, T, Tkv, H, dtype) <= kMaxWorkspace;
