@@ -42,14 +42,18 @@ template <> struct Mfma<uint16_t> {
   }
 };
 
+// (Step s contracts dims 16(s/4) + 4g + s%4 of the lane groups g = 0..3: a lane's
+// four steps are 16 consecutive bytes of its row, one load.)
 template <> struct Mfma<float> {
   static constexpr int kSteps = 16;         // 64 dims / 4 per MFMA
   typedef float Op;
   __device__ static Op load(const float* rowp, int off, int s, int g) {
-    return rowp[off + s * 4 + g];
+    return rowp[off + 16 * (s >> 2) + 4 * g + (s & 3)];
   }
-  __device__ static uint32_t group_bytes(int g) { return (uint32_t)g * 4u; }
-  __device__ static Op load_at(const char* p, int s) { return *reinterpret_cast<const float*>(p + s * 16); }
+  __device__ static uint32_t group_bytes(int g) { return (uint32_t)g * 16u; }
+  __device__ static Op load_at(const char* p, int s) {
+    return reinterpret_cast<const float*>(p + 64 * (s >> 2))[s & 3];
+  }
   __device__ static floatx4 mma(Op a, Op b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
@@ -183,55 +187,146 @@ struct RowGroup {
   }
 };
 
+// For lanes of one wave that exchange data through LDS without a workgroup
+// barrier.  Without a fence the compiler may treat another lane's
+// LDS write as invisible and forward a lane's own earlier store to its load
+// (it did: lanes that added nothing read back the zeros they had written).
+// This makes every lane's LDS writes before it visible to every lane's reads
+// after it.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---------------------------------------------------------------------------
-// Full score matrix (the fused_gated_indexer API).  4 waves per block, one
-// 16-row group per wave; causal tiles above the diagonal are filled with -inf
-// without computing them.  A lane writes its row's four consecutive keys of
-// a tile with one 16-byte store when `vec` (scores, s_sb and s_st allow it).
+// Full score matrix (the fused_gated_indexer API).  One wave takes 16 query
+// rows and `tpw` consecutive 16-key tiles (a multiple of four), so that the chip
+// is full whatever T is; the 4 waves of a block take neighbouring tiles of one
+// row group.  Four tiles at a time go through the wave's LDS tile and out by
+// rows: 256 contiguous bytes of 4 rows per store instruction when `vec` (scores,
+// s_sb and s_st allow 16-byte stores), of one row otherwise.  Causal tiles above
+// the diagonal are filled with -inf without computing them.
+// Bound by writing the matrix (268 MB at T = 8192, 41 us at the rate of a fill) and
+// by the 5 transcendental instructions per score (36 us there): 77 us in bf16,
+// 231 in fp32 (its matrix instruction: 125).  One wave per row group for the whole
+// row, 64-byte pieces of 16 rows per store: 475 and 1078.
 // ---------------------------------------------------------------------------
+constexpr int kScoreStride = 68;          // floats per row of the LDS tile (64 keys, padded)
+
 template <typename T>
 __global__ __launch_bounds__(256) void indexer_scores_kernel(IdxArgs p, int causal, float* S,
-                                                             int64_t s_sb, int64_t s_st, int vec) {
+                                                             int64_t s_sb, int64_t s_st, int vec, int tpw,
+                                                             int nchunks, int row_step) {
+  __shared__ __align__(16) float st[4][16 * kScoreStride];
   const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ngroups = (p.T + 15) >> 4;
-  const int wv = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wv >= p.B * ngroups) return;
-  const int b = wv / ngroups;
-  const int r0 = (wv % ngroups) * 16;
-  const int g = lane >> 4, lr = lane & 15;
-  const int row = r0 + lr;
+  const int unit = blockIdx.x / nchunks;                 // (batch, row group)
+  const int b = unit / ngroups;
+  // Causal rows compute their first chunks and only fill the rest, the more the
+  // later the row.  Blocks go round robin over 8 XCDs and their 32 CUs, so a
+  // plain order gives a CU always the same chunk: the chunks shift with the row
+  // group and with every 32 of them, and the row groups come in steps of about
+  // 0.62 of their number, which spreads any regular pick of them over the matrix.
+  // (T = 8192, bf16: 97 us in the plain order.)
+  const int r0 = (int)((int64_t)(unit % ngroups) * row_step % ngroups) * 16, nrows = min(16, p.T - r0);
+  const int j_first = ((int)(blockIdx.x + unit + unit / 32) % nchunks * 4 + wave) * tpw * 16;
+  const int j_last = min(p.T, j_first + tpw * 16);       // this wave's keys [j_first, j_last)
+  if (j_first >= p.T) return;
+  const float ninf = -__builtin_inff();
+  float* const s0 = S + b * s_sb + (int64_t)r0 * s_st;
+  const int jend = causal ? min(j_last, r0 + 16) : j_last;    // keys from here on are above the diagonal
 
-  RowGroup<T> rg;
-  rg.init(p, b, r0, lane);
-  float* srow = S + b * s_sb + (int64_t)min(row, p.T - 1) * s_st;
-  auto put = [&](int col0, const float (&v)[4]) {
-    if (row >= p.T) return;
-    if (vec && col0 + 3 < p.T) {
-      *reinterpret_cast<floatx4*>(srow + col0) = floatx4{v[0], v[1], v[2], v[3]};
-    } else {
+  if (j_first < jend) {
+    const int g = lane >> 4, lr = lane & 15;
+    const int row = r0 + lr;
+    float* const tile = st[wave];
+    RowGroup<T> rg;
+    rg.init(p, b, r0, lane);
+    // Whole quads below the diagonal.  Keys are requested two tiles ahead.  Loads
+    // and stores complete in one order, so a wait for keys also waits for the
+    // stores issued before them: with two tiles between, those have had the time.
+    typename Mfma<T>::Op k[4][Mfma<T>::kSteps];
+    const int jfull =
+        nrows < 16 ? j_first : j_first + max(0, (causal ? min(j_last, r0) : j_last) - j_first) / 64 * 64;
+    int jq = j_first;
+    if (jq < jfull) {
+      rg.load_keys(jq, p.T, lane, k[0]);
+      rg.load_keys(jq + 16, p.T, lane, k[1]);
+      for (; jq < jfull; jq += 64) {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (col0 + e < p.T) srow[col0 + e] = v[e];
+        for (int u = 0; u < 4; ++u) {
+          rg.load_keys(min(jq + 16 * (u + 2), jfull - 16), p.T, lane, k[(u + 2) & 3]);
+          floatx4 acc[kHi];
+          float v[4];
+          rg.mma(k[u], acc);
+          rg.score4(acc, v);
+          *reinterpret_cast<floatx4*>(tile + lr * kScoreStride + 16 * u + 4 * g) = floatx4{v[0], v[1], v[2], v[3]};
+        }
+        wave_lds_sync();
+        if (vec) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int r = 4 * i + (lane >> 4), c = 4 * (lane & 15);
+            *reinterpret_cast<floatx4*>(s0 + (int64_t)r * s_st + jq + c) =
+                *reinterpret_cast<const floatx4*>(tile + r * kScoreStride + c);
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s0[(int64_t)r * s_st + jq + lane] = tile[r * kScoreStride + lane];
+        }
+        wave_lds_sync();                                 // the reads before the next tiles' writes
+      }
     }
-  };
-
-  const int jend = causal ? min(p.T, r0 + 16) : p.T;
-  typename Mfma<T>::Op kb[Mfma<T>::kSteps], kn[Mfma<T>::kSteps];
-  rg.load_keys(0, p.T, lane, kn);
-  for (int j0 = 0; j0 < jend; j0 += 16) {
+    // the quad with the diagonal or the last keys, or whatever the above leaves
+    for (; jq < jend; jq += 64) {
 #pragma unroll
-    for (int s = 0; s < Mfma<T>::kSteps; ++s) kb[s] = kn[s];
-    if (j0 + 16 < jend) rg.load_keys(j0 + 16, p.T, lane, kn);
-    floatx4 acc[kHi];
-    rg.mma(kb, acc);
-    const int col0 = j0 + 4 * g;
-    float v[4];
+      for (int u = 0; u < 4; ++u) {
+        const int j0 = jq + 16 * u;
+        float v[4] = {ninf, ninf, ninf, ninf};
+        if (j0 < jend) {
+          rg.load_keys(j0, p.T, lane, k[0]);
+          floatx4 acc[kHi];
+          rg.mma(k[0], acc);
+          rg.score4(acc, v);
+          if (causal && j0 == r0) {                      // the diagonal tile
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = (causal && col0 + e > row) ? -__builtin_inff() : rg.score(acc, e);
-    put(col0, v);
+            for (int e = 0; e < 4; ++e) v[e] = j0 + 4 * g + e > row ? ninf : v[e];
+          }
+        }
+        *reinterpret_cast<floatx4*>(tile + lr * kScoreStride + 16 * u + 4 * g) = floatx4{v[0], v[1], v[2], v[3]};
+      }
+      wave_lds_sync();
+      if (vec) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * i + (lane >> 4), c = 4 * (lane & 15);
+          const floatx4 x = *reinterpret_cast<const floatx4*>(tile + r * kScoreStride + c);
+          float* dst = s0 + (int64_t)r * s_st + jq + c;
+          if (r < nrows) {
+            if (jq + c + 3 < j_last) *reinterpret_cast<floatx4*>(dst) = x;
+            else
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                if (jq + c + e < j_last) dst[e] = x[e];
+          }
+        }
+      } else {
+        for (int r = 0; r < nrows; ++r)
+          if (jq + lane < j_last) s0[(int64_t)r * s_st + jq + lane] = tile[r * kScoreStride + lane];
+      }
+      wave_lds_sync();                                   // the reads before the next tiles' writes
+    }
   }
-  const float ninf[4] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-  for (int j0 = ((jend + 15) >> 4) << 4; j0 < p.T; j0 += 16) put(j0 + 4 * g, ninf);
+  // the rest of the wave's keys, above the diagonal, one row after another
+  const int jf = j_first < jend ? min(j_last, j_first + (jend - j_first + 63) / 64 * 64) : j_first;
+  for (int r = 0; r < nrows; ++r) {
+    float* const row = s0 + (int64_t)r * s_st;
+    const int nv = vec ? (j_last - jf) & ~3 : 0;
+    for (int j = 4 * lane; j < nv; j += 256) *reinterpret_cast<floatx4*>(row + jf + j) = floatx4{ninf, ninf, ninf, ninf};
+    for (int j = jf + nv + lane; j < j_last; j += 64) row[j] = ninf;
+  }
 }
 // ---------------------------------------------------------------------------
 // Fused indexer + exact top-k.
@@ -356,18 +451,6 @@ __device__ __forceinline__ int wave_suffix(int v, int lane) {
   }
   return v;
 }
-// The lanes of one wave exchange counts through LDS in the resolve, without
-// a workgroup barrier.  Without a fence the compiler may treat another lane's
-// LDS write as invisible and forward a lane's own earlier store to its load
-// (it did: lanes that added nothing read back the zeros they had written).
-// This makes every lane's LDS writes before it visible to every lane's reads
-// after it.
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Inclusive prefix sum over the lanes.
 __device__ __forceinline__ int wave_prefix(int v, int lane) {
 #pragma unroll
@@ -1112,6 +1195,7 @@ static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 // ---------------------------------------------------------------------------
 #include <atomic>
 #include <mutex>
+#include <numeric>
 
 using namespace gsa_host;
 
@@ -1157,14 +1241,23 @@ extern "C" int gsa_indexer_scores(const void* q_idx, int64_t q_sb, int64_t q_st,
   if (!aligned(scores, 4)) return GSA_ERR_ALIGN;
   gsa::IdxArgs a = make_idx_args(q_idx, q_sb, q_st, k_idx, k_sb, k_st, w, w_sb, w_st, bias, scale, B, T);
   const int ngroups = (T + 15) / 16;
-  const int waves = B * ngroups;
   const int vec = aligned(scores, 16) && (s_st % 4) == 0 && (s_sb % 4) == 0;
-  dim3 grid((waves + 3) / 4), block(256);
+  // tiles per wave: 16 (a wave's q and gates are loaded once for them), 4 while
+  // that leaves fewer than 4 waves per CU (us with 4 / 16: T = 512 13.4 / 17.2,
+  // T = 2048 21.4 / 19.3, T = 8192 110 / 77)
+  const int tpw = (int64_t)B * ngroups * ngroups >= 16 * 1024 ? 16 : 4;
+  const int nchunks = (ngroups + 4 * tpw - 1) / (4 * tpw);
+  if ((int64_t)B * ngroups * (nchunks + 2) > 0x7fffffffLL) return GSA_ERR_SHAPE;
+  int row_step = std::max(1, (int)(ngroups * 0.618));           // coprime to ngroups: every row group once
+  while (std::gcd(row_step, ngroups) != 1) ++row_step;
+  dim3 grid(B * ngroups * nchunks), block(256);
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (dtype == GSA_DTYPE_BF16)
-    hipLaunchKernelGGL(gsa::indexer_scores_kernel<uint16_t>, grid, block, 0, s, a, causal, scores, s_sb, s_st, vec);
+    hipLaunchKernelGGL(gsa::indexer_scores_kernel<uint16_t>, grid, block, 0, s, a, causal, scores, s_sb, s_st, vec, tpw,
+                       nchunks, row_step);
   else
-    hipLaunchKernelGGL(gsa::indexer_scores_kernel<float>, grid, block, 0, s, a, causal, scores, s_sb, s_st, vec);
+    hipLaunchKernelGGL(gsa::indexer_scores_kernel<float>, grid, block, 0, s, a, causal, scores, s_sb, s_st, vec, tpw,
+                       nchunks, row_step);
   return launch_status();
 }
 

@@ -61,6 +61,36 @@ def test_indexer_scores_noncausal(dev):
     assert torch.allclose(s, ref, rtol=2e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,T", [(1, 1), (3, 17), (1, 79), (2, 257), (1, 1100), (1, 2048), (1, 2063)])
+def test_indexer_scores_tiling(dev, dtype, causal, B, T):
+    """The score matrix at the edges of its tiling -- row groups, quads of tiles, both
+    numbers of tiles per wave, unaligned rows (odd T, a wider buffer) -- against the
+    oracle's formula in float64 on the device: fp32 sums of 64 products and of four
+    sigmoids, within rtol 2e-5 (as the other score tests), -inf exactly above the diagonal."""
+    _log(f"scores tiling {dtype} causal={causal} B={B} T={T}")
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(B, T, 4, 64, generator=g).to(dtype).to(dev)
+    k = torch.randn(B, T, 64, generator=g).to(dtype).to(dev)
+    w = torch.randn(B, T, 4, generator=g).to(dtype).to(dev)
+    bias = torch.randn(4, generator=g).to(dev)
+    ref = torch.zeros(B, T, T, dtype=torch.float64, device=dev)
+    for b in range(B):
+        for h in range(4):
+            z = (q[b, :, h].double() @ k[b].double().t().contiguous()) * 0.125 + bias[h].double()
+            ref[b] += torch.sigmoid(w[b, :, h, None].double()) * torch.sigmoid(z)
+    if causal:
+        ref.masked_fill_(torch.ones(T, T, dtype=torch.bool, device=dev).triu_(1), float("-inf"))
+    wide = torch.full((B, T + 1, T + 3), 7.0, device=dev)
+    for out in (torch.empty(B, T, T, device=dev), wide[:, :T, :T]):
+        s = _abi.indexer_scores(q, k, w, bias, 0.125, causal=causal, out=out)
+        assert torch.equal(torch.isinf(s), torch.isinf(ref))
+        fin = torch.isfinite(ref)
+        assert torch.allclose(s[fin].double(), ref[fin], rtol=2e-5, atol=1e-6)
+    assert torch.all(wide[:, T] == 7.0) and torch.all(wide[..., T:] == 7.0)     # nothing past the matrix
+
+
 def _tie_scores(B, T, levels, seed):
     g = torch.Generator().manual_seed(seed)
     s = torch.randint(0, levels, (B, T, T), generator=g).float() / levels
