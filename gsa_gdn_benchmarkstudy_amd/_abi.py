@@ -30,6 +30,7 @@ ATTN_ROPE_Q = 1
 ATTN_OUT_GATE = 2
 ATTN_MASKS_READY = 4
 ATTN_ROPE_HALVES = 8
+ATTN_SPLIT = 32
 
 # Every symbol include/gsa_hip.h declares.
 EXPORTS = (
@@ -42,6 +43,7 @@ EXPORTS = (
     "gsa_prologue_vt_lane_masks", "gsa_debug_force_select_fallback",
     "gsa_indexer_select_noalloc", "gsa_indexer_select_noalloc_max_bytes", "gsa_topk_select_i64",
     "gsa_selected_attn", "gsa_selected_attn_workspace_bytes", "gsa_masked_attn", "gsa_masked_attn_workspace_bytes",
+    "gsa_dense_attn_split_bytes",
 )
 
 _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
@@ -88,6 +90,7 @@ _PROTOS = {
                         _vp, _i64, _i64, _vp, _vp, _i64, _vp, _i64, _i64,
                         _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp], _i32),
     "gsa_dense_attn_workspace_bytes": ([_i32, _i32, _i32], ctypes.c_size_t),
+    "gsa_dense_attn_split_bytes": ([_i32, _i32, _i32, _i32, _i32], ctypes.c_size_t),
     "gsa_proj_packed_bytes": ([_i32, _i32], ctypes.c_size_t),
     "gsa_dense_lane_masks": ([_vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp], _i32),
     "gsa_prologue_vt_lane_masks": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64,
@@ -577,13 +580,14 @@ def dense_block_rows(Tkv: int) -> int:
 
 
 def prologue_vt(v, vg, k=None, cos=None, sin=None, k_out=None, vt=None, bits=None, Tkv=None, ws=None,
-                causal: bool = False):
+                causal: bool = False, split_heads: int = 0):
     """RoPE(k) -> k_out [B,T,H,d] and (v*sigmoid(vg))^T -> vt [B,H,d,ldv] (bf16).
 
     With ``bits`` (the selection bitmask [B,T,W] of keys 0..Tkv-1): the dense
     attention's lane masks are built in the same launch (gsa_prologue_vt_lane_masks)
     into ``ws`` (allocated when None), returned third: (k_out, vt, ws).  ``causal``:
-    only the tiles a causal dense_attn reads (the masks then serve causal calls only)."""
+    only the tiles a causal dense_attn reads (the masks then serve causal calls only).
+    ``split_heads``: as in dense_lane_masks."""
     lib = load()
     _need_cuda(k, v, vg, cos, sin, bits, ws)
     B, T, H, d = v.shape
@@ -614,10 +618,7 @@ def prologue_vt(v, vg, k=None, cos=None, sin=None, k_out=None, vt=None, bits=Non
     Tkv = T if Tkv is None else Tkv
     _expect(tuple(bits.shape) == (B, T, mask_words(Tkv)) and bits.stride(2) == 1 and bits.dtype == torch.int32,
             "bits: int32 [B,T,W]")
-    nbytes = lib.gsa_dense_attn_workspace_bytes(B, T, Tkv)
-    if ws is None:
-        ws = torch.empty(nbytes, device=v.device, dtype=torch.uint8)
-    _expect(ws.numel() * ws.element_size() >= nbytes and ws.is_contiguous(), "workspace too small")
+    ws, nbytes = _mask_workspace(ws, B, T, Tkv, causal, split_heads, v.device)
     st = lib.gsa_prologue_vt_lane_masks(_ptr(k), *ks, _ptr(v), *_rows(v, HD), _ptr(vg), *_rows(vg, HD), _ptr(cos),
                                         _ptr(sin), cs, B, T, H, d, dtype_code(v.dtype), _ptr(k_out), _ptr(vt),
                                         ldv, _ptr(bits), bits.stride(0), bits.stride(1), Tkv, int(bool(causal)),
@@ -717,19 +718,36 @@ def _tag_masks(ws: torch.Tensor, causal: bool) -> None:
     ws._gsa_causal_masks = bool(causal)
 
 
-def dense_lane_masks(bits, Tkv: int, ws: Optional[torch.Tensor] = None, causal: bool = False) -> torch.Tensor:
+def dense_attn_split_bytes(B: int, T: int, Tkv: int, H: int, causal: bool = True) -> int:
+    """Workspace that dense_attn(split=True) takes behind the masks; 0 where a split does not pay."""
+    return int(load().gsa_dense_attn_split_bytes(B, T, Tkv, H, int(bool(causal))))
+
+
+def _mask_workspace(ws, B: int, T: int, Tkv: int, causal: bool, split_heads: int, device):
+    """(workspace, bytes of it to use) for the dense attention's masks and, with
+    ``split_heads``, its split query blocks."""
+    nbytes = load().gsa_dense_attn_workspace_bytes(B, T, Tkv)
+    if split_heads:
+        nbytes += dense_attn_split_bytes(B, T, Tkv, split_heads, causal)
+    if ws is None:
+        ws = torch.empty(nbytes, device=device, dtype=torch.uint8)
+    _expect(ws.numel() * ws.element_size() >= nbytes and ws.is_contiguous(), "workspace too small")
+    return ws, nbytes
+
+
+def dense_lane_masks(bits, Tkv: int, ws: Optional[torch.Tensor] = None, causal: bool = False,
+                     split_heads: int = 0) -> torch.Tensor:
     """Mask operands of the dense attention from the selection bitmask [B,T,W] -> the
     workspace tensor holding them (pass it to dense_attn with masks_ready=True).
     ``causal``: only the tiles a causal dense_attn reads, up to the last row of each
-    query block (such masks serve causal calls only); otherwise every tile."""
+    query block (such masks serve causal calls only); otherwise every tile.
+    ``split_heads``: the attention's number of heads when it is to be called with
+    split=True (its workspace, counters cleared, is then part of ``ws``)."""
     lib = load()
     _need_cuda(bits, ws)
     B, T, W = bits.shape
     _expect(W == mask_words(Tkv) and bits.stride(2) == 1 and bits.dtype == torch.int32, "bits: int32 [B,T,W]")
-    nbytes = lib.gsa_dense_attn_workspace_bytes(B, T, Tkv)
-    if ws is None:
-        ws = torch.empty(nbytes, device=bits.device, dtype=torch.uint8)
-    _expect(ws.numel() * ws.element_size() >= nbytes and ws.is_contiguous(), "workspace too small")
+    ws, nbytes = _mask_workspace(ws, B, T, Tkv, causal, split_heads, bits.device)
     st = lib.gsa_dense_lane_masks(_ptr(bits), bits.stride(0), bits.stride(1), B, T, Tkv, int(bool(causal)),
                                   _ptr(ws), nbytes, _stream(bits))
     _check(st, "gsa_dense_lane_masks")
@@ -739,10 +757,12 @@ def dense_lane_masks(bits, Tkv: int, ws: Optional[torch.Tensor] = None, causal: 
 
 def dense_attn(q, k, vt, bits, scale: float, og=None, cos=None, sin=None, flags: int = 0,
                causal: bool = True, out: Optional[torch.Tensor] = None,
-               ws: Optional[torch.Tensor] = None, masks_ready: bool = False) -> torch.Tensor:
+               ws: Optional[torch.Tensor] = None, masks_ready: bool = False, split: bool = False) -> torch.Tensor:
     """Block-dense masked attention -> out [B,T,H,d] (bf16).  ``ws``: optional
     workspace (uint8 device tensor of at least dense_attn_workspace_bytes);
-    ``masks_ready``: ws already holds dense_lane_masks(bits) (bits is then not read)."""
+    ``masks_ready``: ws already holds dense_lane_masks(bits) (bits is then not read).
+    ``split``: long query blocks in parts, where dense_attn_split_bytes is not 0 (with
+    masks_ready: the masks built with split_heads=H, for one call)."""
     lib = load()
     _need_cuda(q, k, vt, bits, og, cos, sin)
     B, T, H, d = q.shape
@@ -773,17 +793,15 @@ def dense_attn(q, k, vt, bits, scale: float, og=None, cos=None, sin=None, flags:
     if out is None:
         out = torch.empty(B, T, H, d, device=q.device, dtype=q.dtype)
     _expect(tuple(out.shape) == (B, T, H, d) and out.dtype == q.dtype, "out: [B,T,H,d] in q's dtype")
-    nbytes = lib.gsa_dense_attn_workspace_bytes(B, T, Tkv)
-    if ws is None:
-        ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
-    _expect(ws.numel() * ws.element_size() >= nbytes and ws.is_contiguous(), "workspace too small")
+    ws, nbytes = _mask_workspace(ws, B, T, Tkv, causal, H if split else 0, q.device)
     os_ = _rows(og, HD) if og is not None else (0, 0)
     cs = cos.stride(0) if cos is not None else 0
     st = lib.gsa_dense_attn(_ptr(q), *_rows(q, HD), _ptr(k), *_rows(k, HD), _ptr(vt), vt.stride(0),
                             vt.stride(1), vt.shape[3], _ptr(bits), bits.stride(0), bits.stride(1),
                             _ptr(og), *os_, _ptr(cos), _ptr(sin), cs, _ptr(out), *_rows(out, HD),
                             B, T, Tkv, H, d, float(scale), dtype_code(q.dtype),
-                            int(flags) | (ATTN_MASKS_READY if masks_ready else 0), int(bool(causal)),
+                            int(flags) | (ATTN_MASKS_READY if masks_ready else 0) | (ATTN_SPLIT if split else 0),
+                            int(bool(causal)),
                             _ptr(ws), nbytes, _stream(q))
     _check(st, "gsa_dense_attn")
     return out

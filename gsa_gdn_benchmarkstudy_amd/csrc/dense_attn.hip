@@ -21,6 +21,9 @@
 // order described at the dense kernel.
 #include "gsa_common.h"
 
+#include <cmath>
+#include <type_traits>
+
 namespace gsa {
 
 // Waves per dense-attention block (32 query rows each).  The mask-operand
@@ -158,6 +161,7 @@ struct LaneMaskArgs {
   int block_rows;         // causal: query rows per attention block (tiles past a block's last row are skipped); else 0
   u32x4* lm;
   const int2* range;      // kSel: each row's tile range (Selection::range); a block's tiles outside its rows' are skipped
+  uint32_t* clear; int nclear;   // words to zero besides: the arrival counters of split query blocks
 };
 
 // Bit i of an 8-bit value moved to bit 4i.
@@ -179,6 +183,7 @@ __device__ __forceinline__ u32x4 mask_nibbles(uint32_t word) {
 template <bool kSel>
 __device__ __forceinline__ void lane_mask_block(const LaneMaskArgs& a, int blk) {
   const int gt = blk * 256 + (int)threadIdx.x;
+  if (gt < a.nclear) a.clear[gt] = 0u;
   const int unit = gt >> 5, n = gt & 31;
   if (unit >= a.nunits) return;
   const int nq = (a.NT + kLmTiles - 1) / kLmTiles;
@@ -273,7 +278,9 @@ struct DenseArgs {
   float scale_l2;
   int flags;
   const int2* range; uint8_t* redo;       // kSel: Selection::range and ::redo
+  float* parts; uint32_t* counters;       // kSplit: slots [B*H][plan.slots], arrivals [B*H][nqb]
 };
+struct NoPlan {};
 
 constexpr int kDenseCausal = 1 << 8;   // internal flag: skip key tiles after the block's last row
 constexpr float kLazy = 8.f;           // log2 headroom of the lazy softmax reference
@@ -323,8 +330,12 @@ template <int N> struct Int { static constexpr int value = N; };
 // whose sums are not positive finite numbers (no valid key, infinities or NaN
 // anywhere in its tiles, products beyond the masks' range) is marked for the
 // gather kernel.
-template <bool kSel>
-__global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseArgs p, const u32x4* __restrict__ lm) {
+//
+// kSplit: the blocks are the units of a plan, parts of long query blocks among
+// them (gsa_common.h, merge_parts), longest first over all sequences.
+template <bool kSel, bool kSplit>
+__global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(
+    DenseArgs p, const u32x4* __restrict__ lm, std::conditional_t<kSplit, UnitPlan, NoPlan> plan) {
   extern __shared__ __align__(16) u32x4 dsm[];   // K slots 0, 1 (kKU units each), V^T slots 0, 1 (kVU), mask slots 0, 1 (512)
   constexpr int kDW = kDenseWaves;                // waves per block
   constexpr int kDQ = 32 * kDW;                   // query rows per block
@@ -343,11 +354,20 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   // Block order: batch by batch (the blocks in flight then share one
   // sequence's K and V^T, which stays in the last-level cache), within a
   // sequence the heaviest query blocks first, heads fastest.
-  const int per_b = p.nqb * p.H;
-  const int b = (int)(blockIdx.x / per_b);
-  const int r2 = (int)(blockIdx.x % per_b);
-  const int qb = p.nqb - 1 - r2 / p.H;
-  const int hd = r2 % p.H;
+  int b, qb, hd;
+  Unit unit{0, 0, 1, 0};
+  if constexpr (kSplit) {
+    hd = (int)(blockIdx.x % p.H);
+    b = (int)(blockIdx.x / p.H % p.B);
+    unit = plan_unit(plan, (int)(blockIdx.x / (p.H * p.B)));
+    qb = unit.qb;
+  } else {
+    const int per_b = p.nqb * p.H;
+    b = (int)(blockIdx.x / per_b);
+    const int r2 = (int)(blockIdx.x % per_b);
+    qb = p.nqb - 1 - r2 / p.H;
+    hd = r2 % p.H;
+  }
   const int q0 = qb * kDQ;
 
   const int last_key = (p.flags & kDenseCausal) ? min(p.Tkv - 1, q0 + kDQ - 1) : p.Tkv - 1;
@@ -356,6 +376,14 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
     const int2 tr = tile_range<64>(p.range, (int64_t)b * p.T, q0, min(q0 + kDQ, p.T));
     kt0 = __builtin_amdgcn_readfirstlane(tr.x);
     nkt = __builtin_amdgcn_readfirstlane(tr.y) - kt0;
+  }
+  int parts = 1;
+  if constexpr (kSplit) {                  // this unit's share of them (a part past the tiles has none)
+    parts = min(unit.parts, nkt);
+    if (unit.part >= parts) return;
+    const int t0 = nkt * unit.part / parts, t1 = nkt * (unit.part + 1) / parts;
+    kt0 += t0;
+    nkt = t1 - t0;
   }
   const int64_t kstep = (int64_t)kDK * p.k_st * 2;             // bytes from one K tile to the next
   const char* kbase = reinterpret_cast<const char*>(p.k + b * p.k_sb + hd * 128) + kt0 * kstep;
@@ -682,7 +710,7 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
   // S^T of tile kt in sc[kt & 1]: with the loop unrolled by two, each
   // iteration writes the other pair, so no accumulator is copied
   // key tiles this wave computes: up to its last row when causal (uniform)
-  const int nkw_t = (p.flags & kDenseCausal) ? min(nkt, min(p.Tkv - 1, q0 + 32 * gw + 31) / kDK + 1) : nkt;
+  const int nkw_t = (p.flags & kDenseCausal) ? min(nkt, min(p.Tkv - 1, q0 + 32 * gw + 31) / kDK + 1 - kt0) : nkt;
   floatx16 sc[2][2];
   {
     const intx8 mop = mask_op(0);
@@ -736,6 +764,14 @@ __global__ __launch_bounds__(64 * kDenseWaves, 1) void dense_attn_kernel(DenseAr
 
   // ---- epilogue: normalise, bf16, optional output gate ----
   l = sum_halves(l);
+  if constexpr (kSplit) {
+    if (parts > 1) {
+      const int64_t bh = (int64_t)b * p.H + hd;
+      if (!merge_parts(o, m, l, p.parts + (bh * plan.slots + unit.slot) * (kDW * kPartWave), unit.part, parts, kDW, wu,
+                       lane, p.counters + bh * p.nqb + qb, reinterpret_cast<uint32_t*>(dsm)))
+        return;
+    }
+  }
   if constexpr (kSel) {
     // l and every sum of the row are finite and l > 0, and its scores stayed
     // far inside the masks' +-8e36; else the gather kernel computes the row
@@ -797,13 +833,13 @@ using namespace gsa_host;
 static constexpr int kMaxDevices = 64;
 
 // Raises the LDS limit of one instantiation on the current device (more than the default 64 KiB per block).
-template <bool kSel>
+template <bool kSel, bool kSplit>
 static int dense_lds_limit() {
   static bool done[kMaxDevices] = {};
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return GSA_ERR_SHAPE;
   if (!done[dev]) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gsa::dense_attn_kernel<kSel>),
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(gsa::dense_attn_kernel<kSel, kSplit>),
                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)gsa::kDenseLds);
     if (e != hipSuccess) return -static_cast<int>(e);
     done[dev] = true;
@@ -898,18 +934,25 @@ int lane_mask_checks(const uint32_t* bits, int64_t b_sb, int64_t b_st, int B, in
   return GSA_OK;
 }
 
+// The arrival counters behind the mask operands (room for 64 heads).
+int counter_words(int B, int T) { return B * 64 * (int)(dense_groups(T, 0) / gsa::kDenseWaves); }
+
 gsa::LaneMaskArgs lane_mask_args(const uint32_t* bits, int64_t b_sb, int64_t b_st, int B, int T, int Tkv,
-                                  int causal, void* ws) {
+                                  int causal, void* ws, size_t ws_bytes) {
   const int NT = (Tkv + 63) / 64;
   const int G = (int)dense_groups(T, Tkv);
   const int nunits = B * G * ((NT + gsa::kLmTiles - 1) / gsa::kLmTiles);
   const int block_rows = causal ? 32 * gsa::kDenseWaves : 0;
-  return gsa::LaneMaskArgs{bits, b_sb, b_st, T, G, NT, nunits, block_rows, static_cast<gsa::u32x4*>(ws), nullptr};
+  // a workspace with room for them gets its arrival counters cleared
+  const size_t base = gsa_dense_attn_workspace_bytes(B, T, Tkv);
+  const int nclear = ws_bytes >= base + (size_t)counter_words(B, T) * 4 ? counter_words(B, T) : 0;
+  return gsa::LaneMaskArgs{bits, b_sb, b_st, T, G, NT, nunits, block_rows, static_cast<gsa::u32x4*>(ws), nullptr,
+                           reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + base), nclear};
 }
 
 int launch_lane_masks(const uint32_t* bits, int64_t b_sb, int64_t b_st, int B, int T, int Tkv, int causal,
-                      void* ws, hipStream_t s) {
-  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws);
+                      void* ws, size_t ws_bytes, hipStream_t s) {
+  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes);
   hipLaunchKernelGGL(gsa::lane_mask_kernel, dim3((l.nunits + 7) / 8), dim3(256), 0, s, l);
   return launch_status();
 }
@@ -919,7 +962,7 @@ extern "C" int gsa_dense_lane_masks(const uint32_t* bits, int64_t b_sb, int64_t 
                                     int causal, void* ws, size_t ws_bytes, void* stream) {
   const int st = lane_mask_checks(bits, b_sb, b_st, B, T, Tkv, ws, ws_bytes);
   if (st) return st;
-  return launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, static_cast<hipStream_t>(stream));
+  return launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int gsa_prologue_vt_lane_masks(const void* k, int64_t k_sb, int64_t k_st,
@@ -938,13 +981,53 @@ extern "C" int gsa_prologue_vt_lane_masks(const void* k, int64_t k_sb, int64_t k
                    static_cast<const uint16_t*>(vg), g_sb, g_st, static_cast<const uint16_t*>(cos),
                    static_cast<const uint16_t*>(sin), cs_st, static_cast<uint16_t*>(k_out),
                    static_cast<uint16_t*>(vt), T, H, ldv, ldv / 64};
-  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws);
+  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes);
   const int n_pro = B * H * (ldv / 64), n_lm = (l.nunits + 7) / 8;
   if ((int64_t)n_pro + n_lm > 0x7fffffffLL) return GSA_ERR_SHAPE;
   hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel<false>, dim3(n_pro + n_lm), dim3(256), 0,
                      static_cast<hipStream_t>(stream), a, l, n_pro, n_lm);
   return launch_status();
 }
+
+namespace {
+// How the query blocks are split, by sizes alone: into parts of 1.4 of a CU's mean
+// share of the tiles, at least 8 (a part costs its prologue, its share of the sum
+// and about 4 us of exchange).  16 heads, causal, us without / with: T = 1024
+// 49 / 45, T = 1537 64 / 49, T = 2048 72 / 53, T = 3000 95 / 74, T = 4096 125 / 109;
+// from T = 5000 on the blocks balance by themselves and none is split.  Short
+// sequences of a batch (K and V of all within half the last-level cache) take the
+// plan's order, longest blocks of all sequences first: B = 3 T = 2000 98 / 87, B = 4
+// T = 4096 329 / 317.
+gsa::UnitPlan bf16_plan(int B, int T, int Tkv, int H, bool causal) {
+  const int nqb = (T + 255) / 256, nt = (Tkv + 63) / 64;
+  const int step = causal ? 4 : 0;
+  const double tiles = causal ? 2.0 * nqb * (nqb + 1) : (double)nt * nqb;
+  const double share = tiles * B * H / 256;
+  gsa::UnitPlan plan = split_plan(nqb, nt, step, (int)std::max(8.0, std::ceil(share * 1.4)));
+  if (!plan.n && B > 1 && (int64_t)B * Tkv * H * 512 <= (int64_t)128 << 20) {
+    plan = split_plan(nqb, nt, step, std::max(8, plan.tiles(nqb - 1)));
+    plan.n = nqb;
+  }
+  return plan;
+}
+
+// Behind the mask operands: the arrival counters, then the slots.
+size_t split_bytes(const gsa::UnitPlan& plan, int B, int T, int H) {
+  return (size_t)counter_words(B, T) * 4 + (size_t)B * H * plan.slots * gsa::kDenseWaves * gsa::kPartWave * 4;
+}
+
+// The units of a plan; `area`: split_bytes, its counters cleared.
+template <bool kSel>
+int launch_units(gsa::DenseArgs& a, const gsa::UnitPlan& plan, void* area, const gsa::u32x4* lm, hipStream_t s) {
+  const int st = dense_lds_limit<kSel, true>();
+  if (st) return st;
+  a.counters = static_cast<uint32_t*>(area);
+  a.parts = reinterpret_cast<float*>(a.counters + counter_words(a.B, a.T));
+  hipLaunchKernelGGL((gsa::dense_attn_kernel<kSel, true>), dim3(a.B * a.H * plan.n), dim3(64 * gsa::kDenseWaves),
+                     gsa::kDenseLds, s, a, lm, plan);
+  return launch_status();
+}
+}  // namespace
 
 extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
                               const void* k, int64_t k_sb, int64_t k_st,
@@ -959,7 +1042,7 @@ extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
                               void* stream) {
   const bool ready = (flags & GSA_ATTN_MASKS_READY) != 0;
   if (!q || !k || !vt || !out || !ws || (!ready && !bits)) return GSA_ERR_NULL;
-  if (flags & ~(GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE | GSA_ATTN_MASKS_READY | GSA_ATTN_ROPE_HALVES))
+  if (flags & ~(GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE | GSA_ATTN_MASKS_READY | GSA_ATTN_ROPE_HALVES | GSA_ATTN_SPLIT))
     return GSA_ERR_FLAGS;
   if ((flags & GSA_ATTN_ROPE_HALVES) && !(flags & GSA_ATTN_ROPE_Q)) return GSA_ERR_FLAGS;
   const bool halves = (flags & GSA_ATTN_ROPE_HALVES) != 0;
@@ -970,6 +1053,13 @@ extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
   const int NT = (Tkv + 63) / 64;
   if (ldv < NT * 64 || ldv % 64 != 0) return GSA_ERR_SHAPE;
   if (ws_bytes < gsa_dense_attn_workspace_bytes(B, T, Tkv)) return GSA_ERR_SHAPE;
+  const bool split = (flags & GSA_ATTN_SPLIT) != 0;
+  gsa::UnitPlan plan;
+  if (split) {
+    plan = bf16_plan(B, T, Tkv, H, causal != 0);
+    if (plan.n == 0 || ws_bytes < gsa_dense_attn_workspace_bytes(B, T, Tkv) + split_bytes(plan, B, T, H))
+      return GSA_ERR_SHAPE;
+  }
   // per-lane load offsets within a tile are 32-bit byte offsets
   if (k_st > (1 << 24) || (int64_t)ldv > (1 << 23)) return GSA_ERR_SHAPE;
   // the staging tiles' row offsets (32 rows) are 32-bit byte offsets
@@ -993,27 +1083,38 @@ extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
   hipStream_t s = static_cast<hipStream_t>(stream);
   const gsa::u32x4* lm = static_cast<const gsa::u32x4*>(ws);
   if (!ready) {
-    const int st = launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, s);
+    const int st = launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes, s);
     if (st) return st;
   }
-  flags &= ~GSA_ATTN_MASKS_READY;
+  flags &= ~(GSA_ATTN_MASKS_READY | GSA_ATTN_SPLIT);
   gsa::DenseArgs a{static_cast<const uint16_t*>(q), q_sb, q_st, static_cast<const uint16_t*>(k), k_sb, k_st,
                    static_cast<const uint16_t*>(vt), vt_sb, vt_sh, ldv, (int)G, NT,
                    static_cast<const uint16_t*>(og), o_sb, o_st, static_cast<const uint16_t*>(cos),
                    static_cast<const uint16_t*>(sin), cs_st, static_cast<uint16_t*>(out), out_sb, out_st,
-                   B, T, Tkv, H, nqb, scale * gsa::kLog2e, flags | (causal ? gsa::kDenseCausal : 0), nullptr, nullptr};
-  const int st = dense_lds_limit<false>();
+                   B, T, Tkv, H, nqb, scale * gsa::kLog2e, flags | (causal ? gsa::kDenseCausal : 0), nullptr, nullptr,
+                   nullptr, nullptr};
+  if (split) return launch_units<false>(a, plan, static_cast<char*>(ws) + gsa_dense_attn_workspace_bytes(B, T, Tkv), lm, s);
+  const int st = dense_lds_limit<false, false>();
   if (st) return st;
-  hipLaunchKernelGGL(gsa::dense_attn_kernel<false>, dim3(B * H * nqb), dim3(64 * W), gsa::kDenseLds, s, a, lm);
+  hipLaunchKernelGGL((gsa::dense_attn_kernel<false, false>), dim3(B * H * nqb), dim3(64 * W), gsa::kDenseLds, s, a, lm,
+                     gsa::NoPlan{});
   return launch_status();
 }
 
-// Workspace of launch_dense_selected: V^T, then the mask operands.
+extern "C" size_t gsa_dense_attn_split_bytes(int B, int T, int Tkv, int H, int causal) {
+  if (B < 1 || T < 1 || Tkv < 1 || H < 1 || H > 64) return 0;
+  const gsa::UnitPlan plan = bf16_plan(B, T, Tkv, H, causal != 0);
+  return plan.n ? split_bytes(plan, B, T, H) : 0;
+}
+
+// Workspace of launch_dense_selected: V^T, the mask operands, and the area of
+// split query blocks (query and key length alike are taken for causal).
 static size_t selected_vt_bytes(int B, int Tkv, int H) {
   return (size_t)B * H * 128 * (size_t)((Tkv + 63) / 64 * 64) * 2;
 }
 size_t gsa_host::dense_selected_bytes(int B, int T, int Tkv, int H) {
-  return selected_vt_bytes(B, Tkv, H) + gsa_dense_attn_workspace_bytes(B, T, Tkv);
+  return selected_vt_bytes(B, Tkv, H) + gsa_dense_attn_workspace_bytes(B, T, Tkv) +
+         gsa_dense_attn_split_bytes(B, T, Tkv, H, T == Tkv);
 }
 
 // V^T and the mask operands in one launch, then the attention.
@@ -1022,17 +1123,19 @@ int gsa_host::launch_dense_selected(const AttnShape& s, const gsa::Selection& se
   const int nqb = (s.T + 32 * gsa::kDenseWaves - 1) / (32 * gsa::kDenseWaves);
   uint16_t* vt = static_cast<uint16_t*>(ws);
   void* lm = static_cast<char*>(ws) + selected_vt_bytes(s.B, s.Tkv, s.H);
-  int st = dense_lds_limit<true>();
-  if (st) return st;
+  const gsa::UnitPlan plan = bf16_plan(s.B, s.T, s.Tkv, s.H, s.T == s.Tkv);
+  const size_t lm_bytes = gsa_dense_attn_workspace_bytes(s.B, s.T, s.Tkv);
   gsa::ProVtArgs p{};
   p.v = static_cast<const uint16_t*>(s.v); p.v_sb = s.v_sb; p.v_st = s.v_st;
   p.vt = vt; p.T = s.Tkv; p.H = s.H; p.ldv = ldv; p.ntiles = NT;
-  gsa::LaneMaskArgs l = lane_mask_args(sel.bits, (int64_t)s.T * 2 * NT, 2 * NT, s.B, s.T, s.Tkv, 0, lm);
+  gsa::LaneMaskArgs l = lane_mask_args(sel.bits, (int64_t)s.T * 2 * NT, 2 * NT, s.B, s.T, s.Tkv, 0, lm,
+                                       plan.n ? lm_bytes + split_bytes(plan, s.B, s.T, s.H) : lm_bytes);
   l.range = sel.range;
   const int n_pro = s.B * s.H * NT, n_lm = (l.nunits + 7) / 8;
   hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel<true>, dim3(n_pro + n_lm), dim3(256), 0, stream, p, l, n_pro,
                      n_lm);
-  if ((st = launch_status())) return st;
+  int st = launch_status();
+  if (st) return st;
   gsa::DenseArgs a{};
   a.q = static_cast<const uint16_t*>(s.q); a.q_sb = s.q_sb; a.q_st = s.q_st;
   a.k = static_cast<const uint16_t*>(s.k); a.k_sb = s.k_sb; a.k_st = s.k_st;
@@ -1042,7 +1145,10 @@ int gsa_host::launch_dense_selected(const AttnShape& s, const gsa::Selection& se
   a.B = s.B; a.T = s.T; a.Tkv = s.Tkv; a.H = s.H; a.nqb = nqb;
   a.scale_l2 = s.scale * gsa::kLog2e;
   a.range = sel.range; a.redo = sel.redo;
-  hipLaunchKernelGGL(gsa::dense_attn_kernel<true>, dim3(s.B * s.H * nqb), dim3(64 * gsa::kDenseWaves),
-                     gsa::kDenseLds, stream, a, static_cast<const gsa::u32x4*>(lm));
+  const gsa::u32x4* masks = static_cast<const gsa::u32x4*>(lm);
+  if (plan.n) return launch_units<true>(a, plan, static_cast<char*>(lm) + lm_bytes, masks, stream);
+  if ((st = dense_lds_limit<true, false>())) return st;
+  hipLaunchKernelGGL((gsa::dense_attn_kernel<true, false>), dim3(s.B * s.H * nqb), dim3(64 * gsa::kDenseWaves),
+                     gsa::kDenseLds, stream, a, masks, gsa::NoPlan{});
   return launch_status();
 }

@@ -282,14 +282,10 @@ __global__ __launch_bounds__(256) void clear_kernel(uint32_t* p, int n) {
 // 815 / 611 725, B = 2 T = 4096 1225 / 1160 1224.
 gsa::UnitPlan f32_plan(int B, int T, int Tkv, int H) {
   const int nqb = (T + gsa::kFRows - 1) / gsa::kFRows, nt = (Tkv + gsa::kFKeys - 1) / gsa::kFKeys;
-  std::vector<int> tiles(nqb, nt);
-  int64_t total = 0;
-  for (int i = 0; i < nqb; ++i) {
-    if (T == Tkv) tiles[i] = std::min(nt, 4 * (i + 1));
-    total += tiles[i];
-  }
-  const double share = (double)total * B * H / 256;
-  return split_plan(tiles, std::max(4, (int)std::ceil(share * (share < 40 ? 0.6 : 0.33))));
+  const int step = T == Tkv ? gsa::kFRows / gsa::kFKeys : 0;
+  const double tiles = step ? 0.5 * step * nqb * (nqb + 1) : (double)nt * nqb;
+  const double share = tiles * B * H / 256;
+  return split_plan(nqb, nt, step, (int)std::max(4.0, std::ceil(share * (share < 40 ? 0.6 : 0.33))));
 }
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }

@@ -6,7 +6,6 @@
 #include <stdint.h>
 
 #include <algorithm>
-#include <vector>
 
 #include "../../include/gsa_hip.h"
 
@@ -153,17 +152,35 @@ __device__ __forceinline__ void rope8(float (&x)[8], const float (&c)[8], const 
 // sums and softmax state to its slot and counts itself; the last one to arrive
 // adds all parts in their order (so the result does not depend on which was
 // last) and goes on to the epilogue.  No unit waits for another.
+//
+// Query block qb has min(nt, step * (qb + 1)) tiles (causal) or nt (step 0).
+// Blocks qs and up are split into parts of at most `chunk` tiles.  The order is
+// longest first, roughly: the unsplit blocks above 3/4 of chunk (qa .. qs-1), the
+// parts, the shorter blocks.  (A sorted table in the kernel arguments cost every
+// block 3 us to look its unit up.)
 // ---------------------------------------------------------------------------
-constexpr int kMaxUnits = 512;            // 2 KiB of kernel arguments
 struct UnitPlan {
-  int n;                                  // units per (batch, head), longest first; 0: one unit per query block, in the kernel's own order
+  int n;                                  // units per (batch, head); 0: no plan, the kernel's own order
   int slots;                              // partial slots per (batch, head)
-  uint32_t unit[kMaxUnits];               // query block | part << 10 | parts << 15 | first slot << 20
+  int nqb, nt, step, chunk, qs, qa;
+  uint32_t inv;                           // ceil(2^32 / chunk)
+  __host__ __device__ int tiles(int qb) const {
+    const int t = step * (qb + 1);
+    return step && t < nt ? t : nt;
+  }
 };
 struct Unit { int qb, part, parts, slot; };
-__device__ __forceinline__ Unit plan_unit(const UnitPlan& plan, int u) {
-  const uint32_t w = plan.unit[u];
-  return Unit{(int)(w & 1023u), (int)((w >> 10) & 31u), (int)((w >> 15) & 31u), (int)(w >> 20)};
+__device__ __forceinline__ Unit plan_unit(const UnitPlan& p, int u) {
+  if (u < p.qs - p.qa) return Unit{p.qs - 1 - u, 0, 1, 0};
+  u -= p.qs - p.qa;
+  int slot = 0;
+  for (int qb = p.nqb - 1; qb >= p.qs; --qb) {
+    const int parts = (int)__umulhi((uint32_t)(p.tiles(qb) + p.chunk - 1), p.inv);
+    if (u < parts) return Unit{qb, u, parts, slot};
+    u -= parts;
+    slot += parts;
+  }
+  return Unit{p.qa - 1 - u, 0, 1, 0};
 }
 // Floats of one slot: per wave 64 accumulator registers, m and l of 64 lanes.
 constexpr int kPartWave = 66 * 64;
@@ -172,27 +189,35 @@ constexpr int kPartWave = 66 * 64;
 // both lanes) and, in the last unit to arrive, replaces them by the sums over
 // all parts; false in the other units, which have nothing left to do.
 // slots: the query block's first slot; `flag`: one word of LDS that no wave
-// uses any more.  Plain stores and loads with an agent-scope release by the
-// counting thread and an acquire after it: units run on different XCDs.
+// uses any more.  The units may run on different XCDs, whose L2 caches are not
+// coherent: every value goes out and comes back by agent-scope accesses (written
+// through and read past L2), complete (vmcnt(0)) before the workgroup counts
+// itself.  (Plain stores with an agent-scope release write a whole L2 back for
+// each unit: T = 2048, bf16,
+// 63 us, 53 this way.)
+__device__ __forceinline__ void part_store(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float part_load(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ bool merge_parts(floatx16 (&o)[4], float& m, float& l, float* slots, int part, int parts,
                                             int waves, int wave, int lane, uint32_t* counter, uint32_t* flag) {
   float* const mine = slots + ((int64_t)part * waves + wave) * kPartWave + lane;
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mine[(16 * dt + r) * 64] = o[dt][r];
-  mine[64 * 64] = m;
-  mine[65 * 64] = l;
-  __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xf << 8));     // vmcnt(0): this wave's stores are in L2
+    for (int r = 0; r < 16; ++r) part_store(mine + (16 * dt + r) * 64, o[dt][r]);
+  part_store(mine + 64 * 64, m);
+  part_store(mine + 65 * 64, l);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (threadIdx.x == 0)
-    *flag = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) *flag = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   __syncthreads();
   if (*flag != (uint32_t)(parts - 1)) return false;
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   const float* const all = slots + (int64_t)wave * kPartWave + lane;
   float top = -__builtin_inff();
-  for (int s = 0; s < parts; ++s) top = fmaxf(top, all[(int64_t)s * waves * kPartWave + 64 * 64]);
+  for (int s = 0; s < parts; ++s) top = fmaxf(top, part_load(all + (int64_t)s * waves * kPartWave + 64 * 64));
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
@@ -200,13 +225,13 @@ __device__ __forceinline__ bool merge_parts(floatx16 (&o)[4], float& m, float& l
   l = 0.f;
   for (int s = 0; s < parts; ++s) {
     const float* const at = all + (int64_t)s * waves * kPartWave;
-    const float ms = at[64 * 64];
+    const float ms = part_load(at + 64 * 64);
     const float w = ms == -__builtin_inff() ? 0.f : __builtin_amdgcn_exp2f(ms - top);
-    l = __builtin_fmaf(at[65 * 64], w, l);
+    l = __builtin_fmaf(part_load(at + 65 * 64), w, l);
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) o[dt][r] = __builtin_fmaf(at[(16 * dt + r) * 64], w, o[dt][r]);
+      for (int r = 0; r < 16; ++r) o[dt][r] = __builtin_fmaf(part_load(at + (16 * dt + r) * 64), w, o[dt][r]);
   }
   m = top;
   return true;
@@ -306,28 +331,16 @@ __device__ __forceinline__ int2 tile_range(const int2* range, int64_t row_base, 
 // ---------------------------------------------------------------------------
 namespace gsa_host {
 
-// Query blocks of `tiles` key tiles each, split into parts of at most `chunk`
-// tiles, longest parts first.  n = 0 (no plan) where nothing is split or the
-// units do not fit.
-inline gsa::UnitPlan split_plan(const std::vector<int>& tiles, int chunk) {
-  gsa::UnitPlan p;
-  p.n = p.slots = 0;
-  struct U { int size; uint32_t w; };
-  std::vector<U> units;
-  if (tiles.size() > 1024 || *std::max_element(tiles.begin(), tiles.end()) <= chunk) return p;
-  for (int qb = (int)tiles.size() - 1; qb >= 0; --qb) {
-    const int parts = std::min(31, std::max(1, (tiles[qb] + chunk - 1) / chunk));
-    for (int i = 0; i < parts; ++i)
-      units.push_back({tiles[qb] * (i + 1) / parts - tiles[qb] * i / parts,
-                       (uint32_t)qb | (uint32_t)i << 10 | (uint32_t)parts << 15 | (uint32_t)p.slots << 20});
-    if (parts > 1) p.slots += parts;
-  }
-  if (p.slots == 0 || (int)units.size() > gsa::kMaxUnits) {
-    p.slots = 0;
-    return p;
-  }
-  std::stable_sort(units.begin(), units.end(), [](const U& a, const U& b) { return a.size > b.size; });
-  for (const U& u : units) p.unit[p.n++] = u.w;
+// The plan for nqb query blocks (UnitPlan) with parts of at most `chunk` >= 4
+// tiles; n = 0 where nothing is split.
+inline gsa::UnitPlan split_plan(int nqb, int nt, int step, int chunk) {
+  gsa::UnitPlan p{};
+  p.nqb = nqb; p.nt = nt; p.step = step; p.chunk = chunk;
+  p.inv = (uint32_t)((((uint64_t)1 << 32) + chunk - 1) / chunk);
+  while (p.qs < nqb && p.tiles(p.qs) <= chunk) ++p.qs;
+  while (p.qa < p.qs && 4 * p.tiles(p.qa) <= 3 * chunk) ++p.qa;
+  for (int qb = p.qs; qb < nqb; ++qb) p.slots += (p.tiles(qb) + chunk - 1) / chunk;
+  if (p.slots) p.n = p.qs + p.slots;
   return p;
 }
 

@@ -95,9 +95,11 @@ constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 // measured at 16 heads).  The gather, bf16: 20 + the larger of 0.5 per key of a
 // row (its loads are a chain within the row's block) and 0.0009 per row and
 // key (what it reads); T = 512, k = 128 89; T = 8192, k = 2048 13002.  The
-// matrix cores: 30 for the launches and 2.4 for each 64-key tile of a block's
-// 256 rows, one block per CU at a time: T = 512, k = 128 54; T = 8192, k = 2048
-// 502; T = 256, Tkv = 8192, k = 128 340, where the gather takes 89.  In
+// matrix cores: 35 for the launches and 2.4 for each 64-key tile that a CU takes one
+// after another (all tiles of its 256-row blocks, or where those are split, 1.4
+// times the mean over the CUs, 8 at least, and 25 to add the parts): T = 512, k =
+// 128 54; T = 8192, k = 2048 502; T = 64, Tkv = 4096 75 where the gather takes 52 at k
+// = 64 and 161 at k = 256.  In
 // fp32 the gather reads twice as much and takes 0.6 per key of a row; the matrix
 // cores, whose blocks are split evenly over the chip there, take 40, 9.6 for each
 // 64-key tile of a 128-row block per CU, and up to 30 to add the parts: T = 512,
@@ -116,7 +118,9 @@ bool dense_serves(int B, int T, int Tkv, int H, int k_sel, float scale, int dtyp
   const int64_t NT = (Tkv + 63) / 64, groups = ((int64_t)T + 255) / 256 * 8;
   const double reads = 0.0009 * B * T * (double)k_sel * H / 16;
   const double gather = 20.0 + (bf16 ? std::max(0.5 * k_sel, reads) : std::max(0.6 * k_sel, 2 * reads));
-  const double dense = bf16 ? 30.0 + 2.4 * NT * std::ceil(B * H * (groups / 8) / 256.0)
+  const double blocks = B * (double)H * (groups / 8), whole = NT * std::ceil(blocks / 256);
+  const double serial = std::min(whole, std::max(8.0, 1.4 * NT * blocks / 256));
+  const double dense = bf16 ? 35.0 + 2.4 * serial + (serial < whole ? 25.0 : 0.0)
                             : 40.0 + 9.6 * NT * (B * (double)H * ((T + 127) / 128) / 256.0) + std::min(30.0, 3.0 * NT);
   if (dense > gather) return false;
   if (B * groups * NT > 0x3fffffffLL / 32 || (int64_t)B * H * NT > 0x3fffffffLL) return false;

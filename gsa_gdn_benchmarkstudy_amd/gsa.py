@@ -595,6 +595,8 @@ class GatedSparseAttention(nn.Module):
         # (lane_masks_with_producer), else on a second stream that starts after
         # the indexer.
         lm_ws, lm_stream = None, None
+        # heads of a split attention (0: the sizes do not ask for one)
+        split = self.num_heads if dense and _abi.dense_attn_split_bytes(B, T, T, self.num_heads) else 0
         lm_in_producer = (dense and not fused_proj and mode == "serial" and self.lane_masks_with_producer)
         if dense and not lm_in_producer:
             lm_stream = side if side is not cur else self._side_stream(dev)
@@ -602,7 +604,7 @@ class GatedSparseAttention(nn.Module):
                 lm_stream.wait_stream(cur)
             with torch.cuda.stream(lm_stream):
                 _range_push("gsa_hip/lane_masks")
-                lm_ws = _abi.dense_lane_masks(bits, T, causal=True)   # the layer's attention is causal
+                lm_ws = _abi.dense_lane_masks(bits, T, causal=True, split_heads=split)   # the layer's attention is causal
                 _range_pop()
         if mode != "producer":
             _range_push("gsa_hip/main_gemm")
@@ -615,7 +617,7 @@ class GatedSparseAttention(nn.Module):
             k_rope, v_gated = views["_k_rope"], views["_vt"]
         elif lm_in_producer:
             k_rope, v_gated, lm_ws = _abi.prologue_vt(views["v"], views["vg"], k=views["k"], cos=cos, sin=sin,
-                                                      bits=bits, Tkv=T, causal=True)
+                                                      bits=bits, Tkv=T, causal=True, split_heads=split)
         elif dense:
             k_rope, v_gated = _abi.prologue_vt(views["v"], views["vg"], k=views["k"], cos=cos, sin=sin)
         else:
@@ -645,10 +647,11 @@ class GatedSparseAttention(nn.Module):
             if cs is not None:
                 attn = _abi.dense_attn(views["q"], k_rope, v_gated, bits, self.scale, og=views["og"],
                                        cos=cs, flags=flags | _abi.ATTN_ROPE_HALVES, causal=True, ws=lm_ws,
-                                       masks_ready=True)
+                                       masks_ready=True, split=split > 0)
             else:
                 attn = _abi.dense_attn(views["q"], k_rope, v_gated, bits, self.scale, og=views["og"],
-                                       cos=cos, sin=sin, flags=flags, causal=True, ws=lm_ws, masks_ready=True)
+                                       cos=cos, sin=sin, flags=flags, causal=True, ws=lm_ws, masks_ready=True,
+                                       split=split > 0)
         elif masked:
             attn = _abi.masked_attn(views["q"], k_rope, v_gated, bits, k_sel, self.scale, og=views["og"], cos=cos,
                                     sin=sin, flags=flags)

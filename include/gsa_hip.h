@@ -59,6 +59,7 @@ extern "C" {
 #define GSA_ATTN_ROPE_Q   1  /* q is pre-RoPE: apply RoPE with cos/sin in the prologue  */
 #define GSA_ATTN_OUT_GATE 2  /* multiply the output by sigmoid(og) (the G1 output gate) */
 #define GSA_ATTN_MASKS_READY 4  /* gsa_dense_attn: ws already holds gsa_dense_lane_masks of bits */
+#define GSA_ATTN_SPLIT    32  /* gsa_dense_attn: split long query blocks along their keys (ws holds split_bytes more) */
 #define GSA_ATTN_ROPE_HALVES 8  /* gsa_dense_attn with GSA_ATTN_ROPE_Q: cos is the packed table below */
 
 /* Largest k_eff of gsa_topk_select in GSA_ORDER_SCORE_DESC order. */
@@ -388,6 +389,19 @@ int gsa_selection_mask(const int32_t* idx, int64_t i_sb, int64_t i_st, int k_sel
  * bit-identical to the call with the full cos and sin tables.
  */
 size_t gsa_dense_attn_workspace_bytes(int B, int T, int Tkv);
+
+/*
+ * GSA_ATTN_SPLIT: where the query blocks are few or, causal, of very different
+ * length, the long ones are split along their keys and their parts added in a
+ * fixed order (other sums than without the flag, same accuracy, the same bits on
+ * each call).  It takes gsa_dense_attn_split_bytes more workspace behind the
+ * masks -- 0 where a split does not pay; the flag is then GSA_ERR_SHAPE.  The
+ * call that writes the masks (gsa_dense_lane_masks, gsa_prologue_vt_lane_masks,
+ * or gsa_dense_attn itself) clears the counters there, if its ws_bytes covers
+ * them: with GSA_ATTN_MASKS_READY that call has to have had the same ws_bytes, and
+ * each GSA_ATTN_SPLIT call needs such a call before it.
+ */
+size_t gsa_dense_attn_split_bytes(int B, int T, int Tkv, int H, int causal);
 
 /*
  * The first step of gsa_dense_attn on its own: the selection bitmask ->

@@ -745,6 +745,54 @@ def test_dense_attention_masked_tiles_add_nothing(dev):
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("B,T,Tkv,H,causal", [
+    (1, 768, 768, 16, True), (1, 1537, 1537, 16, True), (1, 2049, 2049, 16, True),    # split causal blocks
+    (3, 1100, 1100, 16, True),                                                          # the plan's order alone
+    (1, 100, 3000, 4, False), (2, 300, 1000, 8, False), (1, 513, 9000, 1, False),       # every block split alike, up to 18 parts
+])
+def test_dense_attention_split_blocks(dev, B, T, Tkv, H, causal):
+    """GSA_ATTN_SPLIT: query blocks in parts, against the unsplit call; the same bits on
+    every call; rows without a key are 0.  A part's weights p = 2^(s - m) are rounded to
+    bf16 against its own reference m, so each of the two calls is within 2^-9 sum p|v| / l
+    <= 2^-9 max|v| of the unrounded weights' result, 2^-8 max|v| apart in all, before the
+    two roundings of the output (the attention, the gated product: 2^-7 each)."""
+    _log(f"split dense B={B} T={T} Tkv={Tkv} H={H} causal={causal}")
+    g = torch.Generator().manual_seed(T + Tkv)
+    q = torch.randn(B, T, H, 128, generator=g).to(torch.bfloat16).to(dev)
+    k = torch.randn(B, Tkv, H, 128, generator=g).to(torch.bfloat16).to(dev)
+    v = torch.randn(B, Tkv, H, 128, generator=g).to(torch.bfloat16).to(dev)
+    og = torch.randn(B, T, H, 128, generator=g).to(torch.bfloat16).to(dev)
+    vt = torch.zeros(B, H, 128, _abi.vt_len(Tkv), dtype=torch.bfloat16, device=dev)
+    vt[..., :Tkv] = v.permute(0, 2, 3, 1)
+    sel = torch.rand(B, T, Tkv, generator=g) < 0.3
+    if causal:
+        sel &= torch.ones(T, Tkv, dtype=torch.bool).tril()
+    sel[:, 5] = False
+    pad = torch.zeros(B, T, 32 * _abi.mask_words(Tkv), dtype=torch.bool)
+    pad[..., :Tkv] = sel
+    bits = torch.from_numpy(np.packbits(pad.numpy(), axis=-1, bitorder="little").view(np.int32)).to(dev)
+    assert _abi.dense_attn_split_bytes(B, T, Tkv, H, causal) > 0
+    kw = dict(og=og, flags=_abi.ATTN_OUT_GATE, causal=causal)
+    one = _abi.dense_attn(q, k, vt, bits, 128 ** -0.5, **kw)
+    ws = _abi.dense_lane_masks(bits, Tkv, causal=causal, split_heads=H)
+    a = _abi.dense_attn(q, k, vt, bits, 128 ** -0.5, ws=ws, masks_ready=True, split=True, **kw)
+    for _ in range(3):
+        assert torch.equal(a, _abi.dense_attn(q, k, vt, bits, 128 ** -0.5, split=True, **kw))
+    diff = (a.double() - one.double()).abs()
+    assert torch.all(diff <= one.double().abs() * 2.0 ** -6 + v.double().abs().max() * 2.0 ** -8)
+    assert torch.all(a[:, 5] == 0)
+
+
+def test_dense_attention_split_refused_where_it_does_not_pay(dev):
+    """No plan, no split: GSA_ERR_SHAPE, as for a workspace without its area."""
+    assert _abi.dense_attn_split_bytes(1, 16384, 16384, 16) == 0 and _abi.dense_attn_split_bytes(1, 2048, 2048, 65) == 0
+    q = torch.zeros(1, 64, 2, 128, dtype=torch.bfloat16, device=dev)
+    vt = torch.zeros(1, 2, 128, 64, dtype=torch.bfloat16, device=dev)
+    bits = torch.zeros(1, 64, 2, dtype=torch.int32, device=dev)
+    with pytest.raises(RuntimeError, match="status 2"):
+        _abi.dense_attn(q, q, vt, bits, 0.1, split=True)
+
+
 @pytest.mark.parametrize("causal_masks", [True, False])
 def test_dense_lane_masks_then_attention_equals_one_call(dev, causal_masks):
     """gsa_dense_lane_masks on another stream, then gsa_dense_attn with
