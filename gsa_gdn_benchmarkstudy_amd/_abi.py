@@ -43,7 +43,7 @@ EXPORTS = (
     "gsa_prologue_vt_lane_masks", "gsa_debug_force_select_fallback",
     "gsa_indexer_select_noalloc", "gsa_indexer_select_noalloc_max_bytes", "gsa_topk_select_i64",
     "gsa_selected_attn", "gsa_selected_attn_workspace_bytes", "gsa_masked_attn", "gsa_masked_attn_workspace_bytes",
-    "gsa_dense_attn_split_bytes",
+    "gsa_dense_attn_split_bytes", "gsa_layer_attn", "gsa_layer_workspace_bytes",
 )
 
 _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
@@ -91,6 +91,9 @@ _PROTOS = {
                         _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp], _i32),
     "gsa_dense_attn_workspace_bytes": ([_i32, _i32, _i32], ctypes.c_size_t),
     "gsa_dense_attn_split_bytes": ([_i32, _i32, _i32, _i32, _i32], ctypes.c_size_t),
+    "gsa_layer_workspace_bytes": ([_i32, _i32, _i32, _i32], ctypes.c_size_t),
+    "gsa_layer_attn": ([_vp, _i64, _i64, _vp, _vp, _f32, _vp, _vp, _i64, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _i32,
+                        _f32, _i32, _i32, _i32, _i32, _vp, _vp, _i64, _i64, _vp, ctypes.c_size_t, _vp], _i32),
     "gsa_proj_packed_bytes": ([_i32, _i32], ctypes.c_size_t),
     "gsa_dense_lane_masks": ([_vp, _i64, _i64, _i32, _i32, _i32, _i32, _vp, ctypes.c_size_t, _vp], _i32),
     "gsa_prologue_vt_lane_masks": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64,
@@ -805,3 +808,36 @@ def dense_attn(q, k, vt, bits, scale: float, og=None, cos=None, sin=None, flags:
                             _ptr(ws), nbytes, _stream(q))
     _check(st, "gsa_dense_attn")
     return out
+
+
+def row_offsets(offsets) -> ctypes.Array:
+    """The eight element offsets of layer_attn's projection rows, as the library takes them."""
+    return (ctypes.c_int64 * 8)(*offsets)
+
+
+def layer_attn(proj, offsets, bias32, idx_scale: float, cos, sin, halves, H: int, d: int, Hi: int, di: int,
+               scale: float, k_eff: int, adaptive=None, stream: Optional[int] = None):
+    """The layer between its GEMMs in one call (gsa_layer_attn) -> (attention output
+    [B,T,H,d], per-row k int32 [B,T] or None).  proj: contiguous bf16 [B,T,N] rows of all
+    eight projections at ``offsets`` (row_offsets); ``adaptive``: (k_base, k_min, k_max) of
+    the variance rule, or None for k_eff keys per row."""
+    lib = load()
+    _need_cuda(proj, bias32, cos, sin, halves)
+    B, T, N = proj.shape
+    _expect(proj.dtype == torch.bfloat16 and proj.is_contiguous() and N >= offsets[7] + Hi, "proj: bf16 rows")
+    for t in (cos, sin, halves):
+        _expect(t.dtype == proj.dtype and t.dim() == 2 and t.shape[0] >= T and t.shape[1] == d and t.is_contiguous(),
+                "cos, sin, halves: contiguous [>=T, d]")
+    _expect(bias32.dtype == torch.float32 and bias32.numel() == Hi and bias32.is_contiguous(), "bias: fp32 [Hi]")
+    dev = proj.device
+    need = lib.gsa_layer_workspace_bytes(B, T, H, int(adaptive is not None))
+    ws = torch.empty(need, device=dev, dtype=torch.uint8)
+    out = torch.empty(B, T, H, d, device=dev, dtype=proj.dtype)
+    k_rows = torch.empty(B, T, device=dev, dtype=torch.int32) if adaptive is not None else None
+    kb, kmin, kmax = adaptive if adaptive is not None else (0, 0, 0)
+    st = lib.gsa_layer_attn(proj.data_ptr(), T * N, N, offsets, bias32.data_ptr(), idx_scale, cos.data_ptr(),
+                            sin.data_ptr(), d, halves.data_ptr(), d, B, T, H, d, Hi, di, scale,
+                            0 if adaptive is not None else k_eff, kb, kmin, kmax, _ptr(k_rows), out.data_ptr(),
+                            T * H * d, H * d, ws.data_ptr(), need, _stream(proj) if stream is None else stream)
+    _check(st, "gsa_layer_attn")
+    return out, k_rows

@@ -26,7 +26,7 @@ ARCH = "gfx950"
 
 HIP_SOURCES = ("indexer.hip", "topk_select.hip", "sparse_attn.hip", "dense_attn.hip", "dense_attn_f32.hip",
                "selected_attn.hip", "proj_fused.hip")
-CXX_SOURCES = ("abi.cpp",)
+CXX_SOURCES = ("abi.cpp", "layer.cpp")
 
 # Packed fp32 VALU forms are disabled in device code: the compiler would
 # otherwise form v_pk_{add,mul,fma}_f32 from ordinary float code.

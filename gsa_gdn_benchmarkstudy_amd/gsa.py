@@ -33,17 +33,8 @@ from .roctx import range_pop as _range_pop, range_push as _range_push
 FUSED_ALIGN = 64
 
 
-_CU_COUNT = {}
 # Last-level (Infinity) cache of one MI355X.
 _LLC_BYTES = 256 << 20
-
-
-def _cu_count(dev: torch.device) -> int:
-    """Compute units of the device (cached)."""
-    idx = dev.index if dev.index is not None else torch.cuda.current_device()
-    if idx not in _CU_COUNT:
-        _CU_COUNT[idx] = torch.cuda.get_device_properties(idx).multi_processor_count
-    return _CU_COUNT[idx]
 
 
 # ---------------------------------------------------------------------------
@@ -317,9 +308,9 @@ class GatedSparseAttention(nn.Module):
          writing the selection as a bitmask, and for the gather attention
          ascending int32 indices with per-row counts (no score is stored:
          they are recomputed pass by pass and the candidates near each row's
-         threshold stay in LDS) -- beside the q/k/v/gate GEMM while its grid leaves
-         CUs free, before it while RoPE(k) and V^T fit the last-level cache,
-         else beside the producer; the dense attention's lane masks
+         threshold stay in LDS) -- before the q/k/v/gate GEMM while RoPE(k) and
+         V^T fit the last-level cache, else beside the producer (or beside the
+         GEMM, on request); the dense attention's lane masks
          (gsa_dense_lane_masks) follow on the second stream (with the
          indexer on the current stream: built in the producer's launch);
       3. current stream: RoPE(k) and v * sigmoid(vg) (gsa_prologue_vt, V
@@ -328,6 +319,8 @@ class GatedSparseAttention(nn.Module):
          gsa_dense_attn (bf16: MFMA over every causal key tile, masked to the
          selection), gsa_masked_attn (its fp32 form) or gsa_sparse_attn
          (per-row gather of the selected keys) -- and the o_proj GEMM.
+    Short bf16 sequences: steps 1 (one GEMM for all projections), 2-4 (one
+    library call, gsa_layer_attn) and o_proj, on the current stream.
     """
 
     def __init__(self, hidden_size: int, num_heads: int, k_max: int = 4096, d_indexer: int = 64,
@@ -353,6 +346,7 @@ class GatedSparseAttention(nn.Module):
         self._fused_bias: Optional[torch.Tensor] = None
         self._packed: Optional[tuple] = None
         self._idx_bias32: Optional[torch.Tensor] = None
+        self._row_offsets = None
         self._proj_sizes = [
             hidden_size, hidden_size, hidden_size, hidden_size, hidden_size,
             n_idx_heads * d_indexer, d_indexer, n_idx_heads,
@@ -369,12 +363,15 @@ class GatedSparseAttention(nn.Module):
         # Where the fused indexer + top-k runs relative to the main projection
         # GEMM: "gemm" (on a side stream beside the GEMM), "producer" (after
         # the GEMM, on a side stream beside the RoPE/gate producer), "serial"
-        # (everything on the current stream) or "auto": "gemm" while the
-        # indexer's grid (one block per 16 query rows) leaves CUs free for the
-        # GEMM -- fewer than 4 blocks per CU; else "serial" while RoPE(k) and
-        # V^T together fit the 256 MB last-level cache (the producer then
-        # runs right before the attention, which finds them cached); else
-        # "producer".
+        # (everything on the current stream) or "auto": bf16 up to
+        # SHORT_TOKENS tokens, one GEMM for all eight projections and one call
+        # for everything between it and o_proj (_forward_short); else "serial"
+        # while RoPE(k) and V^T together fit the 256 MB last-level cache (the
+        # producer then runs right before the attention, which finds them
+        # cached); else "producer".  Two streams cost two event pairs and gain
+        # little while the select fills the chip: us per forward, "gemm" /
+        # "serial", T=2048 274 / 184, B=2 T=3001 444 / 408, T=8192 781 / 751,
+        # T=4096 342 / 356.
         self.indexer_overlap = "auto"
         # Main projection on the bf16 block-dense path: "gemm" (hipBLASLt GEMM,
         # then the RoPE / value-gate producer kernel) or "fused" (own MFMA GEMM
@@ -534,6 +531,45 @@ class GatedSparseAttention(nn.Module):
             return False
         return True
 
+    # Tokens (B*T) up to which one GEMM over the whole fused weight is faster than
+    # the indexer's and the main one, bf16, D=2048, us: 512 30 against 51, 2048 96
+    # against 109, 4096 147 against 175, 6002 200 against 205, 7000 315 against 238.
+    SHORT_TOKENS = 6144
+
+    def _short(self, x: torch.Tensor) -> bool:
+        """Whether forward takes _forward_short (bf16, block-dense attention, one stream)."""
+        B, T, _ = x.shape
+        return (0 < B * T <= self.SHORT_TOKENS and x.dtype == torch.bfloat16 and self.indexer_overlap == "auto"
+                and self.attn_impl in ("auto", "dense") and self.proj_impl == "gemm" and self.attn_events is None
+                and self.lane_masks_with_producer and T <= self.FUSED_SELECT_MAX_T)
+
+    def _forward_short(self, x: torch.Tensor, cs: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.Tensor:
+        """The forward of a short sequence, whose pace the host would set: one GEMM,
+        one library call (gsa_layer_attn) and o_proj, on the current stream."""
+        B, T, D = x.shape
+        w, b = self._get_fused_weight(x)
+        bias = self._idx_bias32
+        if bias is None or bias.device != x.device:
+            bias = self._idx_bias32 = self.indexer.idx_bias.detach().float().contiguous()
+        if self._row_offsets is None:
+            self._row_offsets = _abi.row_offsets(self._offsets().values())
+        sel = self.topk_selector
+        _range_push("gsa_hip/projections")
+        comb = F.linear(x, w, b)
+        _range_pop()
+        _range_push("gsa_hip/select_attn")
+        attn, k_rows = _abi.layer_attn(
+            comb, self._row_offsets, bias, self.indexer.scale, cos, sin, cs, self.num_heads, self.d_head,
+            self.indexer.n_idx_heads, self.indexer.d_indexer, self.scale, sel.k_effective(T),
+            (sel.k_base, sel.k_min, sel.k_max) if sel.adaptive() else None)
+        if k_rows is not None:
+            sel.last_k = k_rows
+        _range_pop()
+        _range_push("gsa_hip/o_proj")
+        out = F.linear(attn.view(B, T, D), self.o_proj.weight)
+        _range_pop()
+        return out
+
     def forward(self, x: torch.Tensor, attention_mask: Optional[torch.Tensor] = None) -> torch.Tensor:
         if not x.is_cuda:
             raise RuntimeError("GatedSparseAttention (HIP) needs a device tensor")
@@ -542,6 +578,12 @@ class GatedSparseAttention(nn.Module):
             raise ValueError(f"hidden size {D} != {self.hidden_size}")
         _range_push("gsa_hip/forward")
         dev = x.device
+        if self._short(x):
+            cs = self.rotary_emb.halves(T, dev, x.dtype)
+            if cs is not None:                       # (None: a cache edited by hand)
+                out = self._forward_short(x, cs, *self.rotary_emb(T, dev, x.dtype))
+                _range_pop()
+                return out
         cur = torch.cuda.current_stream(dev)
 
         dense = self.uses_dense(x.dtype)
@@ -567,12 +609,7 @@ class GatedSparseAttention(nn.Module):
         # that size the producer is better hidden beside the indexer.
         mode = self.indexer_overlap
         if mode == "auto":
-            if B * ((T + 15) // 16) < 4 * _cu_count(dev):
-                mode = "gemm"
-            elif 2 * B * T * D * x.element_size() <= _LLC_BYTES:
-                mode = "serial"
-            else:
-                mode = "producer"
+            mode = "serial" if 2 * B * T * D * x.element_size() <= _LLC_BYTES else "producer"
         elif mode not in ("producer", "gemm", "serial"):
             raise ValueError(f"indexer_overlap {mode!r}: expected 'auto', 'producer', 'gemm' or 'serial'")
         _range_push("gsa_hip/indexer_gemm")

@@ -446,6 +446,29 @@ int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
                    void* stream);
 
 /*
+ * The layer between its projection GEMM and o_proj (gsa_triton/gsa_opt.py:
+ * 640-721) in one call, causal, bf16: gsa_indexer_select (k_eff >= 1) or
+ * gsa_indexer_select_adaptive (k_eff == 0: k_base, k_min, k_max; k_out nullable
+ * int32 [B*T]), gsa_prologue_vt_lane_masks and gsa_dense_attn with RoPE(q), the
+ * output gate and, where it pays, GSA_ATTN_SPLIT, in stream order; same checks,
+ * results and limits as those.
+ * proj: the projections of all tokens, [B,T,..] rows (p_sb, p_st); offsets: the
+ * eight element offsets of q, k, v, vg, og, idx_q, idx_k, idx_w in a row.
+ * cos, sin [T,d] (cs_st) for k; halves: the packed table of GSA_ATTN_ROPE_HALVES
+ * (h_st) for q.  out [B,T,H,d].  ws: gsa_layer_workspace_bytes(B, T, H, k_eff == 0)
+ * bytes, 256-byte aligned, overwritten.
+ */
+size_t gsa_layer_workspace_bytes(int B, int T, int H, int adaptive);
+
+int gsa_layer_attn(const void* proj, int64_t p_sb, int64_t p_st, const int64_t* offsets,
+                   const float* idx_bias, float idx_scale,
+                   const void* cos, const void* sin, int64_t cs_st, const void* halves, int64_t h_st,
+                   int B, int T, int H, int d, int Hi, int di, float scale,
+                   int k_eff, int k_base, int k_min, int k_max, int32_t* k_out,
+                   void* out, int64_t out_sb, int64_t out_st,
+                   void* ws, size_t ws_bytes, void* stream);
+
+/*
  * Main projection GEMM with the producer fused into its epilogue.
  * Replaces the phase-1 projection GEMM and its split (gsa_triton/gsa_opt.py:
  * 629-638) together with the track-B producer steps that follow it: the
