@@ -44,6 +44,7 @@ EXPORTS = (
     "gsa_indexer_select_noalloc", "gsa_indexer_select_noalloc_max_bytes", "gsa_topk_select_i64",
     "gsa_selected_attn", "gsa_selected_attn_workspace_bytes", "gsa_masked_attn", "gsa_masked_attn_workspace_bytes",
     "gsa_dense_attn_split_bytes", "gsa_layer_attn", "gsa_layer_workspace_bytes",
+    "gsa_rope_qk",
 )
 
 _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_float
@@ -71,6 +72,8 @@ _PROTOS = {
                                      _vp, ctypes.c_size_t, _vp], _i32),
     "gsa_indexer_select_adaptive_workspace_bytes": ([_i32, _i32], ctypes.c_size_t),
     "gsa_debug_force_select_fallback": ([_i32], _i32),
+    "gsa_rope_qk": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp],
+                    _i32),
     "gsa_prologue": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i64,
                       _i32, _i32, _i32, _i32, _i32, _vp, _vp, _vp], _i32),
     "gsa_sparse_attn": ([_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64,
@@ -428,6 +431,23 @@ def prologue(k=None, v=None, vg=None, cos=None, sin=None, k_out=None, v_out=None
                           B, T, H, d, dtype_code(ref.dtype), _ptr(k_out), _ptr(v_out), _stream(ref))
     _check(st, "gsa_prologue")
     return k_out, v_out
+
+
+def rope_qk(q, k, cos, sin):
+    """RoPE of q and k (one shape, one dtype) in one launch -> (q_out, k_out), contiguous."""
+    lib = load()
+    _need_cuda(q, k, cos, sin)
+    B, T, H, d = q.shape
+    _expect(tuple(k.shape) == (B, T, H, d) and k.dtype == q.dtype, "k: q's shape and dtype")
+    _expect(cos.dim() == 2 and cos.shape[0] >= T and cos.shape[1] == d and tuple(sin.shape) == tuple(cos.shape)
+            and cos.dtype == sin.dtype == q.dtype and cos.stride(1) == 1 and sin.stride() == cos.stride(),
+            "cos/sin: [>=T, d] in q's dtype")
+    q_out = torch.empty(B, T, H, d, device=q.device, dtype=q.dtype)
+    k_out = torch.empty(B, T, H, d, device=q.device, dtype=q.dtype)
+    st = lib.gsa_rope_qk(_ptr(q), *_rows(q, H * d), _ptr(k), *_rows(k, H * d), _ptr(cos), _ptr(sin), cos.stride(0),
+                         B, T, H, d, dtype_code(q.dtype), _ptr(q_out), _ptr(k_out), _stream(q))
+    _check(st, "gsa_rope_qk")
+    return q_out, k_out
 
 
 def sparse_attn(q, k, v, idx, scale: float, count=None, mask=None, og=None, cos=None, sin=None,

@@ -55,6 +55,49 @@ __global__ __launch_bounds__(1024) void prologue_kernel(ProArgs p) {
 }
 
 // ---------------------------------------------------------------------------
+// RoPE of q and k in one launch (apply_rotary_pos_emb): grid.y picks the tensor,
+// kRopeRows rows a block with all their loads issued before the first use.
+// Bound by memory.  bf16 H = 16, the whole call, two launches of prologue_kernel
+// -> this: B = 2, T = 8192 (272 MB) 47.0 -> 43.8 us; T <= 2048, where the host
+// bounds both, 28 -> 18.  Rows a block, B = 2, T = 8192: 1 / 2 / 4 take 46.1 / 46.5 /
+// 43.8 us; B = 4, T = 8192, H = 32: 185 / 184 / 180 (two launches: 180).  Both
+// tensors in one block (the table read once) takes 189 there: two more streams in
+// flight cost more than the table, which the L2 holds.
+// ---------------------------------------------------------------------------
+constexpr int kRopeRows = 4;
+
+struct RopeArgs {
+  const void* in[2]; int64_t sb[2], st[2];
+  const void* cos; const void* sin; int64_t cs_st;
+  void* out[2];
+  int rows, T, HD;
+};
+
+template <typename T>
+__global__ __launch_bounds__(1024) void rope_qk_kernel(RopeArgs p) {
+  const int z = blockIdx.y;
+  const T* in = static_cast<const T*>(z ? p.in[1] : p.in[0]);
+  T* out = static_cast<T*>(z ? p.out[1] : p.out[0]);
+  const int64_t sb = z ? p.sb[1] : p.sb[0], st = z ? p.st[1] : p.st[0];
+  const int li = threadIdx.x & 15;
+  const int e0 = threadIdx.x * 8;   // == head*128 + li*8
+  float x[kRopeRows][8], c[kRopeRows][8], s[kRopeRows][8];
+#pragma unroll
+  for (int u = 0; u < kRopeRows; ++u) {
+    const int row = min((int)blockIdx.x * kRopeRows + u, p.rows - 1), b = row / p.T, t = row % p.T;
+    load8(in + b * sb + (int64_t)t * st + e0, x[u]);
+    load8(static_cast<const T*>(p.cos) + (int64_t)t * p.cs_st + li * 8, c[u]);
+    load8(static_cast<const T*>(p.sin) + (int64_t)t * p.cs_st + li * 8, s[u]);
+  }
+#pragma unroll
+  for (int u = 0; u < kRopeRows; ++u) {
+    const int row = (int)blockIdx.x * kRopeRows + u;
+    rope8<T>(x[u], c[u], s[u], li);
+    if (row < p.rows) store8(out + (int64_t)row * p.HD + e0, x[u]);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Sparse attention
 // ---------------------------------------------------------------------------
 struct AttnArgs {
@@ -271,6 +314,24 @@ extern "C" int gsa_prologue(const void* k, int64_t k_sb, int64_t k_st,
     hipLaunchKernelGGL(gsa::prologue_kernel<uint16_t>, dim3(B * T), dim3(16 * H), 0, s, a);
   else
     hipLaunchKernelGGL(gsa::prologue_kernel<float>, dim3(B * T), dim3(16 * H), 0, s, a);
+  return launch_status();
+}
+
+extern "C" int gsa_rope_qk(const void* q, int64_t q_sb, int64_t q_st, const void* k, int64_t k_sb, int64_t k_st,
+                           const void* cos, const void* sin, int64_t cs_st, int B, int T, int H, int d, int dtype,
+                           void* q_out, void* k_out, void* stream) {
+  if (!q || !k || !cos || !sin || !q_out || !k_out) return GSA_ERR_NULL;
+  if (dtype_size(dtype) == 0) return GSA_ERR_DTYPE;
+  if (B < 1 || T < 1 || d != 128 || H < 1 || H > 64) return GSA_ERR_SHAPE;
+  if ((int64_t)B * T > 0x7fffffffLL - gsa::kRopeRows) return GSA_ERR_SHAPE;
+  if (!vec_ok(q, q_sb, q_st, dtype) || !vec_ok(k, k_sb, k_st, dtype) || !vec_ok(cos, 0, cs_st, dtype) ||
+      !vec_ok(sin, 0, cs_st, dtype) || !aligned(q_out, 16) || !aligned(k_out, 16))
+    return GSA_ERR_ALIGN;
+  const gsa::RopeArgs a{{q, k}, {q_sb, k_sb}, {q_st, k_st}, cos, sin, cs_st, {q_out, k_out}, B * T, T, H * 128};
+  const dim3 grid((B * T + gsa::kRopeRows - 1) / gsa::kRopeRows, 2), block(16 * H);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (dtype == GSA_DTYPE_BF16) hipLaunchKernelGGL(gsa::rope_qk_kernel<uint16_t>, grid, block, 0, s, a);
+  else hipLaunchKernelGGL(gsa::rope_qk_kernel<float>, grid, block, 0, s, a);
   return launch_status();
 }
 

@@ -89,6 +89,8 @@ def apply_rotary_pos_emb(q: torch.Tensor, k: torch.Tensor, cos: torch.Tensor,
     c, s = _rope_table(cos, d), _rope_table(sin, d)
     q = q if q.stride(-1) == 1 else q.contiguous()
     k = k if k.stride(-1) == 1 else k.contiguous()
+    if q.shape == k.shape and q.dtype == k.dtype:
+        return _abi.rope_qk(q, k, c.to(q.dtype), s.to(q.dtype))
     q_out, _ = _abi.prologue(k=q, cos=c.to(q.dtype), sin=s.to(q.dtype))
     k_out, _ = _abi.prologue(k=k, cos=c.to(k.dtype), sin=s.to(k.dtype))
     return q_out, k_out

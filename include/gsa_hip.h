@@ -260,6 +260,16 @@ int gsa_prologue(const void* k, int64_t k_sb, int64_t k_st,
                  void* stream);
 
 /*
+ * RoPE of q and k [B,T,H,d] in one launch: apply_rotary_pos_emb
+ * (gsa_triton/gsa_opt.py:396-401), each rounded as gsa_prologue's k_out, into
+ * contiguous q_out and k_out.  cos, sin [T,d] (row stride cs_st) in dtype.
+ * Supported: d == 128, 1 <= H <= 64.
+ */
+int gsa_rope_qk(const void* q, int64_t q_sb, int64_t q_st, const void* k, int64_t k_sb, int64_t k_st,
+                const void* cos, const void* sin, int64_t cs_st, int B, int T, int H, int d, int dtype,
+                void* q_out, void* k_out, void* stream);
+
+/*
  * Sparse attention over per-row selected keys (gather, online softmax).
  * Replaces fused_sparse_attention (gsa_triton/gsa_opt.py:349-383) and its
  * kernel (gsa_opt.py:187-346); with GSA_ATTN_ROPE_Q it also applies RoPE to q

@@ -163,6 +163,25 @@ def test_apply_rotary_pos_emb(dev, dtype):
         assert torch.equal(oq.cpu(), rq) and torch.equal(ok.cpu(), rk)
 
 
+@pytest.mark.parametrize("B,T,H,dtype", [(1, 1, 1, torch.bfloat16), (1, 5, 3, torch.float32), (3, 1, 16, torch.bfloat16),
+                                         (2, 67, 64, torch.float32), (1, 258, 16, torch.bfloat16)])
+def test_apply_rotary_pos_emb_rows(dev, B, T, H, dtype):
+    """Row counts around the rows a block takes (4), one to 64 heads, q and k views
+    with strides of their own, in one launch (one shape) and in two (k with a head
+    more): bit-exact with the oracle."""
+    g = torch.Generator().manual_seed(T)
+    qkv = torch.randn(B, T + 1, 3, H, 128, generator=g).to(dtype)
+    q, k, k2 = qkv[:, :T, 0], qkv[:, 1:, 2], torch.randn(B, T, H % 64 + 1, 128, generator=g).to(dtype)
+    cos, sin = orc.RopeCache(128, dtype).tables(T, dtype)
+    ref = [orc.apply_rope(t, cos[None, :, None], sin[None, :, None]) for t in (q, k, k2)]
+    c, s, qd = cos.to(dev), sin.to(dev), qkv.to(dev)
+    oq, ok = G.apply_rotary_pos_emb(qd[:, :T, 0], qd[:, 1:, 2], c, s)
+    assert oq.is_contiguous() and ok.is_contiguous()
+    assert torch.equal(oq.cpu(), ref[0]) and torch.equal(ok.cpu(), ref[1])
+    oq, ok = G.apply_rotary_pos_emb(qd[:, :T, 0], k2.to(dev), c, s)
+    assert torch.equal(oq.cpu(), ref[0]) and torch.equal(ok.cpu(), ref[2])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_rotary_embedding_tables_on_device(dev, dtype):
     """RotaryEmbedding.forward(seq_len, device, dtype) after a module cast: the cached
