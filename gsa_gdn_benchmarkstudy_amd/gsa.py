@@ -367,13 +367,11 @@ class GatedSparseAttention(nn.Module):
         # the GEMM, on a side stream beside the RoPE/gate producer), "serial"
         # (everything on the current stream) or "auto": bf16 up to
         # SHORT_TOKENS tokens, one GEMM for all eight projections and one call
-        # for everything between it and o_proj (_forward_short); else "serial"
-        # while RoPE(k) and V^T together fit the 256 MB last-level cache (the
-        # producer then runs right before the attention, which finds them
-        # cached); else "producer".  Two streams cost two event pairs and gain
-        # little while the select fills the chip: us per forward, "gemm" /
-        # "serial", T=2048 274 / 184, B=2 T=3001 444 / 408, T=8192 781 / 751,
-        # T=4096 342 / 356.
+        # for everything between it and o_proj (_forward_short); else "gemm"
+        # where the GEMM's last round of tiles leaves most CUs idle
+        # (_gemm_leaves_room); else "serial" while RoPE(k) and V^T together fit
+        # the 256 MB last-level cache (the producer then runs right before the
+        # attention, which finds them cached); else "producer".
         self.indexer_overlap = "auto"
         # Main projection on the bf16 block-dense path: "gemm" (hipBLASLt GEMM,
         # then the RoPE / value-gate producer kernel) or "fused" (own MFMA GEMM
@@ -534,9 +532,25 @@ class GatedSparseAttention(nn.Module):
         return True
 
     # Tokens (B*T) up to which one GEMM over the whole fused weight is faster than
-    # the indexer's and the main one, bf16, D=2048, us: 512 30 against 51, 2048 96
-    # against 109, 4096 147 against 175, 6002 200 against 205, 7000 315 against 238.
-    SHORT_TOKENS = 6144
+    # the main one and the indexer's, bf16, D=2048, us: 512 30 against 51, 2048 96
+    # against 109, 4096 135 against 167, 5000 176 against 230; above it depends on
+    # the kernel the library takes: 5200 209 against 188, 5632 183 against 196, 5835
+    # 221 against 201, 7000 299 against 236.
+    SHORT_TOKENS = 5120
+
+    def _gemm_leaves_room(self, x: torch.Tensor) -> bool:
+        """Whether the select runs beside the main GEMM (bf16): while its own grid
+        leaves CUs free, and if the last round of the GEMM's 256x256 tiles fills less
+        than half of them.  us per forward beside the GEMM / before it, with that
+        share: B=2 T=4100 0.16 600 / 622, B=2 T=2600 0.28 366 / 376, T=7000 0.38 592 /
+        609, T=5400 0.44 469 / 480, T=8800 0.47 915 / 922; T=5835 0.59 502 / 502,
+        T=6144 0.75 556 / 524, T=9500 0.94 1044 / 1027, T=8192 1 781 / 751."""
+        B, T, D = x.shape
+        cus = torch.cuda.get_device_properties(x.device).multi_processor_count
+        if x.dtype != torch.bfloat16 or B * ((T + 15) // 16) >= 4 * cus:
+            return False
+        tiles = ((B * T + 255) // 256) * ((5 * D + 255) // 256)
+        return 2 * (-tiles % cus) > cus
 
     def _short(self, x: torch.Tensor) -> bool:
         """Whether forward takes _forward_short (bf16, block-dense attention, one stream)."""
@@ -611,7 +625,10 @@ class GatedSparseAttention(nn.Module):
         # that size the producer is better hidden beside the indexer.
         mode = self.indexer_overlap
         if mode == "auto":
-            mode = "serial" if 2 * B * T * D * x.element_size() <= _LLC_BYTES else "producer"
+            if self._gemm_leaves_room(x):
+                mode = "gemm"
+            else:
+                mode = "serial" if 2 * B * T * D * x.element_size() <= _LLC_BYTES else "producer"
         elif mode not in ("producer", "gemm", "serial"):
             raise ValueError(f"indexer_overlap {mode!r}: expected 'auto', 'producer', 'gemm' or 'serial'")
         _range_push("gsa_hip/indexer_gemm")
