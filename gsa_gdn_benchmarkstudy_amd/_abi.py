@@ -765,7 +765,7 @@ def dense_lane_masks(bits, Tkv: int, ws: Optional[torch.Tensor] = None, causal: 
     ``causal``: only the tiles a causal dense_attn reads, up to the last row of each
     query block (such masks serve causal calls only); otherwise every tile.
     ``split_heads``: the attention's number of heads when it is to be called with
-    split=True (its workspace, counters cleared, is then part of ``ws``)."""
+    split=True (its workspace is then part of ``ws``)."""
     lib = load()
     _need_cuda(bits, ws)
     B, T, W = bits.shape
@@ -785,7 +785,7 @@ def dense_attn(q, k, vt, bits, scale: float, og=None, cos=None, sin=None, flags:
     workspace (uint8 device tensor of at least dense_attn_workspace_bytes);
     ``masks_ready``: ws already holds dense_lane_masks(bits) (bits is then not read).
     ``split``: long query blocks in parts, where dense_attn_split_bytes is not 0 (with
-    masks_ready: the masks built with split_heads=H, for one call)."""
+    masks_ready: ws with room for it, as built with split_heads=H)."""
     lib = load()
     _need_cuda(q, k, vt, bits, og, cos, sin)
     B, T, H, d = q.shape

@@ -20,6 +20,7 @@
 // 32x32 block: head dims of O^T; the rows of S^T are keys in the permuted
 // order described at the dense kernel.
 #include "gsa_common.h"
+#include "layer_steps.h"
 
 #include <cmath>
 #include <type_traits>
@@ -1029,17 +1030,17 @@ int launch_units(gsa::DenseArgs& a, const gsa::UnitPlan& plan, void* area, const
 }
 }  // namespace
 
-extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
-                              const void* k, int64_t k_sb, int64_t k_st,
-                              const void* vt, int64_t vt_sb, int64_t vt_sh, int ldv,
-                              const uint32_t* bits, int64_t b_sb, int64_t b_st,
-                              const void* og, int64_t o_sb, int64_t o_st,
-                              const void* cos, const void* sin, int64_t cs_st,
-                              void* out, int64_t out_sb, int64_t out_st,
-                              int B, int T, int Tkv, int H, int d, float scale,
-                              int dtype, int flags, int causal,
-                              void* ws, size_t ws_bytes,
-                              void* stream) {
+int gsa_host::dense_attn(const void* q, int64_t q_sb, int64_t q_st,
+                         const void* k, int64_t k_sb, int64_t k_st,
+                         const void* vt, int64_t vt_sb, int64_t vt_sh, int ldv,
+                         const uint32_t* bits, int64_t b_sb, int64_t b_st,
+                         const void* og, int64_t o_sb, int64_t o_st,
+                         const void* cos, const void* sin, int64_t cs_st,
+                         void* out, int64_t out_sb, int64_t out_st,
+                         int B, int T, int Tkv, int H, int d, float scale,
+                         int dtype, int flags, int causal,
+                         void* ws, size_t ws_bytes, bool cleared,
+                         void* stream) {
   const bool ready = (flags & GSA_ATTN_MASKS_READY) != 0;
   if (!q || !k || !vt || !out || !ws || (!ready && !bits)) return GSA_ERR_NULL;
   if (flags & ~(GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE | GSA_ATTN_MASKS_READY | GSA_ATTN_ROPE_HALVES | GSA_ATTN_SPLIT))
@@ -1054,7 +1055,7 @@ extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
   if (ldv < NT * 64 || ldv % 64 != 0) return GSA_ERR_SHAPE;
   if (ws_bytes < gsa_dense_attn_workspace_bytes(B, T, Tkv)) return GSA_ERR_SHAPE;
   const bool split = (flags & GSA_ATTN_SPLIT) != 0;
-  gsa::UnitPlan plan;
+  gsa::UnitPlan plan{};
   if (split) {
     plan = bf16_plan(B, T, Tkv, H, causal != 0);
     if (plan.n == 0 || ws_bytes < gsa_dense_attn_workspace_bytes(B, T, Tkv) + split_bytes(plan, B, T, H))
@@ -1085,6 +1086,11 @@ extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
   if (!ready) {
     const int st = launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes, s);
     if (st) return st;
+  } else if (plan.slots && !cleared) {      // ready masks say nothing of the counters behind them
+    const int st = launch_clear(
+        reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + gsa_dense_attn_workspace_bytes(B, T, Tkv)),
+        counter_words(B, T), s);
+    if (st) return st;
   }
   flags &= ~(GSA_ATTN_MASKS_READY | GSA_ATTN_SPLIT);
   gsa::DenseArgs a{static_cast<const uint16_t*>(q), q_sb, q_st, static_cast<const uint16_t*>(k), k_sb, k_st,
@@ -1099,6 +1105,22 @@ extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
   hipLaunchKernelGGL((gsa::dense_attn_kernel<false, false>), dim3(B * H * nqb), dim3(64 * W), gsa::kDenseLds, s, a, lm,
                      gsa::NoPlan{});
   return launch_status();
+}
+
+extern "C" int gsa_dense_attn(const void* q, int64_t q_sb, int64_t q_st,
+                              const void* k, int64_t k_sb, int64_t k_st,
+                              const void* vt, int64_t vt_sb, int64_t vt_sh, int ldv,
+                              const uint32_t* bits, int64_t b_sb, int64_t b_st,
+                              const void* og, int64_t o_sb, int64_t o_st,
+                              const void* cos, const void* sin, int64_t cs_st,
+                              void* out, int64_t out_sb, int64_t out_st,
+                              int B, int T, int Tkv, int H, int d, float scale,
+                              int dtype, int flags, int causal,
+                              void* ws, size_t ws_bytes,
+                              void* stream) {
+  return dense_attn(q, q_sb, q_st, k, k_sb, k_st, vt, vt_sb, vt_sh, ldv, bits, b_sb, b_st, og, o_sb, o_st, cos, sin,
+                    cs_st, out, out_sb, out_st, B, T, Tkv, H, d, scale, dtype, flags, causal, ws, ws_bytes, false,
+                    stream);
 }
 
 extern "C" size_t gsa_dense_attn_split_bytes(int B, int T, int Tkv, int H, int causal) {

@@ -295,6 +295,11 @@ size_t counter_bytes(int B, int T, int H) {
 
 }  // namespace
 
+int gsa_host::launch_clear(uint32_t* p, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(clear_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, p, n);
+  return launch_status();
+}
+
 size_t gsa_host::dense_f32_bytes(int B, int T, int Tkv, int H) {
   const gsa::UnitPlan plan = f32_plan(B, T, Tkv, H);
   if (!plan.n) return 0;
@@ -318,9 +323,7 @@ int gsa_host::launch_dense_f32(const AttnShape& s, const gsa::Selection& sel, vo
   uint32_t* counters = static_cast<uint32_t*>(ws);
   float* parts = reinterpret_cast<float*>(static_cast<char*>(ws) + counter_bytes(s.B, s.T, s.H));
   if (plan.n) {
-    const int n = s.B * s.H * nqb;
-    hipLaunchKernelGGL(clear_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, counters, n);
-    const int st = launch_status();
+    const int st = launch_clear(counters, s.B * s.H * nqb, stream);
     if (st) return st;
   }
   const gsa::DenseF32Args a{

@@ -365,6 +365,9 @@ inline int launch_status() {
 int launch_adaptive_k(const float* var, int n, int k_base, int k_min, int k_max, int k_cap, int32_t* k_rows,
                       hipStream_t stream);
 
+// Zeroes n words (a kernel, so that a graph may record it; dense_attn_f32.hip).
+int launch_clear(uint32_t* p, int n, hipStream_t stream);
+
 // Attention over a selection of Tkv keys per row: q, out [B,T,H,128], k, v
 // [B,Tkv,H,128], innermost dimensions contiguous, 16-byte aligned rows.
 struct AttnShape {

@@ -5,6 +5,7 @@
 // tensor views and an event pair per step, a forward of 512 tokens took 260 us
 // of which the GPU worked 91.  The steps' own entry points do the checks.
 #include "../../include/gsa_hip.h"
+#include "layer_steps.h"
 
 namespace {
 
@@ -70,8 +71,9 @@ extern "C" int gsa_layer_attn(const void* proj, int64_t p_sb, int64_t p_st, cons
   if (st) return st;
   const int64_t hd = (int64_t)H * d;
   const int split = gsa_dense_attn_split_bytes(B, T, T, H, 1) ? GSA_ATTN_SPLIT : 0;
-  return gsa_dense_attn(q, p_sb, p_st, k_rope, T * hd, hd, vt, hd * ldv, (int64_t)d * ldv, ldv, bits, b_sb, W, og, p_sb,
-                        p_st, halves, nullptr, h_st, out, out_sb, out_st, B, T, T, H, d, scale, GSA_DTYPE_BF16,
-                        GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE | GSA_ATTN_ROPE_HALVES | GSA_ATTN_MASKS_READY | split, 1,
-                        base + at.masks, mask_bytes, stream);
+  return gsa_host::dense_attn(
+      q, p_sb, p_st, k_rope, T * hd, hd, vt, hd * ldv, (int64_t)d * ldv, ldv, bits, b_sb, W, og, p_sb, p_st, halves,
+      nullptr, h_st, out, out_sb, out_st, B, T, T, H, d, scale, GSA_DTYPE_BF16,
+      GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE | GSA_ATTN_ROPE_HALVES | GSA_ATTN_MASKS_READY | split, 1, base + at.masks,
+      mask_bytes, true, stream);
 }

@@ -405,11 +405,9 @@ size_t gsa_dense_attn_workspace_bytes(int B, int T, int Tkv);
  * length, the long ones are split along their keys and their parts added in a
  * fixed order (other sums than without the flag, same accuracy, the same bits on
  * each call).  It takes gsa_dense_attn_split_bytes more workspace behind the
- * masks -- 0 where a split does not pay; the flag is then GSA_ERR_SHAPE.  The
- * call that writes the masks (gsa_dense_lane_masks, gsa_prologue_vt_lane_masks,
- * or gsa_dense_attn itself) clears the counters there, if its ws_bytes covers
- * them: with GSA_ATTN_MASKS_READY that call has to have had the same ws_bytes, and
- * each GSA_ATTN_SPLIT call needs such a call before it.
+ * masks -- 0 where a split does not pay; the flag is then GSA_ERR_SHAPE.  Each
+ * call clears its counters there itself, with ready masks by one launch more, so
+ * masks serve any number of calls, split or not.
  */
 size_t gsa_dense_attn_split_bytes(int B, int T, int Tkv, int H, int causal);
 

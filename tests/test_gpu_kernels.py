@@ -783,6 +783,29 @@ def test_dense_attention_split_blocks(dev, B, T, Tkv, H, causal):
     assert torch.all(a[:, 5] == 0)
 
 
+@pytest.mark.parametrize("built_for_split", [True, False])
+def test_dense_attention_split_reuses_masks(dev, built_for_split):
+    """Ready masks serve several split calls, also in a workspace whose words behind the
+    masks hold anything: every call writes every row, with the same bits."""
+    B, T, H = 1, 1537, 16
+    _log(f"split dense on ready masks, built for split: {built_for_split}")
+    g = torch.Generator().manual_seed(1)
+    q, k = (torch.randn(B, T, H, 128, generator=g).to(torch.bfloat16).to(dev) for _ in range(2))
+    vt = torch.zeros(B, H, 128, _abi.vt_len(T), dtype=torch.bfloat16, device=dev)
+    vt[..., :T] = torch.randn(B, H, 128, T, generator=g).to(torch.bfloat16)
+    words = torch.randint(-2 ** 31, 2 ** 31, (B, T, _abi.mask_words(T)), generator=g, dtype=torch.int64)
+    idx = torch.where(torch.ones(T, T, dtype=torch.bool).tril(), torch.arange(T)[None], 0)[None].int()
+    bits = words.int().to(dev) & _abi.selection_mask(idx.to(dev), T)        # random keys of 0 .. t
+    want = _abi.dense_attn(q, k, vt, bits, 128 ** -0.5, split=True)
+    n = int(_abi.load().gsa_dense_attn_workspace_bytes(B, T, T))
+    ws = torch.full((n + _abi.dense_attn_split_bytes(B, T, T, H),), 0xab, device=dev, dtype=torch.uint8)
+    _abi.dense_lane_masks(bits, T, ws=ws, causal=True, split_heads=H if built_for_split else 0)
+    for _ in range(3):
+        out = torch.full_like(q, float("nan"))
+        _abi.dense_attn(q, k, vt, bits, 128 ** -0.5, out=out, ws=ws, masks_ready=True, split=True)
+        assert torch.equal(out, want)
+
+
 def test_dense_attention_split_refused_where_it_does_not_pay(dev):
     """No plan, no split: GSA_ERR_SHAPE, as for a workspace without its area."""
     assert _abi.dense_attn_split_bytes(1, 16384, 16384, 16) == 0 and _abi.dense_attn_split_bytes(1, 2048, 2048, 65) == 0
