@@ -937,23 +937,24 @@ int lane_mask_checks(const uint32_t* bits, int64_t b_sb, int64_t b_st, int B, in
 
 // The arrival counters behind the mask operands (room for 64 heads).
 int counter_words(int B, int T) { return B * 64 * (int)(dense_groups(T, 0) / gsa::kDenseWaves); }
+uint32_t* counters_of(void* ws, int B, int T, int Tkv) {
+  return reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + gsa_dense_attn_workspace_bytes(B, T, Tkv));
+}
 
+// clear: the counters too (the workspace of a GSA_ATTN_SPLIT call alone has them).
 gsa::LaneMaskArgs lane_mask_args(const uint32_t* bits, int64_t b_sb, int64_t b_st, int B, int T, int Tkv,
-                                  int causal, void* ws, size_t ws_bytes) {
+                                  int causal, void* ws, bool clear) {
   const int NT = (Tkv + 63) / 64;
   const int G = (int)dense_groups(T, Tkv);
   const int nunits = B * G * ((NT + gsa::kLmTiles - 1) / gsa::kLmTiles);
   const int block_rows = causal ? 32 * gsa::kDenseWaves : 0;
-  // a workspace with room for them gets its arrival counters cleared
-  const size_t base = gsa_dense_attn_workspace_bytes(B, T, Tkv);
-  const int nclear = ws_bytes >= base + (size_t)counter_words(B, T) * 4 ? counter_words(B, T) : 0;
   return gsa::LaneMaskArgs{bits, b_sb, b_st, T, G, NT, nunits, block_rows, static_cast<gsa::u32x4*>(ws), nullptr,
-                           reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + base), nclear};
+                           counters_of(ws, B, T, Tkv), clear ? counter_words(B, T) : 0};
 }
 
 int launch_lane_masks(const uint32_t* bits, int64_t b_sb, int64_t b_st, int B, int T, int Tkv, int causal,
-                      void* ws, size_t ws_bytes, hipStream_t s) {
-  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes);
+                      void* ws, bool clear, hipStream_t s) {
+  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws, clear);
   hipLaunchKernelGGL(gsa::lane_mask_kernel, dim3((l.nunits + 7) / 8), dim3(256), 0, s, l);
   return launch_status();
 }
@@ -963,7 +964,31 @@ extern "C" int gsa_dense_lane_masks(const uint32_t* bits, int64_t b_sb, int64_t 
                                     int causal, void* ws, size_t ws_bytes, void* stream) {
   const int st = lane_mask_checks(bits, b_sb, b_st, B, T, Tkv, ws, ws_bytes);
   if (st) return st;
-  return launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes, static_cast<hipStream_t>(stream));
+  return launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, false, static_cast<hipStream_t>(stream));
+}
+
+int gsa_host::prologue_vt_lane_masks(const void* k, int64_t k_sb, int64_t k_st,
+                                     const void* v, int64_t v_sb, int64_t v_st,
+                                     const void* vg, int64_t g_sb, int64_t g_st,
+                                     const void* cos, const void* sin, int64_t cs_st,
+                                     int B, int T, int H, int d, int dtype,
+                                     void* k_out, void* vt, int ldv,
+                                     const uint32_t* bits, int64_t b_sb, int64_t b_st, int Tkv,
+                                     int causal, void* ws, size_t ws_bytes, bool clear, void* stream) {
+  int st = prologue_vt_checks(k, k_sb, k_st, v, v_sb, v_st, vg, g_sb, g_st, cos, sin, cs_st, B, T, H, d, dtype,
+                              k_out, vt, ldv);
+  if (st) return st;
+  if ((st = lane_mask_checks(bits, b_sb, b_st, B, T, Tkv, ws, ws_bytes))) return st;
+  gsa::ProVtArgs a{static_cast<const uint16_t*>(k), k_sb, k_st, static_cast<const uint16_t*>(v), v_sb, v_st,
+                   static_cast<const uint16_t*>(vg), g_sb, g_st, static_cast<const uint16_t*>(cos),
+                   static_cast<const uint16_t*>(sin), cs_st, static_cast<uint16_t*>(k_out),
+                   static_cast<uint16_t*>(vt), T, H, ldv, ldv / 64};
+  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws, clear);
+  const int n_pro = B * H * (ldv / 64), n_lm = (l.nunits + 7) / 8;
+  if ((int64_t)n_pro + n_lm > 0x7fffffffLL) return GSA_ERR_SHAPE;
+  hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel<false>, dim3(n_pro + n_lm), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), a, l, n_pro, n_lm);
+  return launch_status();
 }
 
 extern "C" int gsa_prologue_vt_lane_masks(const void* k, int64_t k_sb, int64_t k_st,
@@ -974,20 +999,8 @@ extern "C" int gsa_prologue_vt_lane_masks(const void* k, int64_t k_sb, int64_t k
                                           void* k_out, void* vt, int ldv,
                                           const uint32_t* bits, int64_t b_sb, int64_t b_st, int Tkv,
                                           int causal, void* ws, size_t ws_bytes, void* stream) {
-  int st = prologue_vt_checks(k, k_sb, k_st, v, v_sb, v_st, vg, g_sb, g_st, cos, sin, cs_st, B, T, H, d, dtype,
-                              k_out, vt, ldv);
-  if (st) return st;
-  if ((st = lane_mask_checks(bits, b_sb, b_st, B, T, Tkv, ws, ws_bytes))) return st;
-  gsa::ProVtArgs a{static_cast<const uint16_t*>(k), k_sb, k_st, static_cast<const uint16_t*>(v), v_sb, v_st,
-                   static_cast<const uint16_t*>(vg), g_sb, g_st, static_cast<const uint16_t*>(cos),
-                   static_cast<const uint16_t*>(sin), cs_st, static_cast<uint16_t*>(k_out),
-                   static_cast<uint16_t*>(vt), T, H, ldv, ldv / 64};
-  const gsa::LaneMaskArgs l = lane_mask_args(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes);
-  const int n_pro = B * H * (ldv / 64), n_lm = (l.nunits + 7) / 8;
-  if ((int64_t)n_pro + n_lm > 0x7fffffffLL) return GSA_ERR_SHAPE;
-  hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel<false>, dim3(n_pro + n_lm), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), a, l, n_pro, n_lm);
-  return launch_status();
+  return prologue_vt_lane_masks(k, k_sb, k_st, v, v_sb, v_st, vg, g_sb, g_st, cos, sin, cs_st, B, T, H, d, dtype, k_out,
+                                vt, ldv, bits, b_sb, b_st, Tkv, causal, ws, ws_bytes, false, stream);
 }
 
 namespace {
@@ -1019,10 +1032,10 @@ size_t split_bytes(const gsa::UnitPlan& plan, int B, int T, int H) {
 
 // The units of a plan; `area`: split_bytes, its counters cleared.
 template <bool kSel>
-int launch_units(gsa::DenseArgs& a, const gsa::UnitPlan& plan, void* area, const gsa::u32x4* lm, hipStream_t s) {
+int launch_units(gsa::DenseArgs& a, const gsa::UnitPlan& plan, uint32_t* area, const gsa::u32x4* lm, hipStream_t s) {
   const int st = dense_lds_limit<kSel, true>();
   if (st) return st;
-  a.counters = static_cast<uint32_t*>(area);
+  a.counters = area;
   a.parts = reinterpret_cast<float*>(a.counters + counter_words(a.B, a.T));
   hipLaunchKernelGGL((gsa::dense_attn_kernel<kSel, true>), dim3(a.B * a.H * plan.n), dim3(64 * gsa::kDenseWaves),
                      gsa::kDenseLds, s, a, lm, plan);
@@ -1084,12 +1097,10 @@ int gsa_host::dense_attn(const void* q, int64_t q_sb, int64_t q_st,
   hipStream_t s = static_cast<hipStream_t>(stream);
   const gsa::u32x4* lm = static_cast<const gsa::u32x4*>(ws);
   if (!ready) {
-    const int st = launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, ws_bytes, s);
+    const int st = launch_lane_masks(bits, b_sb, b_st, B, T, Tkv, causal, ws, plan.slots > 0, s);
     if (st) return st;
   } else if (plan.slots && !cleared) {      // ready masks say nothing of the counters behind them
-    const int st = launch_clear(
-        reinterpret_cast<uint32_t*>(static_cast<char*>(ws) + gsa_dense_attn_workspace_bytes(B, T, Tkv)),
-        counter_words(B, T), s);
+    const int st = launch_clear(counters_of(ws, B, T, Tkv), counter_words(B, T), s);
     if (st) return st;
   }
   flags &= ~(GSA_ATTN_MASKS_READY | GSA_ATTN_SPLIT);
@@ -1099,7 +1110,7 @@ int gsa_host::dense_attn(const void* q, int64_t q_sb, int64_t q_st,
                    static_cast<const uint16_t*>(sin), cs_st, static_cast<uint16_t*>(out), out_sb, out_st,
                    B, T, Tkv, H, nqb, scale * gsa::kLog2e, flags | (causal ? gsa::kDenseCausal : 0), nullptr, nullptr,
                    nullptr, nullptr};
-  if (split) return launch_units<false>(a, plan, static_cast<char*>(ws) + gsa_dense_attn_workspace_bytes(B, T, Tkv), lm, s);
+  if (split) return launch_units<false>(a, plan, counters_of(ws, B, T, Tkv), lm, s);
   const int st = dense_lds_limit<false, false>();
   if (st) return st;
   hipLaunchKernelGGL((gsa::dense_attn_kernel<false, false>), dim3(B * H * nqb), dim3(64 * W), gsa::kDenseLds, s, a, lm,
@@ -1146,12 +1157,11 @@ int gsa_host::launch_dense_selected(const AttnShape& s, const gsa::Selection& se
   uint16_t* vt = static_cast<uint16_t*>(ws);
   void* lm = static_cast<char*>(ws) + selected_vt_bytes(s.B, s.Tkv, s.H);
   const gsa::UnitPlan plan = bf16_plan(s.B, s.T, s.Tkv, s.H, s.T == s.Tkv);
-  const size_t lm_bytes = gsa_dense_attn_workspace_bytes(s.B, s.T, s.Tkv);
   gsa::ProVtArgs p{};
   p.v = static_cast<const uint16_t*>(s.v); p.v_sb = s.v_sb; p.v_st = s.v_st;
   p.vt = vt; p.T = s.Tkv; p.H = s.H; p.ldv = ldv; p.ntiles = NT;
   gsa::LaneMaskArgs l = lane_mask_args(sel.bits, (int64_t)s.T * 2 * NT, 2 * NT, s.B, s.T, s.Tkv, 0, lm,
-                                       plan.n ? lm_bytes + split_bytes(plan, s.B, s.T, s.H) : lm_bytes);
+                                       plan.slots > 0);
   l.range = sel.range;
   const int n_pro = s.B * s.H * NT, n_lm = (l.nunits + 7) / 8;
   hipLaunchKernelGGL(gsa::prologue_vt_lane_mask_kernel<true>, dim3(n_pro + n_lm), dim3(256), 0, stream, p, l, n_pro,
@@ -1168,7 +1178,7 @@ int gsa_host::launch_dense_selected(const AttnShape& s, const gsa::Selection& se
   a.scale_l2 = s.scale * gsa::kLog2e;
   a.range = sel.range; a.redo = sel.redo;
   const gsa::u32x4* masks = static_cast<const gsa::u32x4*>(lm);
-  if (plan.n) return launch_units<true>(a, plan, static_cast<char*>(lm) + lm_bytes, masks, stream);
+  if (plan.n) return launch_units<true>(a, plan, counters_of(lm, s.B, s.T, s.Tkv), masks, stream);
   if ((st = dense_lds_limit<true, false>())) return st;
   hipLaunchKernelGGL((gsa::dense_attn_kernel<true, false>), dim3(s.B * s.H * nqb), dim3(64 * gsa::kDenseWaves),
                      gsa::kDenseLds, stream, a, masks, gsa::NoPlan{});

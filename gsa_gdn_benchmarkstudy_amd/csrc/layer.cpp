@@ -65,15 +65,16 @@ extern "C" int gsa_layer_attn(const void* proj, int64_t p_sb, int64_t p_st, cons
   void* k_rope = base + at.k_rope;
   void* vt = base + at.vt;
   const size_t mask_bytes = at.total - at.masks;
-  st = gsa_prologue_vt_lane_masks(k, p_sb, p_st, v, p_sb, p_st, vg, p_sb, p_st, cos, sin, cs_st, B, T, H, d,
-                                  GSA_DTYPE_BF16, k_rope, vt, ldv, bits, b_sb, W, T, 1, base + at.masks, mask_bytes,
-                                  stream);
+  const bool split = gsa_dense_attn_split_bytes(B, T, T, H, 1) != 0;
+  st = gsa_host::prologue_vt_lane_masks(k, p_sb, p_st, v, p_sb, p_st, vg, p_sb, p_st, cos, sin, cs_st, B, T, H, d,
+                                        GSA_DTYPE_BF16, k_rope, vt, ldv, bits, b_sb, W, T, 1, base + at.masks,
+                                        mask_bytes, split, stream);
   if (st) return st;
   const int64_t hd = (int64_t)H * d;
-  const int split = gsa_dense_attn_split_bytes(B, T, T, H, 1) ? GSA_ATTN_SPLIT : 0;
   return gsa_host::dense_attn(
       q, p_sb, p_st, k_rope, T * hd, hd, vt, hd * ldv, (int64_t)d * ldv, ldv, bits, b_sb, W, og, p_sb, p_st, halves,
       nullptr, h_st, out, out_sb, out_st, B, T, T, H, d, scale, GSA_DTYPE_BF16,
-      GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE | GSA_ATTN_ROPE_HALVES | GSA_ATTN_MASKS_READY | split, 1, base + at.masks,
-      mask_bytes, true, stream);
+      GSA_ATTN_ROPE_Q | GSA_ATTN_OUT_GATE | GSA_ATTN_ROPE_HALVES | GSA_ATTN_MASKS_READY |
+          (split ? GSA_ATTN_SPLIT : 0),
+      1, base + at.masks, mask_bytes, true, stream);
 }

@@ -419,7 +419,8 @@ size_t gsa_dense_attn_split_bytes(int B, int T, int Tkv, int H, int causal);
  * on another stream, beside other work, and pass GSA_ATTN_MASKS_READY.
  * causal != 0: only the key tiles a causal gsa_dense_attn reads (up to the
  * last row of each query block) are built; such masks serve causal calls
- * only.  causal == 0: every tile (serves both).
+ * only.  causal == 0: every tile (serves both).  Nothing past
+ * gsa_dense_attn_workspace_bytes is written, whatever ws_bytes is.
  * No counterpart in the reference: part of this library's dense attention.
  */
 int gsa_dense_lane_masks(const uint32_t* bits, int64_t b_sb, int64_t b_st,

@@ -806,6 +806,28 @@ def test_dense_attention_split_reuses_masks(dev, built_for_split):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("call", ["lane_masks", "prologue_vt", "dense_attn"])
+def test_dense_workspace_past_the_masks_is_left_alone(dev, monkeypatch, call):
+    """A caller's whole arena as the workspace (ws_bytes larger than needed, enough for split
+    counters): without GSA_ATTN_SPLIT nothing behind the masks is written."""
+    B, T, H = 2, 700, 4
+    q = torch.zeros(B, T, H, 128, dtype=torch.bfloat16, device=dev)
+    vt = torch.zeros(B, H, 128, _abi.vt_len(T), dtype=torch.bfloat16, device=dev)
+    tab = torch.zeros(T, 128, dtype=torch.bfloat16, device=dev)
+    bits = torch.zeros(B, T, _abi.mask_words(T), dtype=torch.int32, device=dev)
+    n = int(_abi.load().gsa_dense_attn_workspace_bytes(B, T, T))
+    assert _abi.dense_attn_split_bytes(B, T, T, H) > 0
+    ws = torch.full((n + (8 << 20),), 0x5a, device=dev, dtype=torch.uint8)
+    monkeypatch.setattr(_abi, "_mask_workspace", lambda *a: (ws, ws.numel()))
+    if call == "lane_masks":
+        _abi.dense_lane_masks(bits, T, ws=ws, causal=True)
+    elif call == "prologue_vt":
+        _abi.prologue_vt(q, q, k=q, cos=tab, sin=tab, bits=bits, Tkv=T, ws=ws, causal=True)
+    else:
+        _abi.dense_attn(q, q, vt, bits, 0.1, ws=ws)
+    assert torch.all(ws[n:] == 0x5a) and not torch.all(ws[:n] == 0x5a)
+
+
 def test_dense_attention_split_refused_where_it_does_not_pay(dev):
     """No plan, no split: GSA_ERR_SHAPE, as for a workspace without its area."""
     assert _abi.dense_attn_split_bytes(1, 16384, 16384, 16) == 0 and _abi.dense_attn_split_bytes(1, 2048, 2048, 65) == 0
