@@ -545,9 +545,10 @@ def selected_attn(q, k, v, idx, scale: float, mask=None) -> torch.Tensor:
     return out
 
 
-def masked_attn_serves(B: int, T: int, H: int, k_sel: int, dtype: torch.dtype) -> bool:
-    """Whether masked_attn is the faster way at these sizes (fp32; the library's rule)."""
-    return load().gsa_masked_attn_workspace_bytes(B, T, H, k_sel, dtype_code(dtype)) > 0
+def masked_attn_serves(B: int, T: int, H: int, k_sel: int, dtype: torch.dtype, scale: float = 1.0) -> bool:
+    """Whether masked_attn takes the call and is the faster way at these sizes (fp32,
+    scale > 0; the library's rule)."""
+    return scale > 0 and load().gsa_masked_attn_workspace_bytes(B, T, H, k_sel, dtype_code(dtype)) > 0
 
 
 def masked_attn(q, k, v, bits, k_sel: int, scale: float, og=None, cos=None, sin=None, flags: int = 0) -> torch.Tensor:

@@ -604,7 +604,8 @@ class GatedSparseAttention(nn.Module):
 
         dense = self.uses_dense(x.dtype)
         k_sel = self.topk_selector.k_effective(T)
-        masked = self.attn_impl == "auto" and not dense and _abi.masked_attn_serves(B, T, self.num_heads, k_sel, x.dtype)
+        masked = (self.attn_impl == "auto" and not dense
+                  and _abi.masked_attn_serves(B, T, self.num_heads, k_sel, x.dtype, self.scale))
         fused_proj = self.uses_fused_projection(x)
         cos, sin = self.rotary_emb(T, dev, x.dtype)
         cos, sin = cos.contiguous(), sin.contiguous()

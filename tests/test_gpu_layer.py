@@ -346,3 +346,20 @@ def test_long_sequence_select_route_equals_fused(dev, impl, mode):
         routed = m(x)
     torch.cuda.synchronize()
     assert torch.equal(routed, fused)
+
+
+@pytest.mark.parametrize("scale", [-0.05, 0.0, float("nan")])
+def test_fp32_layer_scales_for_the_gather(dev, scale):
+    """A score scale that is not positive: the fp32 layer takes the gather kernel, same bits."""
+    _log(f"layer fp32 scale={scale}")
+    cfg = orc.GSAConfig(hidden_size=512, num_heads=4, k_max=128, k_base=128, k_min=16)
+    sd = orc.synthetic_state(cfg, seed=0)
+    x = orc.synthetic_input(1, 300, cfg.hidden_size, seed=1).to(dev)
+    out = []
+    for impl in ("auto", "gather"):
+        m = _model(cfg, sd, dev, torch.float32, impl)
+        assert m.scale > 0
+        m.scale = scale
+        with torch.no_grad():
+            out.append(m(x))
+    assert torch.equal(out[0].nan_to_num(7.0), out[1].nan_to_num(7.0))
