@@ -366,7 +366,7 @@ class GatedSparseAttention(nn.Module):
         # GEMM: "gemm" (on a side stream beside the GEMM), "producer" (after
         # the GEMM, on a side stream beside the RoPE/gate producer), "serial"
         # (everything on the current stream) or "auto": bf16 up to
-        # SHORT_TOKENS tokens, one GEMM for all eight projections and one call
+        # SHORT_TOKENS tokens (fewer where D > 2048), one GEMM for all eight projections and one call
         # for everything between it and o_proj (_forward_short); else "gemm"
         # where the GEMM's last round of tiles leaves most CUs idle
         # (_gemm_leaves_room); else "serial" while RoPE(k) and V^T together fit
@@ -538,6 +538,16 @@ class GatedSparseAttention(nn.Module):
     # 221 against 201, 7000 299 against 236.
     SHORT_TOKENS = 5120
 
+    @classmethod
+    def _short_limit(cls, D: int) -> int:
+        """Tokens up to which a layer of width D takes _forward_short.  A layer wider than
+        2048 is bound by the GPU sooner, and the one GEMM's extra columns can then cost
+        more than the launches: us per forward with one GEMM / step by step, D=3072 2048
+        tokens 0.9 of the time, 2560 462 / 371; D=4096 2048 530 / 563, 4096 919 / 824; D=5120
+        1500 533 / 559, 2048 738 / 715; D=6144 1280 670 / 707; D=8192 1024 756 / 905, 1280
+        989 / 941."""
+        return cls.SHORT_TOKENS if D <= 2048 else min(2048, (1 << 23) // D)
+
     def _gemm_leaves_room(self, x: torch.Tensor) -> bool:
         """Whether the select runs beside the main GEMM (bf16): while its own grid
         leaves CUs free, and if the last round of the GEMM's 256x256 tiles fills less
@@ -554,8 +564,8 @@ class GatedSparseAttention(nn.Module):
 
     def _short(self, x: torch.Tensor) -> bool:
         """Whether forward takes _forward_short (bf16, block-dense attention, one stream)."""
-        B, T, _ = x.shape
-        return (0 < B * T <= self.SHORT_TOKENS and x.dtype == torch.bfloat16 and self.indexer_overlap == "auto"
+        B, T, D = x.shape
+        return (0 < B * T <= self._short_limit(D) and x.dtype == torch.bfloat16 and self.indexer_overlap == "auto"
                 and self.attn_impl in ("auto", "dense") and self.proj_impl == "gemm" and self.attn_events is None
                 and self.lane_masks_with_producer and T <= self.FUSED_SELECT_MAX_T)
 

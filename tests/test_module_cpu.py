@@ -105,3 +105,16 @@ def test_selector_modes():
     s.mode = "median"
     with pytest.raises(ValueError):
         s.k_effective(10)
+
+
+@pytest.mark.parametrize("D,short,long", [(512, 5120, 5121), (2048, 5120, 5121), (2560, 2048, 2500), (3072, 2048, 2560),
+                                          (4096, 2048, 4096), (5120, 1500, 2048), (6144, 1365, 1366), (8192, 1024, 1280)])
+def test_short_path_limit_by_width(D, short, long):
+    """The one-GEMM path up to SHORT_TOKENS tokens of a layer no wider than 2048, fewer in a
+    wider one, where the step-by-step path is the faster one from there on."""
+    m = GatedSparseAttention(CFG.hidden_size, CFG.num_heads)
+    for tokens, want in ((short, True), (long, False)):
+        for B in (1, 2):
+            if tokens % B == 0:
+                assert m._short(torch.empty(B, tokens // B, D, dtype=torch.bfloat16, device="meta")) is want
+    assert not m._short(torch.empty(1, 128, D, device="meta"))          # bf16 only
