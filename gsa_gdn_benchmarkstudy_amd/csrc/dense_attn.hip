@@ -1008,17 +1008,23 @@ namespace {
 // share of the tiles, at least 8 (a part costs its prologue, its share of the sum
 // and about 4 us of exchange).  16 heads, causal, us without / with: T = 1024
 // 49 / 45, T = 1537 64 / 49, T = 2048 72 / 53, T = 3000 95 / 74, T = 4096 125 / 109;
-// from T = 5000 on the blocks balance by themselves and none is split.  Short
-// sequences of a batch (K and V of all within half the last-level cache) take the
-// plan's order, longest blocks of all sequences first: B = 3 T = 2000 98 / 87, B = 4
-// T = 4096 329 / 317.
+// T = 5000 138 / 129, T = 5120 138 / 130, T = 5376 147 / 143; past that no block is
+// longer than a part.
+// Short sequences of a batch (K and V of all within half the last-level cache)
+// take the plan's order, longest blocks of all sequences first: 16 heads, B = 3
+// T = 2000 0.84 of the time, B = 4 T = 1500 0.80, B = 8 T = 1000 0.81; 24 heads, B = 4
+// T = 1000 0.82.  Not where a sequence is one block (0.5 us more), and not where the
+// blocks of one length fill the chip by themselves: those then share no K and V
+// in L2 (64 heads, B = 4 T = 1000 89 / 103 us, 32 heads, B = 4 T = 2000 148 / 160, 16
+// heads, B = 16 T = 700 61 / 65).
 gsa::UnitPlan bf16_plan(int B, int T, int Tkv, int H, bool causal) {
   const int nqb = (T + 255) / 256, nt = (Tkv + 63) / 64;
   const int step = causal ? 4 : 0;
   const double tiles = causal ? 2.0 * nqb * (nqb + 1) : (double)nt * nqb;
   const double share = tiles * B * H / 256;
   gsa::UnitPlan plan = split_plan(nqb, nt, step, (int)std::max(8.0, std::ceil(share * 1.4)));
-  if (!plan.n && B > 1 && (int64_t)B * Tkv * H * 512 <= (int64_t)128 << 20) {
+  if (causal && !plan.n && B > 1 && nqb > 1 && H <= 24 && B * (int64_t)H <= 192 &&
+      (int64_t)B * Tkv * H * 512 <= (int64_t)128 << 20) {
     plan = split_plan(nqb, nt, step, std::max(8, plan.tiles(nqb - 1)));
     plan.n = nqb;
   }

@@ -339,3 +339,13 @@ def test_proj_validation(lib):
     assert call(xst=2052) == 4                    # rows not 16-byte aligned
     assert call(qst=4098) == 4
     assert call(cst=130) == 4
+
+
+@pytest.mark.parametrize("B,T,H,order", [(3, 2000, 16, True), (4, 1500, 16, True), (2, 3001, 16, True), (4, 1000, 24, True),
+                                         (4, 1000, 64, False), (8, 512, 64, False), (4, 2000, 32, False),
+                                         (2, 1500, 40, False), (16, 700, 16, False), (32, 200, 16, False)])
+def test_batch_order_where_it_pays(lib, B, T, H, order):
+    """Batches whose blocks are not split take the plan's order only where it is faster: the
+    workspace beyond the masks is then the counters alone, else nothing."""
+    assert lib.gsa_dense_attn_split_bytes(B, T, T, H, 1) == (B * 64 * ((T + 255) // 256) * 4 if order else 0)
+    assert lib.gsa_dense_attn_split_bytes(B, T, T, H, 0) == 0        # blocks of one length: no order to gain from
