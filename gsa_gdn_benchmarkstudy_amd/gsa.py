@@ -33,8 +33,17 @@ from .roctx import range_pop as _range_pop, range_push as _range_push
 FUSED_ALIGN = 64
 
 
+_CU_COUNT = {}
 # Last-level (Infinity) cache of one MI355X.
 _LLC_BYTES = 256 << 20
+
+
+def _cu_count(dev: torch.device) -> int:
+    """Compute units of the device (cached: asking torch takes 23 us)."""
+    idx = dev.index if dev.index is not None else torch.cuda.current_device()
+    if idx not in _CU_COUNT:
+        _CU_COUNT[idx] = torch.cuda.get_device_properties(idx).multi_processor_count
+    return _CU_COUNT[idx]
 
 
 # ---------------------------------------------------------------------------
@@ -556,7 +565,7 @@ class GatedSparseAttention(nn.Module):
         609, T=5400 0.44 469 / 480, T=8800 0.47 915 / 922; T=5835 0.59 502 / 502,
         T=6144 0.75 556 / 524, T=9500 0.94 1044 / 1027, T=8192 1 781 / 751."""
         B, T, D = x.shape
-        cus = torch.cuda.get_device_properties(x.device).multi_processor_count
+        cus = _cu_count(x.device)
         if x.dtype != torch.bfloat16 or B * ((T + 15) // 16) >= 4 * cus:
             return False
         tiles = ((B * T + 255) // 256) * ((5 * D + 255) // 256)

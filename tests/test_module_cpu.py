@@ -118,3 +118,18 @@ def test_short_path_limit_by_width(D, short, long):
             if tokens % B == 0:
                 assert m._short(torch.empty(B, tokens // B, D, dtype=torch.bfloat16, device="meta")) is want
     assert not m._short(torch.empty(1, 128, D, device="meta"))          # bf16 only
+
+
+def test_device_properties_asked_once(monkeypatch):
+    """The placement rule of every long forward reads the number of CUs; torch is asked once."""
+    from types import SimpleNamespace
+
+    from gsa_gdn_benchmarkstudy_amd import gsa
+    asked = []
+    monkeypatch.setattr(torch.cuda, "get_device_properties",
+                        lambda d: asked.append(d) or SimpleNamespace(multi_processor_count=256))
+    monkeypatch.setattr(gsa, "_CU_COUNT", {}, raising=False)
+    m = GatedSparseAttention(CFG.hidden_size, CFG.num_heads)
+    x = SimpleNamespace(shape=(1, 7000, 2048), dtype=torch.bfloat16, device=torch.device("cuda", 0))
+    assert m._gemm_leaves_room(x) and m._gemm_leaves_room(x)
+    assert len(asked) == 1
