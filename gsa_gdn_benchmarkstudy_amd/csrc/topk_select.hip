@@ -4,7 +4,7 @@
 // above +inf); ties at the k-th value go to the lowest indices.  One block per
 // row, in one of two ways:
 //
-// topk_sorted_row, for GSA_ORDER_SCORE_DESC (by score descending, index
+// topk_sorted_kernel, for GSA_ORDER_SCORE_DESC (by score descending, index
 // ascending): a counting sort by value.  The row is read once (into registers
 // up to 16384 keys), its valid scores are counted into value-linear bins
 // between their minimum and maximum, a suffix scan turns the counts into
@@ -19,13 +19,15 @@
 // -1e9): four 8-bit radix passes over the row find the k-th largest key theta
 // and how many entries equal to it are taken, then ordered block-wide
 // compaction (valid ascending, then invalid), or a bitonic sort in LDS by
-// (key desc, index asc).
+// (key desc, index asc).  Such a row pays for the first way's passes too: T = 8192,
+// k = 2048, 2048 rows, 37 us on scores of the indexer, 250 - 290 with one far outlier,
+// with two values or rounded to 50 levels.
 //
 // What bounds it: reading the matrix and writing 9 bytes per selected entry
 // would take 79 us at T = 8192, k = 2048 at the rate of a large copy; the
 // counting and scattering through LDS and the block barriers set the pace.
 // Radix passes and a bitonic sort for every row took 1775 us there,
-// this 132.
+// this 115.
 #include "gsa_common.h"
 
 namespace gsa {
@@ -171,13 +173,11 @@ __device__ void topk_general_row(const float* __restrict__ srow, int Tkv, int k,
   // bitonic sort, descending
   for (int size = 2; size <= kp; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = tid; i < kp; i += kThreads) {
-        const int jx = i ^ stride;
-        if (jx > i) {
-          const uint64_t a = sort_buf[i], c = sort_buf[jx];
-          const bool desc = (i & size) == 0;
-          if (desc ? (a < c) : (a > c)) { sort_buf[i] = c; sort_buf[jx] = a; }
-        }
+      for (int q = tid; q < kp / 2; q += kThreads) {           // pair q: entries i and i + stride
+        const int i = 2 * q - (q & (stride - 1)), jx = i + stride;
+        const uint64_t a = sort_buf[i], c = sort_buf[jx];
+        const bool desc = (i & size) == 0;
+        if (desc ? (a < c) : (a > c)) { sort_buf[i] = c; sort_buf[jx] = a; }
       }
       __syncthreads();
     }
@@ -228,21 +228,19 @@ __device__ __forceinline__ TopkOut<IdxT> topk_row_out(const TopkArgs& p, IdxT* i
 constexpr int kAscThreads = 1024;
 
 // Every row by the general way: rows longer than kMaxSorted, whose validity
-// words do not fit the 64 KiB of LDS beside the entry buffer and the bins.
+// words do not fit the 64 KiB of LDS beside the entry buffer and the bins.  Bound by
+// the latency of its passes, so it needs two blocks per CU: one kernel for both orders
+// and index types has 68 VGPRs and one block, T = 70000, k = 2048, 512 rows 530 us.
 constexpr int kMaxSorted = 65536;
 
-__global__ __launch_bounds__(kAscThreads) void topk_general_kernel(TopkArgs p, int order, int32_t* __restrict__ idx32,
-                                                                   int64_t* __restrict__ idx64) {
+template <int kOrder, typename IdxT>
+__global__ __launch_bounds__(kAscThreads, 8) void topk_general_kernel(TopkArgs p, IdxT* __restrict__ idx) {
   __shared__ SelShared<kAscThreads> sm;
   extern __shared__ uint64_t dyn[];          // GSA_ORDER_SCORE_DESC: a power of two above k entries
   const int row = blockIdx.x;
   const float* srow = p.S + (row / p.T) * p.s_sb + (int64_t)(row % p.T) * p.s_st;
   const int k = p.k_rows ? min(p.k_rows[row], p.width) : p.width;
-  if (idx64) {
-    topk_general_row<kAscThreads>(srow, p.Tkv, k, order, sm, dyn, topk_row_out(p, idx64, row, k, kAscThreads));
-  } else {
-    topk_general_row<kAscThreads>(srow, p.Tkv, k, order, sm, dyn, topk_row_out(p, idx32, row, k, kAscThreads));
-  }
+  topk_general_row<kAscThreads>(srow, p.Tkv, k, kOrder, sm, dyn, topk_row_out(p, idx, row, k, kAscThreads));
 }
 
 // ---------------------------------------------------------------------------
@@ -262,7 +260,7 @@ constexpr int sort_slots(int k) {
 }
 
 template <int kThreads, int kPer, int kBpt, typename IdxT>
-__global__ __launch_bounds__(kThreads) void topk_sorted_kernel(TopkArgs p, IdxT* __restrict__ idx_out, int slots) {
+__global__ __launch_bounds__(kThreads, kThreads == 1024 ? 8 : 1) void topk_sorted_kernel(TopkArgs p, IdxT* __restrict__ idx_out, int slots) {
   constexpr int kBins = kBpt * kThreads;
   constexpr int kWaves = kThreads / 64;
   extern __shared__ uint64_t dyn[];          // entry buffer [slots], then the validity words
@@ -341,43 +339,53 @@ __global__ __launch_bounds__(kThreads) void topk_sorted_kernel(TopkArgs p, IdxT*
 
   if (fine)
     each([&](int, float s) {
-      if (s != -__builtin_inff() && s < __builtin_inff()) atomicAdd(&bins[bin_of_score(s)], 1u);
+      const bool valid = s != -__builtin_inff() && s < __builtin_inff();
+      if constexpr (kPer > 0) {
+        if (valid) atomicAdd(&bins[bin_of_score(s)], 1u);
+      } else {
+        // one addition for a wave whose keys share a bin: 64 on one word one after
+        // another are much of what a row with a far outlier pays for nothing (T = 40000,
+        // k = 64, 512 rows 276 us, 230 with it; rows of the indexer 54 and 56.  Where the
+        // keys are in registers it takes 11 - 25 % of the time of such rows.)
+        const int bin = valid ? bin_of_score(s) : -1, first = __builtin_amdgcn_readfirstlane(bin);
+        if (ballot64(bin != first) == 0) {
+          if (first >= 0 && lane == 0) atomicAdd(&bins[first], 64u);
+        } else if (valid) {
+          atomicAdd(&bins[bin], 1u);
+        }
+      }
     });
   __syncthreads();
-  if (st_bad || !fine) {                                     // uniform: shared flag, block-wide range
-    topk_general_row<kThreads>(srow, Tkv, k, GSA_ORDER_SCORE_DESC, sm, buf, out);
-    return;
-  }
+  bool general = st_bad || !fine;                            // uniform: shared flag, block-wide range
 
   // ---- bins -> first output position of each (entries of all higher bins) ----
-  uint32_t cnt[kBpt], own = 0;
+  uint32_t want = 0;                                         // valid entries selected
+  if (!general) {
+    uint32_t cnt[kBpt], own = 0;
 #pragma unroll
-  for (int i = 0; i < kBpt; i += 4) {
-    const u32x4 v = *reinterpret_cast<const u32x4*>(&bins[kBpt * tid + i]);
+    for (int i = 0; i < kBpt; i += 4) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(&bins[kBpt * tid + i]);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      cnt[i + u] = v[u];
-      own += v[u];
+      for (int u = 0; u < 4; ++u) {
+        cnt[i + u] = v[u];
+        own += v[u];
+      }
     }
-  }
-  uint32_t suf = own;                                        // inclusive suffix sum over the wave
+    uint32_t suf = own;                                      // inclusive suffix sum over the wave
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = (uint32_t)__shfl_down((int)suf, o, 64);
-    if (lane + o < 64) suf += y;
-  }
-  if (lane == 0) wsum[wave] = suf;
-  __syncthreads();
-  uint32_t above = suf - own, total = 0;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = (uint32_t)__shfl_down((int)suf, o, 64);
+      if (lane + o < 64) suf += y;
+    }
+    if (lane == 0) wsum[wave] = suf;
+    __syncthreads();
+    uint32_t a = suf - own, total = 0;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    if (w > wave) above += wsum[w];
-    total += wsum[w];
-  }
-  const int n_valid = (int)total;
-  const uint32_t want = (uint32_t)min(k, n_valid);           // valid entries selected
-  {
-    uint32_t a = above;
+    for (int w = 0; w < kWaves; ++w) {
+      if (w > wave) a += wsum[w];
+      total += wsum[w];
+    }
+    want = min((uint32_t)k, total);
 #pragma unroll
     for (int i = kBpt - 1; i >= 0; --i) {
       // the bin that holds the last wanted entry; fuller bins than can be
@@ -393,9 +401,10 @@ __global__ __launch_bounds__(kThreads) void topk_sorted_kernel(TopkArgs p, IdxT*
 #pragma unroll
     for (int i = 0; i < kBpt; i += 4)
       *reinterpret_cast<u32x4*>(&bins[kBpt * tid + i]) = u32x4{cnt[i], cnt[i + 1], cnt[i + 2], cnt[i + 3]};
+    __syncthreads();
+    general = st_bad != 0;
   }
-  __syncthreads();
-  if (st_bad) {
+  if (general) {
     topk_general_row<kThreads>(srow, Tkv, k, GSA_ORDER_SCORE_DESC, sm, buf, out);
     return;
   }
@@ -519,32 +528,32 @@ int launch_sorted(const gsa::TopkArgs& a, int B, IdxT* idx, hipStream_t s) {
   return launch_status();
 }
 
-int launch_general(const gsa::TopkArgs& a, int B, int order, int32_t* idx32, int64_t* idx64, hipStream_t s) {
-  const size_t lds = order == GSA_ORDER_SCORE_DESC ? (size_t)gsa::sort_slots(a.width) * sizeof(uint64_t) : 0;
-  hipLaunchKernelGGL(gsa::topk_general_kernel, dim3(B * a.T), dim3(gsa::kAscThreads), lds, s, a, order, idx32, idx64);
+template <int kOrder, typename IdxT>
+int launch_general(const gsa::TopkArgs& a, int B, IdxT* idx, hipStream_t s) {
+  const size_t lds = kOrder == GSA_ORDER_SCORE_DESC ? (size_t)gsa::sort_slots(a.width) * sizeof(uint64_t) : 0;
+  hipLaunchKernelGGL((gsa::topk_general_kernel<kOrder, IdxT>), dim3(B * a.T), dim3(gsa::kAscThreads), lds, s, a, idx);
   return launch_status();
 }
 
 // Threads and keys per thread by the row's length: a block's barriers cost more
 // with more waves, so a thread takes 16 keys (32 past 8192) before the block
-// grows.  One matrix, k = min(T, 2048), us with 256 / 512 / 1024 threads:
-// T = 2048 32 / 34 / 78, T = 4096 55 / 59 / 117, T = 8192 133 / 136 / 247,
-// T = 16384 - / 366 / 632.  Rows past 16384 keys are read again in each pass
-// (T = 16384 that way: 851).
+// grows.  A causal T x T matrix of indexer scores, k = min(T, 2048), us with 256 / 512 /
+// 1024 threads: T = 2048 23 / 24 / 35, T = 4096 48 / 48 / 68, T = 8192 125 / 117 / 152,
+// T = 16384 499 / 350 / 396.  Rows past 16384 keys are read again in each pass, whose
+// latency 1024 threads hide better (T = 40000, k = 2048, 512 rows 99 us with 512, 60).
 template <typename IdxT>
 int launch_by_length(const gsa::TopkArgs& a, int B, IdxT* idx, hipStream_t s) {
   if (a.Tkv <= 2048) return launch_sorted<256, 8, 4>(a, B, idx, s);
   if (a.Tkv <= 4096) return launch_sorted<256, 16, 4>(a, B, idx, s);
   if (a.Tkv <= 8192) return launch_sorted<512, 16, 4>(a, B, idx, s);
   if (a.Tkv <= 16384) return launch_sorted<512, 32, 8>(a, B, idx, s);
-  if (a.Tkv <= gsa::kMaxSorted) return launch_sorted<512, 0, 8>(a, B, idx, s);
-  if constexpr (sizeof(IdxT) == 8) return launch_general(a, B, GSA_ORDER_SCORE_DESC, nullptr, idx, s);
-  else return launch_general(a, B, GSA_ORDER_SCORE_DESC, idx, nullptr, s);
+  if (a.Tkv <= gsa::kMaxSorted) return launch_sorted<1024, 0, 4>(a, B, idx, s);
+  return launch_general<GSA_ORDER_SCORE_DESC>(a, B, idx, s);
 }
 
 int launch_topk(const gsa::TopkArgs& a, int B, int order, int32_t* idx, hipStream_t s) {
   if (order == GSA_ORDER_SCORE_DESC) return launch_by_length(a, B, idx, s);
-  return launch_general(a, B, order, idx, nullptr, s);
+  return launch_general<GSA_ORDER_INDEX_ASC>(a, B, idx, s);
 }
 
 // Checks shared by the entry points.

@@ -165,6 +165,25 @@ def test_topk_select_sorted_orders(dev, Tkv, k):
     assert torch.equal(_abi.topk_select_i64(zeros.to(dev), k)[0].cpu(), order)
 
 
+@pytest.mark.parametrize("Tkv,k", [(900, 64), (5000, 2048), (16384, 4096), (16385, 64), (40000, 2048), (66000, 4096)])
+def test_topk_select_rows_of_few_bins(dev, Tkv, k):
+    """Rows whose scores share a few of the counting sort's bins: one far outlier (above, below),
+    two values, whole waves of one value, a bin of exactly the most entries it places."""
+    _log(f"topk few bins Tkv={Tkv} k={k}")
+    g = torch.Generator().manual_seed(Tkv)
+    r = torch.rand(Tkv, generator=g)
+    up, down, edge = r.clone(), r.clone(), torch.linspace(0.0, 1.0, Tkv)
+    up[Tkv // 3], down[Tkv // 2] = 1e6, -1e6
+    edge[100:100 + 192] = edge[100].clone()
+    s = torch.stack([up, down, (r * 2).floor(), (torch.arange(Tkv) // 64 % 7).float(), edge, torch.full((Tkv,), -0.5)])[None]
+    ref_idx, ref_mask = orc.select_topk(s, k)
+    idx, mask = _abi.topk_select_i64(s.to(dev), k)
+    assert torch.equal(idx.cpu(), ref_idx) and torch.equal(mask.cpu(), ref_mask)
+    asc, cnt = orc.select_ascending(s, k)
+    i32, c32, _ = _abi.topk_select(s.to(dev), k, _abi.ORDER_INDEX_ASC)
+    assert torch.equal(c32.cpu(), cnt) and torch.equal(i32.cpu(), asc)
+
+
 def test_topk_select_special_values(dev):
     s = torch.tensor([[[0.5, float("nan"), 2.0, float("inf"), -1e9, float("-inf"), -3.0, 0.5]]])
     gi, gc, gm = _abi.topk_select(s.to(dev), 5, _abi.ORDER_INDEX_ASC, want_mask=True)
