@@ -91,21 +91,21 @@ size_t workspace(int B, int T, int Tkv, int H, int dtype) {
 
 constexpr size_t kMaxWorkspace = (size_t)4 << 30;
 
-// Whether the matrix-core way is the faster one, from the time each takes (us,
-// measured at 16 heads).  The gather, bf16: 20 + the larger of 0.5 per key of a
-// row (its loads are a chain within the row's block) and 0.0009 per row and
-// key (what it reads); T = 512, k = 128 89; T = 8192, k = 2048 13002.  The
-// matrix cores: 35 for the launches and 2.4 for each 64-key tile that a CU takes one
-// after another (all tiles of its 256-row blocks, or where those are split, 1.4
-// times the mean over the CUs, 8 at least, and 25 to add the parts): T = 512, k =
-// 128 54; T = 8192, k = 2048 502; T = 64, Tkv = 4096 75 where the gather takes 52 at k
-// = 64 and 161 at k = 256.  In
-// fp32 the gather reads twice as much and takes 0.6 per key of a row; the matrix
-// cores, whose blocks are split evenly over the chip there, take 40, 9.6 for each
-// 64-key tile of a 128-row block per CU, and up to 30 to add the parts: T = 512,
-// k = 128 62 against 98, T = 2048, k = 2048 212 against 2792, T = 64, Tkv = 4096,
-// k = 64 109 against 59, k = 256 109 against 172.  (All Tkv tiles are counted; what a
-// causal selection leaves out is known on the device only.)
+// Whether the matrix-core way is the faster one, from the time each takes (us; fitted
+// to both, whole calls, at 1400 random sizes: 1 - 64 heads, B = 1 - 8, T <= 4096, Tkv <=
+// 20000, k <= 2048; the pick is 0.5 % above the better one on average).
+// The gather: 8 (5 in fp32), and the larger of its chain of loads within a row's
+// block, 0.355 + 0.004 H per key (0.387 + 0.0082 H), and what it reads, 820 (1160) per
+// million rows x keys x 16 heads; at least 20.5, the host's pace.  T = 512, k = 128,
+// H = 16 74; T = 8192, k = 2048 13002; T = 27, Tkv = 12402, k = 126, H = 8 49.
+// The matrix cores: 11 (10) for the launches, 3.6 (9.9) for each 64-key tile that a CU
+// takes one after another -- its mean share, or a block's tiles, or where blocks are
+// split a part of one: 1.4 times the mean, 8 at least (0.6 or 0.33 times, 2 at least)
+// -- 1.55 (1.15) for each part that the last one adds, and 10.5 per million list
+// entries; at least 26.  The same three calls: 37, 502, 84; fp32 T = 50, Tkv = 13628,
+// k = 182, H = 4 146 where the gather takes 92.  (Query and key length alike are taken
+// for causal, else all Tkv tiles are counted: what a selection leaves out is known
+// on the device only.)
 // The masks reach -8e36 times the scale, which has to stay far below every
 // score: a scale outside [1e-10, 1e10] takes the gather.  A row's bits fit the
 // LDS of a block, and the workspace (2 bytes per element of V, 5 bits per row
@@ -116,13 +116,15 @@ bool dense_serves(int B, int T, int Tkv, int H, int k_sel, float scale, int dtyp
   if (!(scale >= 1e-10f && scale <= 1e10f)) return false;
   if ((size_t)((Tkv + 63) / 64) * 8 > 65536 - 64) return false;
   const int64_t NT = (Tkv + 63) / 64, groups = ((int64_t)T + 255) / 256 * 8;
-  const double reads = 0.0009 * B * T * (double)k_sel * H / 16;
-  const double gather = 20.0 + (bf16 ? std::max(0.5 * k_sel, reads) : std::max(0.6 * k_sel, 2 * reads));
-  const double blocks = B * (double)H * (groups / 8), whole = NT * std::ceil(blocks / 256);
-  const double serial = std::min(whole, std::max(8.0, 1.4 * NT * blocks / 256));
-  const double dense = bf16 ? 35.0 + 2.4 * serial + (serial < whole ? 25.0 : 0.0)
-                            : 40.0 + 9.6 * NT * (B * (double)H * ((T + 127) / 128) / 256.0) + std::min(30.0, 3.0 * NT);
-  if (dense > gather) return false;
+  const double entries = 1e-6 * B * T * (double)k_sel, reads = entries * H / 16;
+  const double gather = bf16 ? 8.0 + std::max((0.355 + 0.004 * H) * k_sel, 820.0 * reads)
+                             : 5.0 + std::max((0.387 + 0.0082 * H) * k_sel, 1160.0 * reads);
+  const double nqb = bf16 ? groups / 8 : (T + 127) / 128;
+  const double mean = NT * (B * (double)H * nqb) / 256 * (T == Tkv ? (nqb + 1) / (2 * nqb) : 1.0);
+  const double part = bf16 ? std::max(8.0, 1.4 * mean) : std::max(2.0, (2 * mean < 40 ? 0.6 : 0.33) * mean);
+  const double serial = std::max(mean, std::min((double)NT, part)), parts = part < NT ? std::ceil(NT / part) : 0.0;
+  const double dense = (bf16 ? 11.0 : 10.0) + (bf16 ? 3.6 : 9.9) * serial + (bf16 ? 1.55 : 1.15) * parts + 10.5 * entries;
+  if (std::max(26.0, dense) > std::max(20.5, gather)) return false;
   if (B * groups * NT > 0x3fffffffLL / 32 || (int64_t)B * H * NT > 0x3fffffffLL) return false;
   return workspace(B, T, Tkv, H, dtype) <= kMaxWorkspace;
 }

@@ -349,3 +349,14 @@ def test_batch_order_where_it_pays(lib, B, T, H, order):
     workspace beyond the masks is then the counters alone, else nothing."""
     assert lib.gsa_dense_attn_split_bytes(B, T, T, H, 1) == (B * 64 * ((T + 255) // 256) * 4 if order else 0)
     assert lib.gsa_dense_attn_split_bytes(B, T, T, H, 0) == 0        # blocks of one length: no order to gain from
+
+
+@pytest.mark.parametrize("dtype,B,T,Tkv,H,k,dense", [
+    ("bf16", 1, 512, 512, 16, 128, True), ("bf16", 1, 8192, 8192, 16, 2048, True), ("bf16", 1, 64, 4096, 16, 1024, True),
+    ("bf16", 1, 27, 12402, 8, 126, False), ("bf16", 8, 44, 44, 12, 38, False), ("bf16", 1, 2048, 8192, 40, 128, False),
+    ("bf16", 1, 13, 121, 1, 44, False), ("f32", 2, 1537, 1537, 16, 256, True), ("f32", 1, 200, 200, 16, 128, True),
+    ("f32", 1, 50, 13628, 4, 182, False), ("f32", 1, 300, 20000, 1, 256, False), ("f32", 1, 64, 4096, 2, 128, False)])
+def test_selected_attention_rule(lib, dtype, B, T, Tkv, H, k, dense):
+    """The launcher's choice at sizes where one way was measured clearly faster (workspace 0: the gather)."""
+    dt = _abi.DTYPE_BF16 if dtype == "bf16" else _abi.DTYPE_F32
+    assert (lib.gsa_selected_attn_workspace_bytes(B, T, Tkv, H, k, 128 ** -0.5, dt) > 0) is dense
