@@ -294,7 +294,7 @@ constexpr int kWaitVmcnt0 = (0x7 << 4) | (0xf << 8);
 // ---------------------------------------------------------------------------
 struct Selection {
   const uint32_t* bits;   // [B*T][W] bitmask, W = 2*ceil(Tkv/64): bit j of a row: key j is selected
-  const int2* range;      // [B*T] first and past-last 64-key tile of the row's keys (none: INT_MAX, 0)
+  const int2* range;      // [B*T] first and past-last 64-key tile of the row's keys (none, or named twice: INT_MAX, 0)
   const uint8_t* twice;   // [B*T] nonzero: the row's list names a key twice, so the bitmask cannot stand for it (or null)
   uint8_t* redo;          // [B*T*H] written by the attention kernel: nonzero: that head of the row has to come from the gather kernel
 };

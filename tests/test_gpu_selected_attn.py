@@ -124,6 +124,29 @@ def test_selected_attention_rows_for_the_gather(dev, dtype):
         assert torch.equal(out[~fin].isnan(), ref[~fin].isnan())
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T,Tkv,every", [(600, 600, 1), (600, 2000, 1), (700, 700, 2), (513, 1100, 256)])
+def test_selected_attention_lists_with_repeats(dev, dtype, T, Tkv, every):
+    """Every list, every second one or one a block names a key twice: those rows equal the
+    gather kernel's bit for bit (blocks whose rows all do compute no tile of their own), the
+    others the same call without repeats."""
+    _log(f"selected attention repeats {dtype} T={T} Tkv={Tkv} every={every}")
+    B, H, K = 1, 2, 160
+    g = torch.Generator().manual_seed(T)
+    q = torch.randn(B, T, H, 128, generator=g).to(dtype).to(dev)
+    k, v = (torch.randn(B, Tkv, H, 128, generator=g).to(dtype).to(dev) for _ in range(2))
+    idx, mask = (t.to(dev) for t in _selection(B, T, Tkv, K, seed=11, kind="any"))
+    assert _abi.load().gsa_selected_attn_workspace_bytes(B, T, Tkv, H, K, SCALE, _abi.dtype_code(dtype)) > 0
+    plain = G.fused_sparse_attention(q, k, v, idx, mask, SCALE)
+    idx[:, ::every, 7] = idx[:, ::every, 90]
+    out = G.fused_sparse_attention(q, k, v, idx, mask, SCALE)
+    gather = _abi.sparse_attn(q, k, v, idx.int(), SCALE, mask=mask)
+    twice = torch.arange(T, device=dev) % every == 0
+    assert torch.equal(out[:, twice], gather[:, twice])
+    _close(out, _attend64(q, k, v, idx, mask, SCALE), v, dtype)
+    _close(out[:, ~twice], plain[:, ~twice].double(), v, dtype)
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.5, 1e-20, 1e20])
 def test_selected_attention_scales_for_the_gather(dev, scale):
     """Scales for which a masked score would not vanish take the gather kernel: same bits."""
