@@ -508,8 +508,11 @@ def selected_attn(q, k, v, idx, scale: float, mask=None) -> torch.Tensor:
     lib = load()
     _need_cuda(q, k, v, idx, mask)
 
+    if mask is not None and mask.dtype != torch.bool:
+        mask = mask.to(torch.uint8)
+
     def gather():
-        m = None if mask is None else mask.to(torch.uint8).contiguous()
+        m = None if mask is None else mask.contiguous()
         return sparse_attn(q, k, v, idx.to(torch.int32).contiguous(), scale, mask=m)
 
     if q.dim() != 4 or k.dim() != 4 or idx.dim() != 3 or idx.numel() == 0:
@@ -535,7 +538,7 @@ def selected_attn(q, k, v, idx, scale: float, mask=None) -> torch.Tensor:
         idx = idx.to(torch.int32)
     idx = idx.contiguous()
     if mask is not None:
-        mask = (mask if mask.dtype in (torch.bool, torch.uint8) else mask.to(torch.uint8)).contiguous()
+        mask = mask.contiguous()
     out = torch.empty(B, T, H, d, device=q.device, dtype=q.dtype)
     st = lib.gsa_selected_attn(_ptr(q), *_rows(q, HD), _ptr(k), *_rows(k, HD), _ptr(v), *_rows(v, HD),
                                _ptr(idx), idx.element_size(), idx.stride(0), idx.stride(1), k_sel, None, _ptr(mask),

@@ -147,6 +147,23 @@ def test_selected_attention_lists_with_repeats(dev, dtype, T, Tkv, every):
     _close(out[:, ~twice], plain[:, ~twice].double(), v, dtype)
 
 
+@pytest.mark.parametrize("mtype", [torch.bool, torch.uint8, torch.int64])
+def test_selected_attention_gather_sizes(dev, monkeypatch, mtype):
+    """Sizes that the rule gives to the gather kernel: same bits, and a bool or byte mask goes to
+    it as it is (no conversion launch)."""
+    B, T, H, K = 1, 300, 2, 12
+    g = torch.Generator().manual_seed(4)
+    q, k, v = (torch.randn(B, T, H, 128, generator=g).bfloat16().to(dev) for _ in range(3))
+    idx, mask = (t.to(dev) for t in _selection(B, T, T, K, seed=5, kind="causal"))
+    assert _abi.load().gsa_selected_attn_workspace_bytes(B, T, T, H, K, SCALE, _abi.DTYPE_BF16) == 0
+    want = _abi.sparse_attn(q, k, v, idx.int(), SCALE, mask=mask.to(torch.uint8))
+    seen, real = [], _abi.sparse_attn
+    monkeypatch.setattr(_abi, "sparse_attn", lambda *a, mask, **kw: seen.append(mask) or real(*a, mask=mask, **kw))
+    m = mask.to(mtype)
+    assert torch.equal(G.fused_sparse_attention(q, k, v, idx, m, SCALE), want)
+    assert mtype == torch.int64 or seen[0].data_ptr() == m.data_ptr()
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.5, 1e-20, 1e20])
 def test_selected_attention_scales_for_the_gather(dev, scale):
     """Scales for which a masked score would not vanish take the gather kernel: same bits."""
