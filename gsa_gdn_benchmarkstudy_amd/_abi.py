@@ -434,7 +434,7 @@ def prologue(k=None, v=None, vg=None, cos=None, sin=None, k_out=None, v_out=None
 
 
 def rope_qk(q, k, cos, sin):
-    """RoPE of q and k (one shape, one dtype) in one launch -> (q_out, k_out), contiguous."""
+    """RoPE of q and k (one shape, one dtype) in one call -> (q_out, k_out), contiguous."""
     lib = load()
     _need_cuda(q, k, cos, sin)
     B, T, H, d = q.shape

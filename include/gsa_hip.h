@@ -260,7 +260,7 @@ int gsa_prologue(const void* k, int64_t k_sb, int64_t k_st,
                  void* stream);
 
 /*
- * RoPE of q and k [B,T,H,d] in one launch: apply_rotary_pos_emb
+ * RoPE of q and k [B,T,H,d] in one call: apply_rotary_pos_emb
  * (gsa_triton/gsa_opt.py:396-401), each rounded as gsa_prologue's k_out, into
  * contiguous q_out and k_out.  cos, sin [T,d] (row stride cs_st) in dtype.
  * Supported: d == 128, 1 <= H <= 64.

@@ -182,6 +182,20 @@ def test_apply_rotary_pos_emb_rows(dev, B, T, H, dtype):
     assert torch.equal(oq.cpu(), ref[0]) and torch.equal(ok.cpu(), ref[2])
 
 
+@pytest.mark.parametrize("B,T,H,dtype", [(1, 1279, 64, torch.float32), (1, 1280, 64, torch.float32), (2, 1700, 33, torch.float32),
+                                         (1, 2600, 32, torch.float32), (1, 2560, 64, torch.bfloat16)])
+def test_apply_rotary_pos_emb_large(dev, B, T, H, dtype):
+    """Around the heads and sizes from which q and k are taken one after the other (40 MiB a
+    tensor), q and k as views of one buffer: the oracle's rounding, on the device."""
+    g = torch.Generator(device=dev).manual_seed(T)
+    qk = torch.randn(B, T, 2, H, 128, generator=g, device=dev).to(dtype)
+    cos, sin = (t.to(dev) for t in orc.RopeCache(128, dtype).tables(T, dtype))
+    out = G.apply_rotary_pos_emb(qk[:, :, 0], qk[:, :, 1], cos, sin)
+    for i in (0, 1):
+        assert out[i].is_contiguous()
+        assert torch.equal(out[i], orc.apply_rope(qk[:, :, i], cos[None, :, None], sin[None, :, None]))
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_rotary_embedding_tables_on_device(dev, dtype):
     """RotaryEmbedding.forward(seq_len, device, dtype) after a module cast: the cached
