@@ -1,6 +1,7 @@
 """The C ABI library without a GPU: it loads, exports every declared symbol,
 and rejects bad arguments on the host before anything is enqueued."""
 
+import ctypes
 import os
 import re
 
@@ -360,3 +361,28 @@ def test_selected_attention_rule(lib, dtype, B, T, Tkv, H, k, dense):
     """The launcher's choice at sizes where one way was measured clearly faster (workspace 0: the gather)."""
     dt = _abi.DTYPE_BF16 if dtype == "bf16" else _abi.DTYPE_F32
     assert (lib.gsa_selected_attn_workspace_bytes(B, T, Tkv, H, k, 128 ** -0.5, dt) > 0) is dense
+
+
+def _layer(lib, **kw):
+    off = (ctypes.c_int64 * 8)(0, 256, 512, 768, 1024, 1280, 1536, 1600)
+    a = dict(proj=P, offsets=off, bias=P, cos=P, sin=P, halves=P, B=1, T=32, H=2, d=128, Hi=4, di=64, k_eff=8, kb=0, kmin=0,
+             kmax=0, out=P, ws=P, nws=lib.gsa_layer_workspace_bytes(1, 32, 2, 0), sb=32 * 1664, st=1664)
+    a.update(kw)
+    return lib.gsa_layer_attn(a["proj"], a["sb"], a["st"], a["offsets"], a["bias"], 0.125, a["cos"], a["sin"], 128,
+                              a["halves"], 128, a["B"], a["T"], a["H"], a["d"], a["Hi"], a["di"], 0.1, a["k_eff"], a["kb"],
+                              a["kmin"], a["kmax"], None, a["out"], 32 * 256, 256, a["ws"], a["nws"], None)
+
+
+def test_layer_attn_validation(lib):
+    """What gsa_layer_attn refuses before its first launch."""
+    for name in ("proj", "offsets", "bias", "cos", "sin", "halves", "out", "ws"):
+        assert _layer(lib, **{name: None}) == 1
+    assert _layer(lib, T=0) == _layer(lib, d=64) == _layer(lib, H=65) == _layer(lib, H=0) == 2
+    assert _layer(lib, nws=lib.gsa_layer_workspace_bytes(1, 32, 2, 0) - 1) == 2
+    assert _layer(lib, k_eff=0, kb=8, kmin=2, kmax=16) == 2              # the variance rule needs the larger workspace
+    assert _layer(lib, ws=P + 16) == 4
+    assert _layer(lib, Hi=8) == _layer(lib, di=32) == 2
+    assert _layer(lib, k_eff=33) == 5
+    assert _layer(lib, proj=MIS) == 4
+    assert lib.gsa_layer_workspace_bytes(0, 32, 2, 0) == lib.gsa_layer_workspace_bytes(1, 32, 65, 0) == 0
+    assert lib.gsa_layer_workspace_bytes(1, 32, 2, 1) > lib.gsa_layer_workspace_bytes(1, 32, 2, 0)

@@ -802,6 +802,77 @@ def test_dense_attention_split_blocks(dev, B, T, Tkv, H, causal):
     assert torch.all(a[:, 5] == 0)
 
 
+@pytest.mark.parametrize("B,T,Tkv,H,causal", [
+    (1, 769, 769, 16, True), (1, 2048, 2048, 16, True), (1, 4096, 4096, 8, True), (2, 1500, 1500, 4, True),   # 2 - 4 parts
+    (1, 300, 700, 2, False), (1, 256, 1600, 4, False), (2, 257, 9000, 1, False),                              # 2, 4, 18 parts
+])
+def test_dense_attention_split_blocks_vs_float64(dev, B, T, Tkv, H, causal):
+    """Split and unsplit against float64 by 2-norm.  Two roundings to bf16 make the error, the
+    weights (relative 2^-9 each, independent: a share of 2^-9 / sqrt(3) of sqrt(sum p^2 v^2),
+    the norm of an average of independent v) and the output: below 2^-8 together.  A tile left
+    out or added twice among at most 141 shifts the norm by more than 1 / 141 = 2^-7.2."""
+    _log(f"split dense vs float64 B={B} T={T} Tkv={Tkv} H={H} causal={causal}")
+    g = torch.Generator(device=dev).manual_seed(T + Tkv)
+    q = torch.randn(B, T, H, 128, generator=g, device=dev).bfloat16()
+    k, v = (torch.randn(B, Tkv, H, 128, generator=g, device=dev).bfloat16() for _ in range(2))
+    vt = torch.zeros(B, H, 128, _abi.vt_len(Tkv), dtype=torch.bfloat16, device=dev)
+    vt[..., :Tkv] = v.permute(0, 2, 3, 1)
+    sel = torch.rand(B, T, Tkv, generator=g, device=dev) < 0.4
+    if causal:
+        sel &= torch.ones(T, Tkv, dtype=torch.bool, device=dev).tril()
+    sel[..., 0] = True
+    pad = torch.zeros(B, T, 32 * _abi.mask_words(Tkv), dtype=torch.int64, device=dev)
+    pad[..., :Tkv] = sel
+    words = (pad.view(B, T, -1, 32) << torch.arange(32, device=dev)).sum(-1)
+    bits = torch.where(words >= 2 ** 31, words - 2 ** 32, words).int()
+    ref = torch.empty(B, T, H, 128, dtype=torch.float64, device=dev)
+    for b in range(B):
+        for h in range(H):
+            z = (q[b, :, h].double() @ k[b, :, h].double().t().contiguous()) * 128 ** -0.5
+            ref[b, :, h] = torch.softmax(z.masked_fill_(~sel[b], float("-inf")), -1) @ v[b, :, h].double()
+    err = {}
+    for split in (True, False):
+        out = _abi.dense_attn(q, k, vt, bits, 128 ** -0.5, causal=causal, split=split)
+        err[split] = float((out.double() - ref).norm() / ref.norm())
+    _log(f"  split {err[True]:.6f} unsplit {err[False]:.6f}")
+    assert err[True] < 2.0 ** -8 and err[False] < 2.0 ** -8
+    assert err[True] < 1.02 * err[False]              # (no further off: within the scatter of the roundings)
+
+
+@pytest.mark.parametrize("B,T,H,mode", [(1, 300, 4, "fixed"), (1, 1537, 16, "fixed"), (1, 2049, 16, "variance"),
+                                        (2, 1100, 8, "fixed"), (3, 1100, 16, "variance")])
+def test_layer_attn_equals_its_steps(dev, B, T, H, mode):
+    """gsa_layer_attn against the entry points it stands for on the same projections, bit for
+    bit: with query blocks whole, in parts and in the batch's order, both selector modes."""
+    _log(f"layer_attn B={B} T={T} H={H} {mode}")
+    g = torch.Generator(device=dev).manual_seed(T)
+    D, Hi, di = 128 * H, 4, 64
+    sizes = [D] * 5 + [Hi * di, di, Hi]
+    off = [sum(sizes[:i]) for i in range(8)]
+    N = (sum(sizes) + 63) // 64 * 64
+    proj = torch.randn(B, T, N, generator=g, device=dev).bfloat16()
+    cos, sin = (t.to(dev) for t in orc.RopeCache(128, torch.bfloat16).tables(T, torch.bfloat16))
+    halves = torch.cat((cos[:, :64], sin[:, :64]), dim=-1).contiguous()
+    bias = torch.randn(Hi, generator=g, device=dev)
+    k_eff, adaptive = min(256, T), ((200, 64, 512) if mode == "variance" else None)
+    out, k_rows = _abi.layer_attn(proj, _abi.row_offsets(off), bias, 0.125, cos, sin, halves, H, 128, Hi, di, 128 ** -0.5,
+                                  k_eff, adaptive)
+    q, k, v, vg, og = (proj[..., o:o + D].view(B, T, H, 128) for o in off[:5])
+    iq, ik, iw = proj[..., off[5]:off[6]].view(B, T, Hi, di), proj[..., off[6]:off[7]], proj[..., off[7]:off[7] + Hi]
+    if adaptive:
+        bits, _, _, kr, _ = _abi.indexer_select_adaptive(iq, ik, iw, bias, 0.125, *adaptive, indices=False)
+        assert torch.equal(k_rows, kr)
+    else:
+        bits, _, _ = _abi.indexer_select(iq, ik, iw, bias, 0.125, k_eff, indices=False)
+        assert k_rows is None
+    split = _abi.dense_attn_split_bytes(B, T, T, H) > 0
+    assert split == (T > 300)
+    kr, vt, ws = _abi.prologue_vt(v, vg, k=k, cos=cos, sin=sin, bits=bits, Tkv=T, causal=True, split_heads=H if split else 0)
+    want = _abi.dense_attn(q, kr, vt, bits, 128 ** -0.5, og=og, cos=halves, ws=ws, masks_ready=True, split=split,
+                           flags=_abi.ATTN_ROPE_Q | _abi.ATTN_OUT_GATE | _abi.ATTN_ROPE_HALVES)
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("built_for_split", [True, False])
 def test_dense_attention_split_reuses_masks(dev, built_for_split):
     """Ready masks serve several split calls, also in a workspace whose words behind the

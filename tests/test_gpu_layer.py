@@ -16,7 +16,7 @@ import numpy as np
 import pytest
 import torch
 
-from gsa_gdn_benchmarkstudy_amd import GatedSparseAttention
+from gsa_gdn_benchmarkstudy_amd import GatedSparseAttention, _abi
 from oracle import gsa_oracle as orc
 
 pytestmark = pytest.mark.gpu
@@ -363,3 +363,41 @@ def test_fp32_layer_scales_for_the_gather(dev, scale):
         with torch.no_grad():
             out.append(m(x))
     assert torch.equal(out[0].nan_to_num(7.0), out[1].nan_to_num(7.0))
+
+
+@pytest.mark.parametrize("B,T,mode", [(1, 130, "fixed"), (1, 700, "fixed"), (2, 513, "fixed"), (2, 300, "variance")])
+def test_fp32_masked_layer_vs_oracle(dev, B, T, mode):
+    """The fp32 layer on the matrix cores (attn_impl "auto") at ragged sizes, in parts and
+    whole, against the oracle on the layer's own selection."""
+    _log(f"layer fp32 masked B={B} T={T} {mode}")
+    cfg = orc.GSAConfig(hidden_size=512, num_heads=4, k_max=200, k_base=120, k_min=16)
+    sd = orc.synthetic_state(cfg, seed=5)
+    x = orc.synthetic_input(B, T, cfg.hidden_size, seed=6)
+    m = _model(cfg, sd, dev, torch.float32)
+    m.topk_selector.mode = mode
+    assert _abi.masked_attn_serves(B, T, 4, m.topk_selector.k_effective(T), torch.float32, m.scale)
+    with torch.no_grad():
+        y = m(x.to(dev)).cpu()
+    idx, cnt = _gpu_selection(m, x.to(dev))
+    assert torch.allclose(y, _oracle_on_selection(sd, cfg, x, idx, cnt), atol=1e-4, rtol=0)
+
+
+@pytest.mark.parametrize("B,T,mode", [(2, 2600, "gemm"), (3, 2000, "serial")])
+def test_batch_order_in_the_layer_equals_whole_blocks(dev, monkeypatch, B, T, mode):
+    """Above the short path's sizes a batch's blocks take the plan's order, beside the main GEMM
+    or after the select: the same bits as the kernel's own order, in either placement."""
+    _log(f"layer batch order B={B} T={T}")
+    cfg = orc.GSAConfig(hidden_size=2048, num_heads=16, k_max=512, k_base=512, k_min=64)
+    sd = orc.cast_state(orc.synthetic_state(cfg, seed=2), torch.bfloat16)
+    x = orc.synthetic_input(B, T, 2048, seed=3).to(torch.bfloat16).to(dev)
+    m = _model(cfg, sd, dev, torch.bfloat16)
+    assert not m._short(x) and m._gemm_leaves_room(x) == (mode == "gemm")
+    counters = B * 64 * ((T + 255) // 256) * 4
+    assert _abi.dense_attn_split_bytes(B, T, T, 16) == counters        # an order, no parts
+    with torch.no_grad():
+        y = m(x)
+        m.indexer_overlap = "serial" if mode == "gemm" else "gemm"
+        assert torch.equal(m(x), y)
+        m.indexer_overlap = "auto"
+        monkeypatch.setattr(_abi, "dense_attn_split_bytes", lambda *a: 0)
+        assert torch.equal(m(x), y)

@@ -1,10 +1,12 @@
 """fused_sparse_attention on the matrix cores (gsa_selected_attn) against float64 and
 against the gather kernel, whose semantics it keeps.
 
-Bound, bf16: the weights are exact to 2^-17 and the sums are fp32, so an output is
-within one rounding to bf16 (half an ulp, 2^-9 relative, and 2^-8 allowed for a
-value at a rounding boundary) of the float64 result plus fp32 sum error of
-sum_j p_j |v_j| <= max|v|, far below 2^-16 max|v|.
+Bound, bf16: the weights keep 24 bits (three bf16 parts) and the sums are fp32, so an
+output is within one rounding to bf16 (half an ulp, 2^-9 relative, and 2^-8 allowed
+for a value at a rounding boundary) of the float64 result plus fp32 sum error of
+sum_j p_j |v_j| <= max|v|, far below 2^-16 max|v|.  What those bounds leave open,
+fewer bits in the weights or longer chains of fp32 sums, test_selected_attention_precision
+pins.
 """
 
 import pytest
@@ -87,6 +89,31 @@ def test_selected_attention_vs_float64(dev, dtype, B, T, Tkv, H, K, kind):
     perm = torch.randperm(K, generator=g).to(dev)
     again = G.fused_sparse_attention(q, k, v, idx[..., perm].int(), mask[..., perm], SCALE)
     assert torch.equal(again, out)
+
+
+@pytest.mark.parametrize("B,T,Tkv,K,kind", [(1, 700, 700, 200, "causal"), (1, 300, 3000, 600, "any"), (2, 1100, 1100, 512, "causal")])
+def test_selected_attention_precision(dev, B, T, Tkv, K, kind):
+    """fp32: 3.2e-7 by 2-norm, what the gather kernel's own sums are from float64 (a score in
+    four chains of 32 products comes to 2.4e-7, in one chain of 128 to 4.1e-7).  bf16: the share of outputs that are not the
+    float64 result's own rounding.  An error e relative to the value makes 2 e / 2^-8 of them
+    differ: fp32 sums, e about 2^-22, 1e-4; weights of two bf16 parts, e about 2^-18, 2e-3."""
+    H = 2
+    g = torch.Generator().manual_seed(K)
+    idx, mask = (t.to(dev) for t in _selection(B, T, Tkv, K, seed=3, kind=kind))
+    q, k, v = (torch.randn(B, n, H, 128, generator=g) for n in (T, Tkv, Tkv))
+    for dtype in DTYPES:
+        qd, kd, vd = (t.to(dtype).to(dev) for t in (q, k, v))
+        assert _abi.load().gsa_selected_attn_workspace_bytes(B, T, Tkv, H, K, SCALE, _abi.dtype_code(dtype)) > 0
+        out = G.fused_sparse_attention(qd, kd, vd, idx, mask, SCALE)
+        ref = _attend64(qd, kd, vd, idx, mask, SCALE)
+        if dtype == torch.float32:
+            err = float((out.double() - ref).norm() / ref.norm())
+            _log(f"precision fp32 T={T} Tkv={Tkv}: {err:.2e}")
+            assert err < 3.2e-7
+        else:
+            share = float((out != ref.to(torch.bfloat16)).double().mean())
+            _log(f"precision bf16 T={T} Tkv={Tkv}: {share:.2e} of the outputs rounded elsewhere")
+            assert share < 5e-4
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
