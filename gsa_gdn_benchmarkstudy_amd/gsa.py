@@ -563,8 +563,14 @@ class GatedSparseAttention(nn.Module):
         than half of them.  us per forward beside the GEMM / before it, with that
         share: B=2 T=4100 0.16 600 / 622, B=2 T=2600 0.28 366 / 376, T=7000 0.38 592 /
         609, T=5400 0.44 469 / 480, T=8800 0.47 915 / 922; T=5835 0.59 502 / 502,
-        T=6144 0.75 556 / 524, T=9500 0.94 1044 / 1027, T=8192 1 781 / 751."""
+        T=6144 0.75 556 / 524, T=9500 0.94 1044 / 1027, T=8192 1 781 / 751 (D=2048).  Widths of
+        1024 to 3072: narrower ones wait for the host, which the second stream costs 90 us
+        (D=512 B=3 T=3000 267 / 182, D=1536 B=2 T=3600 389 / 408, D=3072 T=3500 501 / 516), in
+        wider ones the GEMM is slowed by more than is hidden (D=4096 T=3500 759 / 729, B=2
+        T=3600 1535 / 1499; D=8192 T=5200 3611 / 3627)."""
         B, T, D = x.shape
+        if not 1024 <= D <= 3072:
+            return False
         cus = _cu_count(x.device)
         if x.dtype != torch.bfloat16 or B * ((T + 15) // 16) >= 4 * cus:
             return False

@@ -133,3 +133,17 @@ def test_device_properties_asked_once(monkeypatch):
     x = SimpleNamespace(shape=(1, 7000, 2048), dtype=torch.bfloat16, device=torch.device("cuda", 0))
     assert m._gemm_leaves_room(x) and m._gemm_leaves_room(x)
     assert len(asked) == 1
+
+
+@pytest.mark.parametrize("D,B,T,beside", [(512, 3, 3000, False), (512, 2, 3600, False), (1024, 1, 7000, True), (1536, 2, 3600, True),
+                                          (2048, 2, 4100, True), (2048, 1, 8192, False), (3072, 1, 3500, True),
+                                          (4096, 1, 3500, False), (4096, 2, 3600, False), (8192, 1, 5200, False)])
+def test_select_beside_the_gemm_by_width(monkeypatch, D, B, T, beside):
+    """Where the select runs beside the main GEMM: widths at which that was measured faster."""
+    from types import SimpleNamespace
+
+    from gsa_gdn_benchmarkstudy_amd import gsa
+    monkeypatch.setattr(gsa, "_cu_count", lambda dev: 256)
+    m = GatedSparseAttention(CFG.hidden_size, CFG.num_heads)
+    x = SimpleNamespace(shape=(B, T, D), dtype=torch.bfloat16, device=torch.device("cuda", 0))
+    assert m._gemm_leaves_room(x) is beside
