@@ -330,10 +330,10 @@ extern "C" int gsa_rope_qk(const void* q, int64_t q_sb, int64_t q_st, const void
   // Four rows of many heads take the registers of a CU's one block (1024 threads in
   // fp32): large tensors then go through prologue_kernel, one after the other.  us,
   // that way / here: fp32 H = 40 80 MiB a tensor 64 / 67, 160 122 / 128, H = 64 160 117 / 122, 256 186 /
-  // 195, H = 32 256 185 / 186; bf16 H = 64 80 63 / 66, 128 99 / 102, H = 40 84 66 / 62.
+  // 195, H = 32 80 61 / 60, 512 362 / 369; bf16 H = 64 80 63 / 66, 128 99 / 102, H = 40 84 66 / 62.
   // (Below 40 MiB two launches cost the host more.)
   const int64_t mib = ((int64_t)B * T * H * 128 * dtype_size(dtype)) >> 20;
-  if (H > (dtype == GSA_DTYPE_F32 ? 32 : 48) && mib >= 40) {
+  if (H >= (dtype == GSA_DTYPE_F32 ? 32 : 49) && mib >= 40) {
     const int st = gsa_prologue(q, q_sb, q_st, nullptr, 0, 0, nullptr, 0, 0, cos, sin, cs_st, B, T, H, d, dtype, q_out,
                                 nullptr, stream);
     if (st) return st;

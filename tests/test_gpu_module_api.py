@@ -183,7 +183,8 @@ def test_apply_rotary_pos_emb_rows(dev, B, T, H, dtype):
 
 
 @pytest.mark.parametrize("B,T,H,dtype", [(1, 1279, 64, torch.float32), (1, 1280, 64, torch.float32), (2, 1700, 33, torch.float32),
-                                         (1, 2600, 32, torch.float32), (1, 2560, 64, torch.bfloat16)])
+                                         (1, 2600, 32, torch.float32),
+                                         (1, 3400, 31, torch.float32), (1, 2560, 64, torch.bfloat16)])
 def test_apply_rotary_pos_emb_large(dev, B, T, H, dtype):
     """Around the heads and sizes from which q and k are taken one after the other (40 MiB a
     tensor), q and k as views of one buffer: the oracle's rounding, on the device."""
