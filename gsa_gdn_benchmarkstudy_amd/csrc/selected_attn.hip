@@ -197,9 +197,10 @@ static size_t masked_workspace(int B, int T, int H, int k_sel) {
          dense_f32_bytes(B, T, T, H);
 }
 
-// From the time each way takes (us, 16 heads): the gather as in dense_serves, the
-// matrix cores 30 for the launches and 4.9 for each 32-key tile of a 128-row
-// block per CU (T = 2048, k = 256: 191 against 485 and 52 for the index lists).
+// From the time each way takes (us, 16 heads): the gather 20 and the larger of 0.5 per
+// key of a row and 1.8 per 1000 pairs of a row and a key (and the index lists, left
+// out), the matrix cores 30 for the launches and 4.9 for each 32-key tile of a
+// 128-row block per CU (T = 2048, k = 256: 191 against 485 and 52 for the lists).
 extern "C" size_t gsa_masked_attn_workspace_bytes(int B, int T, int H, int k_sel, int dtype) {
   if (B < 1 || T < 1 || H < 1 || H > 64 || k_sel < 1 || k_sel > T || dtype != GSA_DTYPE_F32) return 0;
   if ((int64_t)B * T > 0x7fffffffLL) return 0;

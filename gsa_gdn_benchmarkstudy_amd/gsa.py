@@ -319,9 +319,10 @@ class GatedSparseAttention(nn.Module):
          writing the selection as a bitmask, and for the gather attention
          ascending int32 indices with per-row counts (no score is stored:
          they are recomputed pass by pass and the candidates near each row's
-         threshold stay in LDS) -- before the q/k/v/gate GEMM while RoPE(k) and
-         V^T fit the last-level cache, else beside the producer (or beside the
-         GEMM, on request); the dense attention's lane masks
+         threshold stay in LDS) -- beside the q/k/v/gate GEMM where its last
+         round of tiles leaves CUs idle, else before it while RoPE(k) and V^T
+         fit the last-level cache, else beside the producer (or where
+         ``indexer_overlap`` says); the dense attention's lane masks
          (gsa_dense_lane_masks) follow on the second stream (with the
          indexer on the current stream: built in the producer's launch);
       3. current stream: RoPE(k) and v * sigmoid(vg) (gsa_prologue_vt, V
