@@ -20,14 +20,13 @@
 // and how many entries equal to it are taken, then ordered block-wide
 // compaction (valid ascending, then invalid), or a bitonic sort in LDS by
 // (key desc, index asc).  Such a row pays for the first way's passes too: T = 8192,
-// k = 2048, 2048 rows, 37 us on scores of the indexer, 250 - 290 with one far outlier,
-// with two values or rounded to 50 levels.
+// k = 2048, 2048 rows, 37 us on scores of the indexer, 270 with one far outlier or of
+// two values, 170 rounded to 50 levels (radix passes for every row: 420 - 540).
 //
-// What bounds it: reading the matrix and writing 9 bytes per selected entry
-// would take 79 us at T = 8192, k = 2048 at the rate of a large copy; the
-// counting and scattering through LDS and the block barriers set the pace.
-// Radix passes and a bitonic sort for every row took 1775 us there,
-// this 115.
+// What bounds it: the VALU (91 % busy: the bin and the place of every key; LDS 43 %).
+// Reading the matrix and writing 9 bytes per selected entry would take 79 us at T =
+// 8192, k = 2048 at the rate of a large copy; this takes 110, radix passes and a
+// bitonic sort for every row took 1775.
 #include "gsa_common.h"
 
 namespace gsa {
